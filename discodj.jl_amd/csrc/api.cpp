@@ -5,8 +5,8 @@
 //   tile deposit -> XF -> YF -> ZM(K_phi) -> YI -> XI (potential) -> FD-fused tile gather
 // For grad_order 0 (ik gradient) the spectrum is kept after the forward z pass and three inverse
 // sequences produce -d_a phi, each gathered into one acceleration component (pm.jl:487-492).
-// In dj_run the gather of the last shift also applies the kick, the second drift and, unless a
-// callback needs the state in between, the next step's first drift.
+// In dj_run the kick after the last shift also applies the second drift and, unless a callback needs
+// the state in between, the next step's first drift.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,10 +29,10 @@ namespace {
 
 thread_local std::string g_create_error;
 
-enum KernelId { K_ZERO = 0, K_SCATTER, K_XF, K_YF, K_ZM, K_YI, K_XI, K_GATHER, K_GATHER_KICK, K_KICK, K_DRIFT, K_SORT,
+enum KernelId { K_ZERO = 0, K_SCATTER, K_XF, K_YF, K_ZM, K_YI, K_XI, K_GATHER, K_KICK, K_DRIFT, K_SORT,
                 K_SORT_EXACT, K_RESAMPLE, K_NN, K_GATHER_LAST, K_KICK_LISTED, K_COUNT };
 const char *kernel_names[K_COUNT] = {"zero", "scatter", "fft_x_r2c", "fft_y_fwd", "fft_z_mult", "fft_y_inv",
-                                     "fft_x_c2r", "gather", "gather_kick", "kick_drift", "drift", "bin",
+                                     "fft_x_c2r", "gather", "kick_drift", "drift", "bin",
                                      "bin_recount", "resample", "nn_correction", "gather_last", "kick_listed"};
 
 struct ProfEvent {
@@ -377,9 +377,6 @@ void set_bytes(dj_ctx *c) {
     c->bytes[K_XI] = 2 * T * HC + T * M;
     // FD gather of a pass that stores the acceleration: read the positions and phi, write acc
     c->bytes[K_GATHER] = 3 * T * np * 2 + T * M;
-    // FD gather of the last pass fused with kick and drift: read psi, mom (and acc when averaging
-    // shifts), read phi once, write psi and mom
-    c->bytes[K_GATHER_KICK] = 3 * T * np * (c->nshifts > 1 ? 5 : 4) + T * M;
     c->bytes[K_KICK] = 3 * T * np * 5;
     // the last pass's gather when interlacing: read the positions, the hand-over and phi, write the hand-over
     c->bytes[K_GATHER_LAST] = 3 * T * np * 3 + T * M;
@@ -554,7 +551,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick) {
     (void)mesh_bytes;
     // in a step the passes hand the acceleration over in tile-list order: both walk the same lists, so
     // the hand-over is read and written contiguously instead of at the particles' positions
-    const bool lacc = mode == FORCE_KICK && ns > 1 && !ik;
+    const bool lacc = listed_kick;
     if (lacc && c->acc_list_cap < c->tl.ent_cap) {
         if (c->acc_list) HIPCHK(c, hipFree(c->acc_list));
         c->acc_list = nullptr;
@@ -609,14 +606,13 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick) {
             { Prof p(c, K_XI); c->fft.xi(c->A, c->mesh, c->tw, c->st); }
             if (c->nn_on) c->nn.axpy(c->mesh, c->nn_dphi, c->M, 1.0, c->st);
             const bool last = s == ns - 1;
-            // first pass stores acc, later passes add to it; the last one of a step kicks and drifts (fused
-            // into the gather without interlacing, in particle order after it with)
-            const int gmode = (mode == FORCE_KICK && last && !listed_kick) ? GATHER_KICK
-                                                                           : (s == 0 ? GATHER_ASSIGN : GATHER_ACC);
+            // first pass stores acc, later passes add to it; the kick and drifts follow in particle order.  With
+            // one pass the gather stores acc at the particles: kicking inside it, in list order, took 560 us at
+            // 256^3 (CIC, order 4), the gather and the streaming kick take 204 and 190
+            const int gmode = s == 0 ? GATHER_ASSIGN : GATHER_ACC;
             {
-                Prof p(c, gmode == GATHER_KICK ? K_GATHER_KICK : (listed_kick && last ? K_GATHER_LAST : K_GATHER));
-                c->tiles.gather(ta, cfg.worder, cfg.grad_order, c->shifts[s], c->mesh, c->fdc, gmode, kick, c->psi,
-                                c->st);
+                Prof p(c, listed_kick && last ? K_GATHER_LAST : K_GATHER);
+                c->tiles.gather(ta, cfg.worder, cfg.grad_order, c->shifts[s], c->mesh, c->fdc, gmode, c->st);
             }
             if (listed_kick && last) {
                 Prof p(c, K_KICK_LISTED);
@@ -635,7 +631,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick) {
         dj_status r = check_launch(c, "force pass");
         if (r) return r;
     }
-    if (ik && mode == FORCE_KICK) {
+    if (mode == FORCE_KICK && !listed_kick) {
         Prof p(c, K_KICK);
         c->part.kick_drift(c->psi, c->mom, c->acc, c->n3, kick, c->st);
     } else if (mode == FORCE_ACC && ns > 1) {

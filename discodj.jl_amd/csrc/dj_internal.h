@@ -49,7 +49,7 @@ struct PartArgs {
     double shift[3];      // interlacing shift of this pass
 };
 
-enum { GATHER_ACC = 0, GATHER_ASSIGN = 1, GATHER_KICK = 2 };
+enum { GATHER_ACC = 0, GATHER_ASSIGN = 1 };
 
 struct KickArgs {
     double alpha, beta, dd2, dd1_next;  // FP64 step coefficients, rounded to T at use
@@ -58,12 +58,6 @@ struct KickArgs {
 };
 
 struct PartOps {
-    // unit-mass deposit of X = q + psi + shift (float atomics, or fixed-point int64 when fixed)
-    void (*scatter)(const PartArgs &a, int W, bool fixed, int frac_bits, void *mesh, hipStream_t st);
-    // gather -D phi (FD order 2/4/6) at X; mode GATHER_ACC (acc += s), GATHER_ASSIGN (acc = s, lean
-    // per-axis semantics are equal), GATHER_KICK (final pass fused with kick and drift)
-    void (*gather_fd)(const PartArgs &a, int W, int order, const void *phi, const double *c, int mode,
-                      const KickArgs &k, void *psi_out, hipStream_t st);
     // gather one component of a mesh field at X into acc[comp] (+=)
     void (*gather_comp)(const PartArgs &a, int W, const void *field, int comp, hipStream_t st);
     // psi += dd * mom
@@ -120,7 +114,7 @@ struct TileOps {
     void (*deposit)(const TileArgs &a, int W, bool fixed, const double *shift, void *mesh, double fscale,
                     hipStream_t st);
     void (*gather)(const TileArgs &a, int W, int order, const double *shift, const void *phi, const double *c,
-                   int mode, const KickArgs &k, void *psi_out, hipStream_t st);
+                   int mode, hipStream_t st);
     // the kick and drifts of a step in particle order, the force summed over the ns passes in list order
     // (acc_list[3 e + c], e = own_at[p]): mom = alpha mom + beta acc / ns, psi += (dd2 + dd1n) steps of mom
     void (*kick_listed)(const unsigned *own_at, const void *acc_list, void *psi, void *mom, size_t np,

@@ -1,4 +1,4 @@
-// Particle-side kernels of the PM step: mass assignment, force gather, kick and drift.
+// Particle-side kernels of the PM step: the spectral gradient's gather, kick and drift.
 //
 // Particles are the reference's column-major (n,n,n,3) arrays: particle p = i + n (j + n k) has
 // Lagrangian position (q[i], q[j], q[k]) with q[i] = i L/n (FP64, rounded to T), and its
@@ -82,109 +82,6 @@ __device__ __forceinline__ PIdx pidx(int n) {
     return r;
 }
 
-template <typename T, int W, bool FIXED>
-__global__ __launch_bounds__(256) void k_scatter(const T *__restrict__ psi, const T *__restrict__ q1, int n,
-                                                 T sx, T sy, T sz, void *mesh, int res, T L, double fscale) {
-    PIdx P = pidx(n);
-    if (!P.ok) return;
-    T x = (psi[P.p] + q1[P.i]) + sx;
-    T y = (psi[P.p + P.np] + q1[P.j]) + sy;
-    T z = (psi[P.p + 2 * P.np] + q1[P.k]) + sz;
-    Axis<T, W, 0> ax, ay, az;
-    ax.make(x, res, L);
-    ay.make(y, res, L);
-    az.make(z, res, L);
-#pragma unroll
-    for (int oz = 0; oz < W; oz++)
-#pragma unroll
-        for (int oy = 0; oy < W; oy++) {
-            size_t row = (size_t)res * ((size_t)ay.nb[oy] + (size_t)res * az.nb[oz]);
-#pragma unroll
-            for (int ox = 0; ox < W; ox++) {
-                T w = ax.w[ox] * ay.w[oy] * az.w[oz];
-                size_t c = row + ax.nb[ox];
-                if constexpr (FIXED) {
-                    long long v = __double2ll_rn((double)w * fscale);
-                    atomicAdd((unsigned long long *)mesh + c, (unsigned long long)v);
-                } else {
-                    unsafeAtomicAdd((T *)mesh + c, w);
-                }
-            }
-        }
-}
-
-// -D_a phi at a cell, order 2/4/6 central differences (pm.jl:330-342); nb holds the cell's
-// neighbourhood along the axis with the cell at index t0
-template <typename T, int ORDER>
-__device__ __forceinline__ T fdiff(const T *__restrict__ phi, size_t base, size_t stride, const int *nb, int t0,
-                                   T c1, T c2, T c3) {
-    T d1 = phi[base + stride * nb[t0 + 1]] - phi[base + stride * nb[t0 - 1]];
-    if constexpr (ORDER == 2) return -(c1 * d1);
-    T d2 = phi[base + stride * nb[t0 + 2]] - phi[base + stride * nb[t0 - 2]];
-    if constexpr (ORDER == 4) return -(c1 * d1 + c2 * d2);
-    T d3 = phi[base + stride * nb[t0 + 3]] - phi[base + stride * nb[t0 - 3]];
-    return -(c1 * d1 + c2 * d2 + c3 * d3);
-}
-
-template <typename T, int W, int ORDER, int MODE>
-__global__ __launch_bounds__(256) void k_gather_fd(const T *__restrict__ psi_in, T *__restrict__ psi_out,
-                                                   T *__restrict__ mom, T *__restrict__ acc,
-                                                   const T *__restrict__ q1, int n, T sx, T sy, T sz,
-                                                   const T *__restrict__ phi, int res, T L, T c1, T c2, T c3,
-                                                   T alpha, T beta, T dd2, T dd1n, int has_next, int ns) {
-    PIdx P = pidx(n);
-    if (!P.ok) return;
-    T px = psi_in[P.p], py = psi_in[P.p + P.np], pz = psi_in[P.p + 2 * P.np];
-    T x = (px + q1[P.i]) + sx;
-    T y = (py + q1[P.j]) + sy;
-    T z = (pz + q1[P.k]) + sz;
-    constexpr int HALO = ORDER / 2;
-    Axis<T, W, HALO> ax, ay, az;
-    ax.make(x, res, L);
-    ay.make(y, res, L);
-    az.make(z, res, L);
-    const size_t R = (size_t)res, RR = R * R;
-    T s1 = 0, s2 = 0, s3 = 0;
-#pragma unroll
-    for (int oz = 0; oz < W; oz++)
-#pragma unroll
-        for (int oy = 0; oy < W; oy++)
-#pragma unroll
-            for (int ox = 0; ox < W; ox++) {
-                T w = ax.w[ox] * ay.w[oy] * az.w[oz];
-                const int tx = ox + HALO, ty = oy + HALO, tz = oz + HALO;
-                size_t cx = ax.nb[tx], cy = ay.nb[ty], cz = az.nb[tz];
-                T fx = fdiff<T, ORDER>(phi, R * cy + RR * cz, 1, ax.nb, tx, c1, c2, c3);
-                T fy = fdiff<T, ORDER>(phi, cx + RR * cz, R, ay.nb, ty, c1, c2, c3);
-                T fz = fdiff<T, ORDER>(phi, cx + R * cy, RR, az.nb, tz, c1, c2, c3);
-                s1 += fx * w;
-                s2 += fy * w;
-                s3 += fz * w;
-            }
-    if constexpr (MODE == GATHER_ACC) {
-        acc[P.p] += s1;
-        acc[P.p + P.np] += s2;
-        acc[P.p + 2 * P.np] += s3;
-    } else if constexpr (MODE == GATHER_ASSIGN) {
-        acc[P.p] = s1;
-        acc[P.p + P.np] = s2;
-        acc[P.p + 2 * P.np] = s3;
-    } else {
-        T a[3] = {s1, s2, s3}, ps[3] = {px, py, pz};
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            size_t q = P.p + c * P.np;
-            T ac = a[c];
-            if (ns > 1) ac = (acc[q] + ac) / (T)ns;
-            T m = alpha * mom[q] + beta * ac;
-            T s = ps[c] + dd2 * m;
-            if (has_next) s = s + dd1n * m;
-            mom[q] = m;
-            psi_out[q] = s;
-        }
-    }
-}
-
 template <typename T, int W>
 __global__ __launch_bounds__(256) void k_gather_comp(const T *__restrict__ psi, T *__restrict__ acc,
                                                      const T *__restrict__ q1, int n, T sx, T sy, T sz,
@@ -265,56 +162,6 @@ __global__ __launch_bounds__(256) void k_zero(uint4 *__restrict__ x, size_t n16,
 static dim3 pgrid(int n) { return dim3((n + 255) / 256, n, n); }
 static unsigned lgrid(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-template <typename T, int W>
-static void scatter_w(const PartArgs &a, bool fixed, int frac_bits, void *mesh, hipStream_t st) {
-    double fs = ldexp(1.0, frac_bits);
-    const T *psi = (const T *)a.psi, *q1 = (const T *)a.q1;
-    T sx = (T)a.shift[0], sy = (T)a.shift[1], sz = (T)a.shift[2], L = (T)a.L;
-    if (fixed)
-        k_scatter<T, W, true><<<pgrid(a.n), 256, 0, st>>>(psi, q1, a.n, sx, sy, sz, mesh, a.res, L, fs);
-    else
-        k_scatter<T, W, false><<<pgrid(a.n), 256, 0, st>>>(psi, q1, a.n, sx, sy, sz, mesh, a.res, L, fs);
-}
-
-template <typename T>
-static void scatter(const PartArgs &a, int W, bool fixed, int frac_bits, void *mesh, hipStream_t st) {
-    if (W == 2) scatter_w<T, 2>(a, fixed, frac_bits, mesh, st);
-    else if (W == 3) scatter_w<T, 3>(a, fixed, frac_bits, mesh, st);
-    else scatter_w<T, 4>(a, fixed, frac_bits, mesh, st);
-}
-
-template <typename T, int W, int ORDER>
-static void gather_fd_wo(const PartArgs &a, const void *phi, const double *c, int mode, const KickArgs &k,
-                         void *psi_out, hipStream_t st) {
-    const T *psi = (const T *)a.psi, *q1 = (const T *)a.q1;
-    T sx = (T)a.shift[0], sy = (T)a.shift[1], sz = (T)a.shift[2], L = (T)a.L;
-    T c1 = (T)c[0], c2 = (T)c[1], c3 = (T)c[2];
-#define GF(M)                                                                                               \
-    k_gather_fd<T, W, ORDER, M><<<pgrid(a.n), 256, 0, st>>>(                                                 \
-        psi, (T *)psi_out, (T *)a.mom, (T *)a.acc, q1, a.n, sx, sy, sz, (const T *)phi, a.res, L, c1, c2, c3, \
-        (T)k.alpha, (T)k.beta, (T)k.dd2, (T)k.dd1_next, k.has_next, k.nshifts)
-    if (mode == GATHER_ACC) GF(GATHER_ACC);
-    else if (mode == GATHER_ASSIGN) GF(GATHER_ASSIGN);
-    else GF(GATHER_KICK);
-#undef GF
-}
-
-template <typename T, int W>
-static void gather_fd_w(const PartArgs &a, int order, const void *phi, const double *c, int mode,
-                        const KickArgs &k, void *psi_out, hipStream_t st) {
-    if (order == 2) gather_fd_wo<T, W, 2>(a, phi, c, mode, k, psi_out, st);
-    else if (order == 4) gather_fd_wo<T, W, 4>(a, phi, c, mode, k, psi_out, st);
-    else gather_fd_wo<T, W, 6>(a, phi, c, mode, k, psi_out, st);
-}
-
-template <typename T>
-static void gather_fd(const PartArgs &a, int W, int order, const void *phi, const double *c, int mode,
-                      const KickArgs &k, void *psi_out, hipStream_t st) {
-    if (W == 2) gather_fd_w<T, 2>(a, order, phi, c, mode, k, psi_out, st);
-    else if (W == 3) gather_fd_w<T, 3>(a, order, phi, c, mode, k, psi_out, st);
-    else gather_fd_w<T, 4>(a, order, phi, c, mode, k, psi_out, st);
-}
-
 template <typename T>
 static void gather_comp(const PartArgs &a, int W, const void *field, int comp, hipStream_t st) {
     const T *psi = (const T *)a.psi, *q1 = (const T *)a.q1;
@@ -363,8 +210,6 @@ static void zero(void *x, size_t bytes, hipStream_t st) {
 }
 
 template <typename T> void part_ops(PartOps &ops) {
-    ops.scatter = scatter<T>;
-    ops.gather_fd = gather_fd<T>;
     ops.gather_comp = gather_comp<T>;
     ops.drift = drift<T>;
     ops.drift_to = drift_to<T>;

@@ -11,9 +11,9 @@
 // Deposit: one workgroup per tile accumulates its list in LDS (float / double / int64 atomics) and
 // writes the tile with plain coalesced stores: no global atomics, no zero fill of the mesh.
 // Gather: one workgroup per tile stages the potential of the tile plus the stencil reach and the
-// finite-difference halo in LDS, evaluates -D phi at the 27 (64) stencil cells from LDS for its own
-// particles, and applies the kick and drifts in place.  A particle whose stencil leaves the staged
-// region (not expected; kept for safety) reads the potential from global memory instead.
+// finite-difference halo in LDS and evaluates -D phi at the 27 (64) stencil cells from LDS for its own
+// particles.  A particle whose stencil leaves the staged region (not expected; kept for safety) reads
+// the potential from global memory instead.
 #include <hip/hip_runtime.h>
 
 #include "dj_internal.h"
@@ -892,22 +892,13 @@ template <typename T, int W> constexpr int gather_threads() { return sizeof(T) =
 // waves per SIMD the register allocation must allow: two FP32 workgroups per CU (128 VGPRs)
 template <typename T, int W> constexpr int gather_min_waves() { return sizeof(T) == 4 && W <= 3 ? 4 : 1; }
 
-// a particle's tile entry and the state its gather mode reads
+// a particle's tile entry and, when its gather adds to earlier passes, their sum
 template <typename T, int MODE>
-__device__ __forceinline__ void gather_fetch(const Entry<T> *__restrict__ ent, unsigned e, const T *psi_in,
-                                             const T *__restrict__ mom, const T *__restrict__ acc, size_t np, int ns,
-                                             int lacc, Entry<T> &en, T (&m3)[3], T (&p3)[3], T (&a3)[3]) {
+__device__ __forceinline__ void gather_fetch(const Entry<T> *__restrict__ ent, unsigned e, const T *__restrict__ acc,
+                                             size_t np, int lacc, Entry<T> &en, T (&a3)[3]) {
     en = ent[e];
-    const size_t p = (size_t)en.idx;
-    if constexpr (MODE == GATHER_KICK) {
-        // acc (the earlier passes' sum) is read after the stencil, to keep registers for it
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            m3[c] = mom[p + c * np];
-            p3[c] = psi_in[p + c * np];
-        }
-    } else if constexpr (MODE == GATHER_ACC) {
-        const size_t ai = lacc ? 3 * (size_t)e : p, as = lacc ? 1 : np;
+    if constexpr (MODE == GATHER_ACC) {
+        const size_t ai = lacc ? 3 * (size_t)e : (size_t)en.idx, as = lacc ? 1 : np;
 #pragma unroll
         for (int c = 0; c < 3; c++) a3[c] = acc[ai + c * as];
     }
@@ -1058,9 +1049,8 @@ __device__ __forceinline__ void stage_groups(const T *phi, T *ph, const int (&r0
 template <typename T, int W, int ORDER, int MODE, bool FG>
 __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>())) void k_tile_gather(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
                                                       const unsigned *__restrict__ own, TileGeom g, T sx, T sy, T sz,
-                                                      T L, const T *__restrict__ phi, T c1, T c2, T c3, const T *psi_in,
-                                                      T *psi_out, T *__restrict__ mom, T *__restrict__ acc, size_t np,
-                                                      T alpha, T beta, T dd2, T dd1n, int has_next, int ns, int lacc) {
+                                                      T L, const T *__restrict__ phi, T c1, T c2, T c3,
+                                                      T *__restrict__ acc, size_t np, int lacc) {
     constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
     extern __shared__ unsigned char smem[];
     T *ph = (T *)smem;
@@ -1079,8 +1069,8 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
     const unsigned e0 = start[t], e1 = e0 + own[t];
     unsigned e = e0 + threadIdx.x;
     Entry<T> en{};
-    T m3[3] = {0, 0, 0}, p3[3] = {0, 0, 0}, a3[3] = {0, 0, 0};
-    if (e < e1) gather_fetch<T, MODE>(ent, e, psi_in, mom, acc, np, ns, lacc, en, m3, p3, a3);
+    T a3[3] = {0, 0, 0};
+    if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
 
     if (region_ok) {
         const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1124,23 +1114,12 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
         if constexpr (MODE == GATHER_ACC) {
 #pragma unroll
             for (int c = 0; c < 3; c++) acc[ai + c * as] = a3[c] + f3[c];
-        } else if constexpr (MODE == GATHER_ASSIGN) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                T ac = f3[c];
-                if (ns > 1) ac = (acc[ai + c * as] + ac) / (T)ns;
-                T m = alpha * m3[c] + beta * ac;
-                T s = p3[c] + dd2 * m;
-                if (has_next) s = s + dd1n * m;
-                mom[p + c * np] = m;
-                psi_out[p + c * np] = s;
-            }
+            for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
         }
         e += NT;
-        if (e < e1) gather_fetch<T, MODE>(ent, e, psi_in, mom, acc, np, ns, lacc, en, m3, p3, a3);
+        if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
     }
 }
 
@@ -1157,11 +1136,20 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
 // is the staged gather's (same sums, same order).
 struct MarchMap {
     int G;          // tiles per segment (divides ntz)
+    int parts;      // workgroups that share a segment, each with its part of every tile's list
     bool patches;   // 4 x 4 column patches dealt round-robin to the XCDs
 };
-__host__ __device__ __forceinline__ MarchMap march_map(const TileGeom &g) {
+// Segments are as long as leaves MARCH_WGS workgroups (four per CU; 16 tiles at most, where a tile stages
+// TZ of S2 planes and longer ones gain nothing).  A mesh of too few tiles for that gives every tile up to
+// four workgroups, each of which stages the tile and takes its part of the list.  16 tiles everywhere left
+// a 64^3 mesh with 8 workgroups (97 us; 20 us with 256) and a 256^3 mesh with one per CU (279 us a pass,
+// CIC, order 4; 204 us with four).
+constexpr int MARCH_WGS = 1024;
+inline MarchMap march_map(const TileGeom &g) {
     MarchMap m;
-    m.G = (g.ntz % 16 == 0) ? 16 : (g.ntz % 8 == 0) ? 8 : (g.ntz % 4 == 0) ? 4 : (g.ntz % 2 == 0) ? 2 : 1;
+    m.G = 1;
+    while (m.G < 16 && g.ntz % (2 * m.G) == 0 && g.nt / (2 * m.G) >= MARCH_WGS) m.G *= 2;
+    m.parts = g.nt <= 128 ? 4 : g.nt <= 256 ? 2 : 1;
     m.patches = g.ntx % 4 == 0 && g.nty % 4 == 0 && ((g.ntx / 4) * (g.nty / 4)) % 8 == 0;
     return m;
 }
@@ -1189,9 +1177,8 @@ __device__ __forceinline__ void march_segment(int b, const TileGeom &g, const Ma
 template <typename T, int W, int ORDER, int MODE>
 __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>())) void k_tile_gather_march(
     const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start, const unsigned *__restrict__ own, TileGeom g,
-    T sx, T sy, T sz, T L, const T *__restrict__ phi, T c1, T c2, T c3, const T *psi_in, T *psi_out,
-    T *__restrict__ mom, T *__restrict__ acc, size_t np, T alpha, T beta, T dd2, T dd1n, int has_next, int ns,
-    int lacc) {
+    T sx, T sy, T sz, T L, const T *__restrict__ phi, T c1, T c2, T c3, T *__restrict__ acc, size_t np, int lacc,
+    MarchMap m) {
     constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
     extern __shared__ unsigned char smem[];
     T *ph = (T *)smem;
@@ -1199,9 +1186,9 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
     constexpr int TXL = 5, TYL = 4, TZ = FIXED_TZ;
     const int S[3] = {q.s[0], q.s[1], q.s[2]};
     const int N = g.N, SX = S[0], SXY = S[0] * S[1], R = S[2];  // R: ring planes
-    const MarchMap m = march_map(g);
     int tx, ty, tz0;
-    march_segment(blockIdx.x, g, m, tx, ty, tz0);
+    march_segment(blockIdx.x / m.parts, g, m, tx, ty, tz0);
+    const int part = blockIdx.x % m.parts, step = NT * m.parts;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rx = (tx << TXL) - q.lo[0], ry = (ty << TYL) - q.lo[1];
     const int zs0 = tz0 * TZ - q.lo[2];  // first staged plane of the segment (ring slot 0)
@@ -1212,10 +1199,10 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
         const int t = tx + g.ntx * (ty + g.nty * tz);
         const int r0[3] = {rx, ry, tz * TZ - q.lo[2]};
         const unsigned e0 = start[t], e1 = e0 + own[t];
-        unsigned e = e0 + threadIdx.x;
+        unsigned e = e0 + part * NT + threadIdx.x;
         Entry<T> en{};
-        T m3[3] = {0, 0, 0}, p3[3] = {0, 0, 0}, a3[3] = {0, 0, 0};
-        if (e < e1) gather_fetch<T, MODE>(ent, e, psi_in, mom, acc, np, ns, lacc, en, m3, p3, a3);
+        T a3[3] = {0, 0, 0};
+        if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
         // stage: the whole region for the first tile, else the TZ planes after the previous region,
         // into the ring slots (zg - zs0) mod R, split where the slots wrap
         {
@@ -1270,23 +1257,12 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
             if constexpr (MODE == GATHER_ACC) {
 #pragma unroll
                 for (int c = 0; c < 3; c++) acc[ai + c * as] = a3[c] + f3[c];
-            } else if constexpr (MODE == GATHER_ASSIGN) {
-#pragma unroll
-                for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
             } else {
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    T ac = f3[c];
-                    if (ns > 1) ac = (acc[ai + c * as] + ac) / (T)ns;
-                    T mm = alpha * m3[c] + beta * ac;
-                    T sp = p3[c] + dd2 * mm;
-                    if (has_next) sp = sp + dd1n * mm;
-                    mom[p + c * np] = mm;
-                    psi_out[p + c * np] = sp;
-                }
+                for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
             }
-            e += NT;
-            if (e < e1) gather_fetch<T, MODE>(ent, e, psi_in, mom, acc, np, ns, lacc, en, m3, p3, a3);
+            e += step;
+            if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
         }
         // every wave is done with this tile's first TZ planes before the next tile's staging overwrites them
         __syncthreads();
@@ -1295,8 +1271,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
 
 // The kick and drifts of a step in particle order (run_nbody.jl:156-158), the last interlacing pass having
 // added its force into the list-ordered hand-over: the state is read and written in order, and each
-// particle's summed force (12 contiguous bytes) is fetched through its own-list entry.  The arithmetic is
-// the kick gather's, in its order.
+// particle's summed force (12 contiguous bytes) is fetched through its own-list entry.
 template <typename T>
 __global__ __launch_bounds__(256) void k_kick_listed(const unsigned *__restrict__ own_at, const T *__restrict__ accl,
                                                      T *__restrict__ psi, T *__restrict__ mom, size_t np, T alpha,
@@ -1413,8 +1388,7 @@ struct TileLaunch {
         else dep_sel<4>(a, fixed, sh, mesh, fscale, st);
     }
     template <int W, int O, int M, bool FG>
-    static void gat_womf(const TileArgs &a, const double *sh, const void *phi, const double *c, const KickArgs &k,
-                         void *psi_out, hipStream_t st) {
+    static void gat_womf(const TileArgs &a, const double *sh, const void *phi, const double *c, hipStream_t st) {
         constexpr int H = O / 2;
         const StageGeom q = gather_geom<T, W, FG>(a.g, H);
         // a region that is not staged (as large as the mesh) is read from global memory by the kernel
@@ -1422,54 +1396,48 @@ struct TileLaunch {
         auto kern = k_tile_gather<T, W, O, M, FG>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         kern<<<a.g.nt, gather_threads<T, W>(), shm, st>>>((const Entry<T> *)a.ent, a.start, a.cur, a.g, (T)sh[0], (T)sh[1], (T)sh[2],
-                                        (T)a.L, (const T *)phi, (T)c[0], (T)c[1], (T)c[2], (const T *)a.psi,
-                                        (T *)psi_out, (T *)a.mom, (T *)a.acc, (size_t)a.n * a.n * a.n, (T)k.alpha,
-                                        (T)k.beta, (T)k.dd2, (T)k.dd1_next, k.has_next, k.nshifts, a.acc_by_entry);
+                                        (T)a.L, (const T *)phi, (T)c[0], (T)c[1], (T)c[2], (T *)a.acc,
+                                        (size_t)a.n * a.n * a.n, a.acc_by_entry);
     }
     template <int W, int O, int M>
-    static void gat_march(const TileArgs &a, const double *sh, const void *phi, const double *c, const KickArgs &k,
-                          void *psi_out, hipStream_t st) {
+    static void gat_march(const TileArgs &a, const double *sh, const void *phi, const double *c, hipStream_t st) {
         constexpr int H = O / 2;
         const StageGeom q = gather_geom<T, W, true>(a.g, H);
         const size_t shm = sizeof(T) * (size_t)q.s[0] * q.s[1] * q.s[2];
         const MarchMap mm = march_map(a.g);
         auto kern = k_tile_gather_march<T, W, O, M>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-        kern<<<a.g.nt / mm.G, gather_threads<T, W>(), shm, st>>>(
+        kern<<<a.g.nt / mm.G * mm.parts, gather_threads<T, W>(), shm, st>>>(
             (const Entry<T> *)a.ent, a.start, a.cur, a.g, (T)sh[0], (T)sh[1], (T)sh[2], (T)a.L, (const T *)phi,
-            (T)c[0], (T)c[1], (T)c[2], (const T *)a.psi, (T *)psi_out, (T *)a.mom, (T *)a.acc,
-            (size_t)a.n * a.n * a.n, (T)k.alpha, (T)k.beta, (T)k.dd2, (T)k.dd1_next, k.has_next, k.nshifts,
-            a.acc_by_entry);
+            (T)c[0], (T)c[1], (T)c[2], (T *)a.acc, (size_t)a.n * a.n * a.n, a.acc_by_entry, mm);
     }
     template <int W, int O, int M>
-    static void gat_wom(const TileArgs &a, const double *sh, const void *phi, const double *c, const KickArgs &k,
-                        void *psi_out, hipStream_t st) {
+    static void gat_wom(const TileArgs &a, const double *sh, const void *phi, const double *c, hipStream_t st) {
         if constexpr (sizeof(T) == 4) {
             if (fixed_geom_fits<W>(a.g) && gather_geom<T, W, true>(a.g, O / 2).ok)
-                return gat_march<W, O, M>(a, sh, phi, c, k, psi_out, st);
-            if (fixed_geom_fits<W>(a.g)) return gat_womf<W, O, M, true>(a, sh, phi, c, k, psi_out, st);
+                return gat_march<W, O, M>(a, sh, phi, c, st);
+            if (fixed_geom_fits<W>(a.g)) return gat_womf<W, O, M, true>(a, sh, phi, c, st);
         }
-        gat_womf<W, O, M, false>(a, sh, phi, c, k, psi_out, st);
+        gat_womf<W, O, M, false>(a, sh, phi, c, st);
     }
     template <int W, int O>
     static void gat_wo(const TileArgs &a, const double *sh, const void *phi, const double *c, int mode,
-                       const KickArgs &k, void *psi_out, hipStream_t st) {
-        if (mode == GATHER_ACC) gat_wom<W, O, GATHER_ACC>(a, sh, phi, c, k, psi_out, st);
-        else if (mode == GATHER_ASSIGN) gat_wom<W, O, GATHER_ASSIGN>(a, sh, phi, c, k, psi_out, st);
-        else gat_wom<W, O, GATHER_KICK>(a, sh, phi, c, k, psi_out, st);
+                       hipStream_t st) {
+        if (mode == GATHER_ACC) gat_wom<W, O, GATHER_ACC>(a, sh, phi, c, st);
+        else gat_wom<W, O, GATHER_ASSIGN>(a, sh, phi, c, st);
     }
     template <int W>
     static void gat_w(const TileArgs &a, int order, const double *sh, const void *phi, const double *c, int mode,
-                      const KickArgs &k, void *psi_out, hipStream_t st) {
-        if (order == 2) gat_wo<W, 2>(a, sh, phi, c, mode, k, psi_out, st);
-        else if (order == 4) gat_wo<W, 4>(a, sh, phi, c, mode, k, psi_out, st);
-        else gat_wo<W, 6>(a, sh, phi, c, mode, k, psi_out, st);
+                      hipStream_t st) {
+        if (order == 2) gat_wo<W, 2>(a, sh, phi, c, mode, st);
+        else if (order == 4) gat_wo<W, 4>(a, sh, phi, c, mode, st);
+        else gat_wo<W, 6>(a, sh, phi, c, mode, st);
     }
     static void gather(const TileArgs &a, int W, int order, const double *sh, const void *phi, const double *c,
-                       int mode, const KickArgs &k, void *psi_out, hipStream_t st) {
-        if (W == 2) gat_w<2>(a, order, sh, phi, c, mode, k, psi_out, st);
-        else if (W == 3) gat_w<3>(a, order, sh, phi, c, mode, k, psi_out, st);
-        else gat_w<4>(a, order, sh, phi, c, mode, k, psi_out, st);
+                       int mode, hipStream_t st) {
+        if (W == 2) gat_w<2>(a, order, sh, phi, c, mode, st);
+        else if (W == 3) gat_w<3>(a, order, sh, phi, c, mode, st);
+        else gat_w<4>(a, order, sh, phi, c, mode, st);
     }
 };
 
