@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "dj_internal.h"
@@ -75,75 +76,130 @@ template void pk_bin<double>(const void *, int, double, int, int, double, double
 // The binning of evaluate_power_spectrum / evaluate_cross_power_spectrum (NR/src/analysis/power_spectrum.jl:
 // 25-123) and of the study estimator (studies/eft_shell_crossing/src/measure.jl:403-447), on the library's
 // x-halved spectrum.  The reference halves the z axis: its modes are (i, j, l), i, j < N, l <= N/2, with
-// signed wavenumbers (i <= N/2 ? i : i - N) kf.  One thread takes one of those modes, forms |k| exactly as
-// the reference does, sqrt((kx kx + ky ky) + kz kz) in FP64, so that every mode lands in the reference's
-// bin, and reads the value from the library's storage: (x = i, y = j, z = l) when i <= N/2, else the
-// conjugate-symmetric (N - i, -j, -l) (the value |F|^2, or Re conj(F1) F2, is the same).  Per bin it sums
-// |k|, w v, w and the count in LDS, then once per block into sums (4 nbins doubles).
+// signed wavenumbers (i <= N/2 ? i : i - N) kf.  A stored entry (x, y, z) is the reference's mode (x, y, z)
+// when z <= N/2, and the conjugate of its mode (N - x, -y, N - z) when 0 < x < N/2 and z is 0 or >= N/2, with
+// the same |F|^2 (and Re conj(F1) F2) and the same |k|: entries on the x = 0 and N/2 planes are one mode or
+// none, the others one, or two at z = 0 and N/2.  |k| is formed exactly as the reference does, in FP64, so
+// that every mode lands in the reference's bin: sqrt((kx kx + ky ky) + kz kz) >= e exactly when the sum is
+// at least pk_threshold(e), so the bins are found by comparing sums.  Per bin |k|, w v, w and the count are
+// summed in LDS, then once per block into sums (4 nbins doubles).
 //   wmode 0: w = 1/2 on the l = 0 and l = N/2 planes, 1 elsewhere (the auto spectrum and the study
 //            estimator, whose 1 / 2 weights have the same ratio); wmode 1: w = 1 (the cross spectrum)
 //   W > 0:   v is divided by |W(k)|^2 = prod_a sinc(k_a dx / 2)^(2 W) (mass-assignment window)
-template <typename T>
+// A thread takes one z and PK_XL consecutive x of a y row, so that its entries stay in one bin for a while:
+// their sums stay in registers until the bin changes (LDS atomics once per run of entries; neighbouring
+// lanes mostly share the bin, so one atomic per entry met 64 others at one address: 1.45 ms for 512^3, FP32,
+// with the window's sin and pow per entry, against 0.2 ms).  The window's factors are a table in LDS.
+constexpr int PK_XL = 16, PK_COPIES = 4;
+
+template <typename T, bool CROSS, bool KSUM>
 __global__ __launch_bounds__(256) void k_pk_edges(const cx<T> *__restrict__ F1, const cx<T> *__restrict__ F2, int N,
-                                                  double kf, double dx, int W, int wmode, double scale, PkEdges ed,
+                                                  double kf, double dx, int W, int wmode, double scale, PkEdges thr,
                                                   double *__restrict__ sums) {
-    __shared__ double se[PK_MAX_BINS + 1];
-    __shared__ double sk[PK_MAX_BINS], sp[PK_MAX_BINS], sw[PK_MAX_BINS], sc[PK_MAX_BINS];
-    const int nb = ed.nbins;
-    for (int b = threadIdx.x; b <= nb; b += blockDim.x) se[b] = ed.e[b];
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) { sk[b] = 0; sp[b] = 0; sw[b] = 0; sc[b] = 0; }
+    extern __shared__ double sh[];
+    const int nb = thr.nbins, H = N / 2 + 1;
+    double *st = sh, *sb = st + nb + 1, *swin = sb + PK_COPIES * 4 * nb;
+    for (int b = threadIdx.x; b <= nb; b += 256) st[b] = thr.e[b];
+    for (int b = threadIdx.x; b < PK_COPIES * 4 * nb; b += 256) sb[b] = 0;
+    if (W > 0)
+        for (int m = threadIdx.x; m < H; m += 256) {
+            const double s0 = (double)m * kf * dx / 2, s = s0 == 0 ? 1.0 : sin(s0) / s0;
+            swin[m] = pow(s, 2 * W);
+        }
     __syncthreads();
-    const int H = N / 2 + 1;
-    const size_t tot = (size_t)N * N * H;
-    const double lo = se[0], hi = se[nb];
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (size_t)gridDim.x * blockDim.x) {
-        const int l = (int)(e % H);
-        const size_t t = e / H;
-        const int i = (int)(t % N), j = (int)(t / N);
-        const double kx = (double)(i <= N / 2 ? i : i - N) * kf, ky = (double)(j <= N / 2 ? j : j - N) * kf,
-                     kz = (double)l * kf;
-        const double k = sqrt(kx * kx + ky * ky + kz * kz);
-        if (!(k > 0) || k < lo || !(k < hi)) continue;
-        int a = 0, b = nb;  // se[a] <= k < se[b]
-        while (b - a > 1) {
-            const int m = (a + b) >> 1;
-            if (se[m] <= k) a = m; else b = m;
-        }
-        size_t idx;
-        if (i <= N / 2) idx = (size_t)l + (size_t)N * ((size_t)i + (size_t)H * j);
-        else idx = (size_t)((N - l) % N) + (size_t)N * ((size_t)(N - i) + (size_t)H * ((N - j) % N));
-        const cx<T> u = F1[idx];
-        double v;
-        if (F2) {
-            const cx<T> w2 = F2[idx];
-            v = ((double)u.x * w2.x + (double)u.y * w2.y) * scale;
-        } else {
-            v = ((double)u.x * u.x + (double)u.y * u.y) * scale;
-        }
-        if (W > 0) {
-            const double k3[3] = {kx, ky, kz};
-            double win = 1;
-            for (int ax = 0; ax < 3; ax++) {
-                const double s0 = k3[ax] * dx / 2, s = s0 == 0 ? 1.0 : sin(s0) / s0;
-                win *= pow(s, 2 * W);
+    double *mine = sb + (threadIdx.x & (PK_COPIES - 1)) * 4 * nb;
+    const double t_lo = st[0], t_hi = st[nb];
+    const int runs = (H + PK_XL - 1) / PK_XL;      // runs of x per (y, z)
+    const int per_y = runs * N;                    // threads' items of a y row, z fastest
+    const int chunks = (per_y + 255) / 256, items = chunks * N;
+    for (int it = blockIdx.x; it < items; it += gridDim.x) {
+        const int y = it / chunks, q = (it - y * chunks) * 256 + threadIdx.x;
+        if (q >= per_y) continue;
+        const int run = q / N, z = q - run * N, x0 = run * PK_XL, x1 = min(x0 + PK_XL, H);
+        const int my = y <= N / 2 ? y : N - y, mz = z <= N / 2 ? z : N - z;
+        const double ky = (double)my * kf, kz = (double)mz * kf, ky2 = ky * ky, kz2 = kz * kz;
+        const bool end = z == 0 || z == N / 2;
+        const double wend = wmode == 0 && end ? 0.5 : 1.0;
+        const cx<T> *f1 = F1 + ((size_t)z + (size_t)N * H * y), *f2 = CROSS ? F2 + ((size_t)z + (size_t)N * H * y) : nullptr;
+        int b = -1;                                // the run's bin and its sums
+        double lo = 1, hi = 0, ak = 0, ap = 0, aw = 0, ac = 0;
+        auto flush = [&]() {
+            if (b < 0 || ac == 0) return;
+            if (KSUM) atomicAdd(&mine[b], ak);
+            atomicAdd(&mine[nb + b], ap);
+            atomicAdd(&mine[2 * nb + b], aw);
+            atomicAdd(&mine[3 * nb + b], ac);
+            ak = ap = aw = ac = 0;
+        };
+        // the entries of four x are loaded before the first is used
+        for (int xb = x0; xb < x1; xb += 4) {
+            cx<T> u4[4], w4[4];
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                const size_t at = (size_t)N * min(xb + d, x1 - 1);
+                u4[d] = f1[at];
+                if constexpr (CROSS) w4[d] = f2[at];
             }
-            v /= win;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                const int x = xb + d;
+                if (x >= x1) break;
+                const bool edge = x == 0 || x == N / 2;
+                const double cnt = edge ? (z <= N / 2 ? 1.0 : 0.0) : (end ? 2.0 : 1.0);
+                const double kx = (double)x * kf, s = kx * kx + ky2 + kz2;
+                if (cnt == 0 || !(s > 0) || s < t_lo || !(s < t_hi)) continue;
+                if (!(s >= lo && s < hi)) {
+                    flush();
+                    int a = 0, c = nb;                 // st[a] <= s < st[c]
+                    while (c - a > 1) {
+                        const int m = (a + c) >> 1;
+                        if (st[m] <= s) a = m; else c = m;
+                    }
+                    b = a;
+                    lo = st[a];
+                    hi = st[a + 1];
+                }
+                const cx<T> u = u4[d];
+                double v;
+                if constexpr (CROSS) {
+                    const cx<T> w2 = w4[d];
+                    v = ((double)u.x * w2.x + (double)u.y * w2.y) * scale;
+                } else {
+                    v = ((double)u.x * u.x + (double)u.y * u.y) * scale;
+                }
+                if (W > 0) v /= swin[x] * swin[my] * swin[mz];
+                const double w = cnt * wend;
+                if constexpr (KSUM) ak += cnt * sqrt(s);
+                ap += w * v;
+                aw += w;
+                ac += cnt;
+            }
         }
-        const double w = wmode == 1 ? 1.0 : ((l == 0 || l == N / 2) ? 0.5 : 1.0);
-        atomicAdd(&sk[a], k);
-        atomicAdd(&sp[a], w * v);
-        atomicAdd(&sw[a], w);
-        atomicAdd(&sc[a], 1.0);
+        flush();
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-        if (sc[b] > 0) {
-            atomicAdd(&sums[b], sk[b]);
-            atomicAdd(&sums[nb + b], sp[b]);
-            atomicAdd(&sums[2 * nb + b], sw[b]);
-            atomicAdd(&sums[3 * nb + b], sc[b]);
+    for (int b = threadIdx.x; b < nb; b += 256) {
+        double t[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < PK_COPIES; c++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) t[k] += sb[(4 * c + k) * nb + b];
+        if (t[3] > 0) {
+            if constexpr (KSUM) atomicAdd(&sums[b], t[0]);
+            atomicAdd(&sums[nb + b], t[1]);
+            atomicAdd(&sums[2 * nb + b], t[2]);
+            atomicAdd(&sums[3 * nb + b], t[3]);
         }
     }
+}
+
+// the smallest double whose square root (rounded to nearest) is at least e
+double pk_threshold(double e) {
+    if (!(e > 0)) return 0.0;
+    double s = e * e;
+    while (std::sqrt(s) < e) s = std::nextafter(s, INFINITY);
+    while (s > 0 && std::sqrt(std::nextafter(s, 0.0)) >= e) s = std::nextafter(s, 0.0);
+    return s;
 }
 
 // Per bin: k_out = mean |k| of its modes (the geometric centre sqrt(e_b e_b+1) of an empty bin, or
@@ -165,16 +221,25 @@ __global__ void k_fill_zero_d(double *p, int n) {
 
 template <typename T>
 void pk_edges(const void *F1, const void *F2, int N, double L, int W, int wmode, double scale, const PkEdges &ed,
-              double *sums, hipStream_t st) {
-    const size_t tot = (size_t)N * N * (N / 2 + 1);
-    const int blocks = (int)std::min<size_t>(4096, (tot + 255) / 256);
-    k_pk_edges<T><<<blocks, 256, 0, st>>>((const cx<T> *)F1, (const cx<T> *)F2, N, 2 * M_PI / L, L / N, W, wmode,
-                                          scale, ed, sums);
+              bool ksum, double *sums, hipStream_t st) {
+    const int nb = ed.nbins, H = N / 2 + 1;
+    PkEdges thr{};
+    thr.nbins = nb;
+    for (int b = 0; b <= nb; b++) thr.e[b] = pk_threshold(ed.e[b]);
+    const size_t shm = sizeof(double) * ((size_t)(nb + 1) + PK_COPIES * 4 * (size_t)nb + (W > 0 ? H : 0));
+    // a block's bins reach memory once, so four blocks per CU walk the rows
+    const int items = N * (((H + PK_XL - 1) / PK_XL * N + 255) / 256), blocks = std::min(1024, items);
+    auto launch = [&](auto kern) {
+        kern<<<blocks, 256, shm, st>>>((const cx<T> *)F1, (const cx<T> *)F2, N, 2 * M_PI / L, L / N, W, wmode, scale,
+                                       thr, sums);
+    };
+    if (F2) ksum ? launch(k_pk_edges<T, true, true>) : launch(k_pk_edges<T, true, false>);
+    else ksum ? launch(k_pk_edges<T, false, true>) : launch(k_pk_edges<T, false, false>);
 }
-template void pk_edges<float>(const void *, const void *, int, double, int, int, double, const PkEdges &, double *,
-                              hipStream_t);
-template void pk_edges<double>(const void *, const void *, int, double, int, int, double, const PkEdges &, double *,
-                               hipStream_t);
+template void pk_edges<float>(const void *, const void *, int, double, int, int, double, const PkEdges &, bool,
+                              double *, hipStream_t);
+template void pk_edges<double>(const void *, const void *, int, double, int, int, double, const PkEdges &, bool,
+                               double *, hipStream_t);
 
 void pk_finalize(const double *sums, const PkEdges &ed, double mult, int ncomp, bool centre_only, double *k_out,
                  double *pk_out, int64_t *nm_out, hipStream_t st) {

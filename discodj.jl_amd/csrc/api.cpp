@@ -1856,9 +1856,9 @@ void field_fft(dj_ctx *c, const void *field, void *S) {
 }
 
 void bin(dj_ctx *c, const void *F1, const void *F2, int N, int W, int wmode, double scale, const PkEdges &ed,
-         double *sums) {
-    if (c->tsize == 8) pk_edges<double>(F1, F2, N, c->cfg.boxsize, W, wmode, scale, ed, sums, c->st);
-    else pk_edges<float>(F1, F2, N, c->cfg.boxsize, W, wmode, scale, ed, sums, c->st);
+         bool ksum, double *sums) {
+    if (c->tsize == 8) pk_edges<double>(F1, F2, N, c->cfg.boxsize, W, wmode, scale, ed, ksum, sums, c->st);
+    else pk_edges<float>(F1, F2, N, c->cfg.boxsize, W, wmode, scale, ed, ksum, sums, c->st);
 }
 
 // outputs of the bins (device pk_work areas) to the host
@@ -1908,7 +1908,7 @@ dj_status dj_field_power_spectrum(dj_ctx *c, const void *field, int32_t nbins, i
     field_fft(c, c->mesh, c->B);
     const size_t B = DJ_PK_MAX_BINS;
     zero_doubles(c->pk_work, 4 * B, c->st);
-    bin(c, c->B, nullptr, N, 0, 0, V / (n3 * n3), ed, c->pk_work);
+    bin(c, c->B, nullptr, N, 0, 0, V / (n3 * n3), ed, true, c->pk_work);
     pk_finalize(c->pk_work, ed, 1.0, 1, false, c->pk_work + 4 * B, c->pk_work + 5 * B, (int64_t *)(c->pk_work + 6 * B),
                 c->st);
     return pk_download(c, nbins, k_out, pk_out, nmodes_out, nullptr);
@@ -1931,7 +1931,7 @@ dj_status dj_field_cross_power_spectrum(dj_ctx *c, const void *field1, const voi
     field_fft(c, c->mesh, c->C);
     const size_t B = DJ_PK_MAX_BINS;
     zero_doubles(c->pk_work, 4 * B, c->st);
-    bin(c, c->B, c->C, N, 0, 1, V / (n3 * n3), ed, c->pk_work);
+    bin(c, c->B, c->C, N, 0, 1, V / (n3 * n3), ed, true, c->pk_work);
     pk_finalize(c->pk_work, ed, 1.0, 1, false, c->pk_work + 4 * B, c->pk_work + 5 * B, nullptr, c->st);
     return pk_download(c, nbins, k_out, pk_out, nullptr, nullptr);
 }
@@ -1968,7 +1968,7 @@ dj_status dj_power_spectra_binned(dj_ctx *c, const void *psi, int32_t nbins, con
         c->tiles.deposit(ta, 2, false, zero3, c->mesh, 1.0, c->st);
         field_fft(c, c->mesh, c->B);
         zero_doubles(c->pk_work, 4 * B, c->st);
-        bin(c, c->B, nullptr, c->res, 2, 0, V / ((double)c->np * (double)c->np), ed, c->pk_work);
+        bin(c, c->B, nullptr, c->res, 2, 0, V / ((double)c->np * (double)c->np), ed, false, c->pk_work);
         pk_finalize(c->pk_work, ed, 1.0, 1, true, c->pk_work + 4 * B, c->pk_work + 5 * B, nullptr, c->st);
     }
     if (pk_psi_out) {
@@ -1988,7 +1988,7 @@ dj_status dj_power_spectra_binned(dj_ctx *c, const void *psi, int32_t nbins, con
             f->xf((const char *)src + (size_t)comp * c->np * c->tsize, false, A, tw, 1.0, c->st);
             f->yf(A, S, tw, c->st);
             f->zm(ZM_NONE, true, false, S, S, tw, c->kmult, c->st);
-            bin(c, S, nullptr, n, 0, 0, V / ((double)c->np * (double)c->np), ed, sums);
+            bin(c, S, nullptr, n, 0, 0, V / ((double)c->np * (double)c->np), ed, false, sums);
         }
         pk_finalize(sums, ed, 3.0, 3, true, c->pk_work + 4 * B, c->pk_work + 7 * B, nullptr, c->st);
     }
@@ -2010,7 +2010,7 @@ dj_status dj_field_power_spectrum_noalloc(dj_ctx *c, const void *d_field, int32_
     const double V = c->cfg.boxsize * c->cfg.boxsize * c->cfg.boxsize, n3 = (double)N * N * N;
     field_fft(c, d_field, c->B);
     zero_doubles(sums, 4 * nbins, c->st);
-    bin(c, c->B, nullptr, N, 0, 0, V / (n3 * n3), ed, sums);
+    bin(c, c->B, nullptr, N, 0, 0, V / (n3 * n3), ed, true, sums);
     pk_finalize(sums, ed, 1.0, 1, false, d_k_out, d_pk_out, d_nmodes_out, c->st);
     HIPCHK(c, hipGetLastError());
     return DJ_OK;

@@ -233,10 +233,11 @@ struct PkEdges {
 };
 // sums (4 nbins: sum |k|, sum w v, sum w, count) += the binned modes of the spectrum F1 (|F1|^2) or of
 // F1, F2 (Re conj(F1) F2), v scaled by scale and divided by the window of order W (0: none); wmode 0:
-// weights 1/2 on the reference's half-axis end planes, 1: unweighted
+// weights 1/2 on the reference's half-axis end planes, 1: unweighted; ksum: sum |k| too
 template <typename T>
 void pk_edges(const void *F1, const void *F2, int N, double L, int W, int wmode, double scale, const PkEdges &ed,
-              double *sums, hipStream_t st);
+              bool ksum, double *sums, hipStream_t st);
+double pk_threshold(double e);
 // k_out, pk_out = mult sum(w v) / sum(w), nm_out = count / ncomp (device pointers, each may be null)
 void pk_finalize(const double *sums, const PkEdges &ed, double mult, int ncomp, bool centre_only, double *k_out,
                  double *pk_out, int64_t *nm_out, hipStream_t st);

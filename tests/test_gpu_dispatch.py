@@ -35,3 +35,18 @@ def test_step_over_the_gather_segment_rule(res, n, prec):
     tol = 2e-5 if prec == 32 else 1e-12
     assert G.rel(pi1, mom) < tol
     assert G.rel(psi1, x + dd2 * mom) < tol
+
+
+@pytest.mark.parametrize("N, bins, log", [(16, 1, False), (24, 256, True), (96, 7, True), (128, 256, False)])
+def test_spectra_over_runs_and_bins(N, bins, log):
+    """Every mode in the oracle's bin and P(k) to 1e-10, for meshes whose x runs end short of N/2 and for one
+    bin and the most bins (many of them empty at 24^3)."""
+    L = 1.7 * N
+    f = np.random.default_rng(N).normal(size=(N, N, N))
+    with D.PMSolverHIP(D.PMConfig(res_pm=N, n_part=16, boxsize=L), precision=64) as S:
+        k, pk, nm = S.field_power_spectrum(f, bins=bins, logarithmic=log)
+    ko, pko, nmo = O.power_spectrum(f, L, bins=bins, logarithmic=log)
+    assert np.array_equal(nm, nmo)
+    assert np.allclose(k, ko, rtol=1e-12, atol=0)
+    ok = nmo > 0
+    assert np.max(np.abs(pk[ok] / pko[ok] - 1)) < 1e-10 and np.all(pk[~ok] == 0)
