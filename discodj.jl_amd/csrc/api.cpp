@@ -35,6 +35,8 @@ const char *kernel_names[K_COUNT] = {"zero", "scatter", "fft_x_r2c", "fft_y_fwd"
                                      "fft_x_c2r", "gather", "kick_drift", "drift", "bin",
                                      "bin_recount", "resample", "nn_correction", "gather_last", "kick_listed"};
 
+constexpr int REPORTS = 4;
+
 struct ProfEvent {
     int id;
     hipEvent_t a, b;
@@ -117,6 +119,7 @@ struct dj_ctx {
     void *nn_dphi = nullptr, *nn_dens = nullptr, *nn_tgt = nullptr, *nn_sum = nullptr;
     void *nn_wpart = nullptr;  // the weight gradient's per-block partial sums (NnOps::wgrad_scratch_bytes)
     void *acc_list = nullptr;  // (entries, 3): the acceleration between interlacing passes, in tile-list order
+    unsigned *report = nullptr;  // (REPORTS) pinned host words: what the kicks of the last steps saw of their sorts
     unsigned *own_at = nullptr;  // (Np): each particle's entry in its own tile list (written by the bin's fill)
     size_t acc_list_cap = 0;
     // binned spectra: bin sums and device copies of the outputs (allocated on first use)
@@ -355,6 +358,7 @@ void free_all(dj_ctx *c) {
     // teardown: failures here have no caller to report to
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    if (c->report) (void)hipHostFree(c->report);
     ic_work_free(c->icw);
     free_lists(c->tl);
     free_lists(c->tlr);
@@ -432,6 +436,7 @@ dj_status alloc_lists(dj_ctx *c, TileLists &tl, size_t ent_cap) {
     HIPCHK(c, hipMalloc(&tl.start, sizeof(unsigned) * (g.nt + 1)));
     HIPCHK(c, hipMalloc(&tl.gstart, sizeof(unsigned) * g.nt));
     HIPCHK(c, hipMalloc(&tl.flag, sizeof(unsigned)));
+    c->part.zero(tl.flag, sizeof(unsigned), c->st);
     HIPCHK(c, hipMalloc(&tl.part, sizeof(unsigned long long) * (g.nt / 1024 + 2)));
     tl.lists = false;
     tl.ent_cap = ent_cap;
@@ -450,9 +455,18 @@ void free_lists(TileLists &tl) {
 // reserved from the previous sort's counts with room to double (particles move less than a tile per step), so
 // one fill pass writes them; a list that outgrows its reserve (or a full entry buffer) raises a flag,
 // and then the sort is repeated exactly: counting pass, lists of the exact sizes, fill.
+// defer: with lists to reserve from, enqueue the sort and leave the flag to the caller, whose kernels are
+// gated by it (SortGate) and read no entry beyond a list's reserve (list_len); a set flag means
+// sort_failed() and the force again.
 dj_status tile_sort_of(dj_ctx *c, TileLists &tl, const void *psi, const void *q1, int n, const double *d_shifts,
-                       int ns, int W) {
+                       int ns, int W, bool defer = false) {
     TileArgs a = tile_args_of(c, tl, psi, q1, n, d_shifts, ns);
+    if (defer && tl.lists) {
+        Prof p(c, K_SORT);
+        c->tiles.scan(a, tl.cur, 1, c->st);
+        c->tiles.fill(a, W, c->st);
+        return check_launch(c, "tile binning");
+    }
     for (int attempt = 0; attempt < 3; attempt++) {
         const bool exact = !tl.lists || attempt > 0;
         {
@@ -490,6 +504,7 @@ dj_status tile_sort_of(dj_ctx *c, TileLists &tl, const void *psi, const void *q1
             return check_launch(c, "tile binning");
         }
         tl.lists = false;
+        c->part.zero(tl.flag, sizeof(unsigned), c->st);
         if (hv[1] > tl.ent_cap) {
             // grow the entry buffer (exact sizes follow in the next attempt)
             if (tl.ent) HIPCHK(c, hipFree(tl.ent));
@@ -504,8 +519,39 @@ dj_status tile_sort_of(dj_ctx *c, TileLists &tl, const void *psi, const void *q1
     return fail(c, DJ_ERR_DEVICE, "tile binning: lists did not fit after an exact recount");
 }
 
-dj_status tile_sort(dj_ctx *c, const void *psi, const double *d_shifts, int ns, int W) {
-    return tile_sort_of(c, c->tl, psi, c->q1, c->n, d_shifts, ns, W);
+dj_status tile_sort(dj_ctx *c, const void *psi, const double *d_shifts, int ns, int W, bool defer = false) {
+    return tile_sort_of(c, c->tl, psi, c->q1, c->n, d_shifts, ns, W, defer);
+}
+
+// after a deferred sort overflowed (the stream is idle): the next one counts first
+void sort_failed(dj_ctx *c) {
+    c->tl.lists = false;
+    c->part.zero(c->tl.flag, sizeof(unsigned), c->st);
+}
+
+// The flag of a call's first sort may wait for the end of the call where a force made in vain is cheaper
+// than the pause: a stop of the stream costs about 25 us, the force of a 128^3 mesh some 250 us, and lists
+// reserved at twice their last counts rarely overflow.  The further steps of a run, sorted from the step
+// before, defer theirs at every size.
+bool defer_first_sort(const dj_ctx *c) {
+    return c->cfg.n_resample == 1 && c->tl.lists && c->M <= ((size_t)1 << 21) && c->np <= ((int64_t)1 << 21);
+}
+
+dj_status sort_reports(dj_ctx *c) {
+    if (!c->report) HIPCHK(c, hipHostMalloc((void **)&c->report, sizeof(unsigned) * REPORTS, hipHostMallocDefault));
+    return DJ_OK;
+}
+
+// the report of a step's kick (1: its sort held, 2: it overflowed): read until the kernel has written it, or,
+// if that takes longer than any step, after the stream has ended
+unsigned wait_report(dj_ctx *c, int slot) {
+    for (long spin = 0; spin < (1l << 28); spin++) {
+        const unsigned r = __atomic_load_n(&c->report[slot], __ATOMIC_RELAXED);
+        if (r) return r;
+        if ((spin & 0xffff) == 0xffff && hipStreamQuery(c->st) != hipErrorNotReady) break;
+    }
+    (void)hipStreamSynchronize(c->st);
+    return __atomic_load_n(&c->report[slot], __ATOMIC_RELAXED);
 }
 
 // ------------------------------------------------------------------------ one force evaluation
@@ -516,7 +562,7 @@ dj_status resample_deposit(dj_ctx *c, const void *psi, const double *sh, void *d
                            void *pts = nullptr);
 void nn_forward_dev(dj_ctx *c, const void *dens, double a);
 
-dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick) {
+dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool defer = false) {
     const dj_pm_config &cfg = c->cfg;
     const bool fixed = cfg.deposit == DJ_DEPOSIT_FIXED64;
     const int ns = c->nshifts;
@@ -545,7 +591,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick) {
     const bool listed_kick = mode == FORCE_KICK && ns > 1 && !ik;
     if (listed_kick && !c->own_at) HIPCHK(c, hipMalloc(&c->own_at, sizeof(unsigned) * (size_t)c->np));
     if (!(rs_tiled && ik)) {
-        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder);
+        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
         if (rs) return rs;
     }
     (void)mesh_bytes;
@@ -1024,10 +1070,20 @@ dj_status dj_acceleration(dj_ctx *c, const void *psi, void *acc_out) {
     }
     KickArgs k{};
     k.nshifts = c->nshifts;
-    dj_status r = force(c, src, FORCE_ACC, k);
+    const bool defer = defer_first_sort(c);
+    dj_status r = defer ? sort_reports(c) : DJ_OK;
+    if (!r) r = force(c, src, FORCE_ACC, k, defer);
     if (r) return r;
+    if (defer) HIPCHK(c, hipMemcpyAsync(c->report, c->tl.flag, sizeof(unsigned), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipMemcpyAsync(acc_out, c->acc, (size_t)c->n3 * c->tsize, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
+    if (defer && c->report[0]) {
+        sort_failed(c);
+        r = force(c, src, FORCE_ACC, k);
+        if (r) return r;
+        HIPCHK(c, hipMemcpyAsync(acc_out, c->acc, (size_t)c->n3 * c->tsize, hipMemcpyDeviceToHost, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
+    }
     drain_prof(c);
     return DJ_OK;
 }
@@ -1037,9 +1093,23 @@ dj_status dj_step(dj_ctx *c, double dd1, double alpha, double beta, double dd2) 
     HIPCHK(c, hipSetDevice(c->dev));
     { Prof p(c, K_DRIFT); c->part.drift(c->psi, c->mom, c->n3, dd1, c->st); }
     KickArgs k{alpha, beta, dd2, 0.0, 0, c->nshifts};
-    dj_status r = force(c, c->psi, FORCE_KICK, k);
+    const bool defer = defer_first_sort(c);
+    if (defer) {
+        dj_status rr = sort_reports(c);
+        if (rr) return rr;
+        c->report[0] = 0;
+        k.gate = SortGate{c->tl.flag, c->report};
+    }
+    dj_status r = force(c, c->psi, FORCE_KICK, k, defer);
     if (r) return r;
     HIPCHK(c, hipStreamSynchronize(c->st));
+    if (defer && c->report[0] != 1) {
+        sort_failed(c);
+        k.gate = SortGate{};
+        r = force(c, c->psi, FORCE_KICK, k);
+        if (r) return r;
+        HIPCHK(c, hipStreamSynchronize(c->st));
+    }
     drain_prof(c);
     return DJ_OK;
 }
@@ -1056,13 +1126,37 @@ dj_status dj_run(dj_ctx *c, int32_t n_steps, const double *dd1, const double *al
     }
     if (n_steps == 0) return DJ_OK;
     { Prof p(c, K_DRIFT); c->part.drift(c->psi, c->mom, c->n3, dd1[0], c->st); }
+    // A step after the first sorts from the step before, and its overflow flag is not waited for: its kick looks
+    // at the flag and reports, and the host, at most two steps ahead, goes back to the step that reports an
+    // overflow (nothing has touched the state since) and sorts it exactly.
+    const bool ahead = c->cfg.n_resample == 1;
+    if (ahead) {
+        dj_status r = sort_reports(c);
+        if (r) return r;
+    }
+    int first = 0, known = 0;  // the step to check at once; the steps below known have held
     for (int s = 0; s < n_steps; s++) {
         if (c->nn_on && (size_t)s < c->nn_sched.size()) c->nn_a = c->nn_sched[s];
         const bool stop = wants(s + 1);
         const bool has_next = s + 1 < n_steps && !stop;
         KickArgs k{alpha[s], beta[s], dd2[s], has_next ? dd1[s + 1] : 0.0, has_next ? 1 : 0, c->nshifts};
-        dj_status r = force(c, c->psi, FORCE_KICK, k);
+        const bool defer = ahead && s > first && c->tl.lists;
+        if (defer) {
+            c->report[s % REPORTS] = 0;
+            k.gate = SortGate{c->tl.flag, c->report + s % REPORTS};
+        }
+        dj_status r = force(c, c->psi, FORCE_KICK, k, defer);
         if (r) return r;
+        if (!defer) known = s + 1;
+        const int upto = stop || s + 1 == n_steps ? s : s - 1;
+        while (known <= upto && wait_report(c, known % REPORTS) == 1) known++;
+        if (known <= upto) {
+            HIPCHK(c, hipStreamSynchronize(c->st));
+            sort_failed(c);
+            first = known;
+            s = known - 1;
+            continue;
+        }
         if (stop) {
             HIPCHK(c, hipStreamSynchronize(c->st));
             cb(s + 1, user);

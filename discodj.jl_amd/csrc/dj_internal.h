@@ -51,10 +51,28 @@ struct PartArgs {
 
 enum { GATHER_ACC = 0, GATHER_ASSIGN = 1 };
 
+// The overflow flag of the sort that a step's force was made from, for the kernels that end the step while
+// the host has not looked at the flag yet: they leave the state alone when it is set, and tell the host
+// (report: 1 + flag, a word of pinned host memory).  No flag: nothing to look at.
+struct SortGate {
+    const unsigned *flag = nullptr;
+    unsigned *report = nullptr;
+#if defined(__HIPCC__)
+    __device__ __forceinline__ bool closed() const {
+        if (!flag) return false;
+        const unsigned f = *flag;
+        if (report && blockIdx.x == 0 && threadIdx.x == 0)
+            __hip_atomic_store(report, 1u + f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return f != 0;
+    }
+#endif
+};
+
 struct KickArgs {
     double alpha, beta, dd2, dd1_next;  // FP64 step coefficients, rounded to T at use
     int has_next;                       // apply the next step's first drift in the same pass
     int nshifts;                        // interlacing passes averaged
+    SortGate gate = {};
 };
 
 struct PartOps {
@@ -103,7 +121,7 @@ struct TileArgs {
 };
 struct TileOps {
     void (*count)(const TileArgs &a, int W, hipStream_t st);  // exact counts into cnt
-    // list capacities from src (2 nt counts; may be cur), plus slack when slack != 0; zeroes cur and flag
+    // list capacities from src (2 nt counts; may be cur), plus slack when slack != 0; zeroes cur
     void (*scan)(const TileArgs &a, const unsigned *src, int slack, hipStream_t st);
     void (*fill)(const TileArgs &a, int W, hipStream_t st);
     // reverse mode: out_c = sum_p W(X_p + sh - cell) vals[p + c np] scale (3 meshes, every cell written);

@@ -133,7 +133,8 @@ __global__ __launch_bounds__(256) void k_drift_to(T *out, const T *psi, const T 
 template <typename T>
 __global__ __launch_bounds__(256) void k_kick_drift(T *__restrict__ psi, T *__restrict__ mom,
                                                     const T *__restrict__ acc, int64_t n3, T alpha, T beta,
-                                                    T dd2, T dd1n, int has_next, int ns) {
+                                                    T dd2, T dd1n, int has_next, int ns, SortGate gate) {
+    if (gate.closed()) return;
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n3) return;
     T a = acc[i];
@@ -193,7 +194,7 @@ static void drift_to(void *out, const void *psi, const void *mom, void *ck_psi, 
 template <typename T>
 static void kick_drift(void *psi, void *mom, const void *acc, int64_t n3, const KickArgs &k, hipStream_t st) {
     k_kick_drift<T><<<lgrid(n3), 256, 0, st>>>((T *)psi, (T *)mom, (const T *)acc, n3, (T)k.alpha, (T)k.beta,
-                                               (T)k.dd2, (T)k.dd1_next, k.has_next, k.nshifts);
+                                               (T)k.dd2, (T)k.dd1_next, k.has_next, k.nshifts, k.gate);
 }
 
 template <typename T>

@@ -322,7 +322,8 @@ __global__ __launch_bounds__(256) void k_tile_bin(const T *__restrict__ psi, con
 // some list almost surely grows by more than a quarter between steps; memory is plentiful):
 // start[t] = sum_{u<t} capacities, gstart[t] = start[t] + own capacity, start[nt] = total reserved.
 // Three parallel kernels: per-block sums, a scan of the block sums, per-block scan and write-out
-// (which also clears the cursors, after reading them when src is cur, and the overflow flag).
+// (which also clears the cursors, after reading them when src is cur).  The overflow flag stays set until
+// the host clears it.
 __device__ __forceinline__ unsigned list_cap(unsigned c, int slack) { return slack ? 2 * c + 64 : c; }
 
 constexpr int SCAN_TILES = 1024;  // tiles per block of the scan (4 per thread)
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(1024) void k_scan_top(unsigned long long *part, int
     if (i < nb) part[i] = v[i] - x;
     if (i == 1023) {
         start[nt] = (unsigned)min(v[1023], 0xffffffffull);
-        flag[0] = v[1023] > 0xffffffffull ? 1u : 0u;
+        if (v[1023] > 0xffffffffull) flag[0] = 1u;
     }
 }
 
@@ -401,6 +402,63 @@ __global__ __launch_bounds__(256) void k_scan_write(const unsigned *src, int nt,
         cur[t] = 0;
         cur[nt + t] = 0;
     }
+}
+
+// The three kernels' work by one workgroup, for meshes of up to SCAN_ONE tiles: thread i takes the tiles
+// [i per, (i + 1) per).  At 64 tiles the three launches take 9 us, this one 4.
+constexpr int SCAN_ONE = 8192;
+
+__global__ __launch_bounds__(1024) void k_scan_one(const unsigned *src, int nt, int slack, unsigned *__restrict__ start,
+                                                   unsigned *__restrict__ gstart, unsigned *cur, unsigned *flag) {
+    constexpr int PER = SCAN_ONE / 1024;
+    __shared__ unsigned long long wsum[16];
+    const int per = (nt + 1023) / 1024, t0 = threadIdx.x * per, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned co[PER], cg[PER];
+    unsigned long long s = 0;
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const bool on = k < per && t0 + k < nt;
+        co[k] = on ? list_cap(src[t0 + k], slack) : 0u;
+        cg[k] = on ? list_cap(src[nt + t0 + k], slack) : 0u;
+        s += (unsigned long long)co[k] + cg[k];
+    }
+    unsigned long long v = s;
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long y = __shfl_up(v, off);
+        if (lane >= off) v += y;
+    }
+    if (lane == 63) wsum[wave] = v;
+    __syncthreads();
+    unsigned long long before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+        if (w < wave) before += wsum[w];
+        total += wsum[w];
+    }
+    unsigned long long run = before + v - s;
+    // src may be cur: this thread read its tiles' counts above, before clearing them here
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int t = t0 + k;
+        if (k >= per || t >= nt) break;
+        start[t] = (unsigned)run;
+        gstart[t] = (unsigned)(run + co[k]);
+        run += (unsigned long long)co[k] + cg[k];
+        cur[t] = 0;
+        cur[nt + t] = 0;
+    }
+    if (threadIdx.x == 0) {
+        start[nt] = (unsigned)min(total, 0xffffffffull);
+        if (total > 0xffffffffull) flag[0] = 1u;
+    }
+}
+
+// Entries of a list of cnt entries that lie in its reserve [begin, end) and in the buffer of cap entries:
+// all of them, except after a sort that overflowed and has not been repeated yet (the fill's cursors then
+// count entries that it did not write)
+__device__ __forceinline__ unsigned list_len(unsigned cnt, unsigned begin, unsigned end, unsigned cap) {
+    end = min(end, cap);
+    return begin < end ? min(cnt, end - begin) : 0u;
 }
 
 // ------------------------------------------------------------------------------------ deposit
@@ -448,8 +506,8 @@ __device__ __forceinline__ void dep_add(Acc *a, T wx, T wy, T wz, T wyz, double 
 template <typename T, int W, int ACC, bool PAD>
 __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
                                              const unsigned *__restrict__ gstart, const unsigned *__restrict__ cnt,
-                                             const TileGeom &g, T sx, T sy, T sz, T L, void *mesh, double fscale,
-                                             int qbits) {
+                                             unsigned cap, const TileGeom &g, T sx, T sy, T sz, T L, void *mesh,
+                                             double fscale, int qbits) {
     using Acc = typename std::conditional<ACC == ACC_T, T,
                                           typename std::conditional<ACC == ACC_Q32, unsigned, unsigned long long>::type>::type;
     extern __shared__ unsigned char smem[];
@@ -462,7 +520,8 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
     const int ox = tx << g.lT[0], oy = ty << g.lT[1], oz = tz << g.lT[2];
     __syncthreads();
     // the tile's own list, then its ghost list
-    const unsigned n_own = cnt[t], n_all = n_own + cnt[g.nt + t], s_own = start[t], s_gh = gstart[t] - n_own;
+    const unsigned s_own = start[t], g0 = gstart[t], n_own = list_len(cnt[t], s_own, g0, cap),
+                   n_all = n_own + list_len(cnt[g.nt + t], g0, start[t + 1], cap), s_gh = g0 - n_own;
     const int o3[3] = {ox, oy, oz}, T3[3] = {g.TX, g.TY, g.TZ};
     for (unsigned i = threadIdx.x; i < n_all; i += blockDim.x) {
         const Entry<T> en = ent[i < n_own ? s_own + i : s_gh + i];
@@ -563,16 +622,17 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
 template <typename T, int W, int ACC, bool PAD>
 __global__ __launch_bounds__(512) void k_tile_deposit(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
                                                       const unsigned *__restrict__ gstart, const unsigned *__restrict__ cnt,
-                                                      TileGeom g, T sx, T sy, T sz, T L, void *mesh, double fscale) {
+                                                      unsigned cap, TileGeom g, T sx, T sy, T sz, T L, void *mesh,
+                                                      double fscale) {
     if constexpr (ACC == ACC_Q31) {
         const unsigned t = blockIdx.x, e = cnt[t] + cnt[g.nt + t];
         const int qbits = 32 - (32 - __clz(e));  // 32 - bits(e): e 2^qbits < 2^32
         if (qbits >= Q32_MIN_BITS) {
-            tile_deposit<T, W, ACC_Q32, PAD>(ent, start, gstart, cnt, g, sx, sy, sz, L, mesh, fscale, min(qbits, 31));
+            tile_deposit<T, W, ACC_Q32, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, min(qbits, 31));
             return;
         }
     }
-    tile_deposit<T, W, ACC, PAD>(ent, start, gstart, cnt, g, sx, sy, sz, L, mesh, fscale, 31);
+    tile_deposit<T, W, ACC, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, 31);
 }
 
 // Vector deposit (reverse mode): out_c(cell) = sum_p W(X_p + s - cell) vals[p + c np] scale for c = 0, 1, 2,
@@ -1048,8 +1108,9 @@ __device__ __forceinline__ void stage_groups(const T *phi, T *ph, const int (&r0
 
 template <typename T, int W, int ORDER, int MODE, bool FG>
 __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>())) void k_tile_gather(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
-                                                      const unsigned *__restrict__ own, TileGeom g, T sx, T sy, T sz,
-                                                      T L, const T *__restrict__ phi, T c1, T c2, T c3,
+                                                      const unsigned *__restrict__ gstart, const unsigned *__restrict__ own,
+                                                      unsigned cap, TileGeom g, T sx, T sy, T sz, T L,
+                                                      const T *__restrict__ phi, T c1, T c2, T c3,
                                                       T *__restrict__ acc, size_t np, int lacc) {
     constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
     extern __shared__ unsigned char smem[];
@@ -1066,7 +1127,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
     const bool region_ok = q.ok;
 
     // this thread's first particle and its state, loaded before the staging so both are in flight together
-    const unsigned e0 = start[t], e1 = e0 + own[t];
+    const unsigned e0 = start[t], e1 = e0 + list_len(own[t], e0, gstart[t], cap);
     unsigned e = e0 + threadIdx.x;
     Entry<T> en{};
     T a3[3] = {0, 0, 0};
@@ -1176,8 +1237,8 @@ __device__ __forceinline__ void march_segment(int b, const TileGeom &g, const Ma
 
 template <typename T, int W, int ORDER, int MODE>
 __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>())) void k_tile_gather_march(
-    const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start, const unsigned *__restrict__ own, TileGeom g,
-    T sx, T sy, T sz, T L, const T *__restrict__ phi, T c1, T c2, T c3, T *__restrict__ acc, size_t np, int lacc,
+    const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start, const unsigned *__restrict__ gstart,
+    const unsigned *__restrict__ own, unsigned cap, TileGeom g, T sx, T sy, T sz, T L, const T *__restrict__ phi, T c1, T c2, T c3, T *__restrict__ acc, size_t np, int lacc,
     MarchMap m) {
     constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
     extern __shared__ unsigned char smem[];
@@ -1198,7 +1259,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
         const int tz = tz0 + it;
         const int t = tx + g.ntx * (ty + g.nty * tz);
         const int r0[3] = {rx, ry, tz * TZ - q.lo[2]};
-        const unsigned e0 = start[t], e1 = e0 + own[t];
+        const unsigned e0 = start[t], e1 = e0 + list_len(own[t], e0, gstart[t], cap);
         unsigned e = e0 + part * NT + threadIdx.x;
         Entry<T> en{};
         T a3[3] = {0, 0, 0};
@@ -1275,7 +1336,8 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
 template <typename T>
 __global__ __launch_bounds__(256) void k_kick_listed(const unsigned *__restrict__ own_at, const T *__restrict__ accl,
                                                      T *__restrict__ psi, T *__restrict__ mom, size_t np, T alpha,
-                                                     T beta, T dd2, T dd1n, int has_next, int ns) {
+                                                     T beta, T dd2, T dd1n, int has_next, int ns, SortGate gate) {
+    if (gate.closed()) return;
     const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
     const size_t e = 3 * (size_t)own_at[p];
@@ -1291,6 +1353,8 @@ __global__ __launch_bounds__(256) void k_kick_listed(const unsigned *__restrict_
 }
 
 // ------------------------------------------------------------------------------------ launchers
+static unsigned cap32(const TileArgs &a) { return (unsigned)std::min<size_t>(a.ent_cap, 0xffffffffu); }
+
 template <typename T>
 struct TileLaunch {
     template <int W>
@@ -1311,6 +1375,10 @@ struct TileLaunch {
         if (W == 2) bin_w<2>(a, st); else if (W == 3) bin_w<3>(a, st); else bin_w<4>(a, st);
     }
     static void scan(const TileArgs &a, const unsigned *src, int slack, hipStream_t st) {
+        if (a.g.nt <= SCAN_ONE) {
+            k_scan_one<<<1, 1024, 0, st>>>(src, a.g.nt, slack, a.start, a.gstart, a.cur, a.flag);
+            return;
+        }
         const int nb = (a.g.nt + SCAN_TILES - 1) / SCAN_TILES;  // <= 1024 (nt <= 2^20)
         k_scan_sums<<<nb, 256, 0, st>>>(src, a.g.nt, slack, a.scan_part);
         k_scan_top<<<1, 1024, 0, st>>>(a.scan_part, nb, a.start, a.g.nt, a.flag);
@@ -1330,7 +1398,7 @@ struct TileLaunch {
         // 512 threads: the four workgroups that the accumulators' LDS allows per CU then hold the
         // CU's full 32 waves, twice as many LDS atomics in flight as with 256 (2.97 -> 2.56 ms at
         // 512^3 on 1024^3, TSC)
-        kern<<<g.nt, 512, shm, st>>>((const Entry<T> *)a.ent, a.start, a.gstart, a.cur, g, (T)sh[0], (T)sh[1],
+        kern<<<g.nt, 512, shm, st>>>((const Entry<T> *)a.ent, a.start, a.gstart, a.cur, cap32(a), g, (T)sh[0], (T)sh[1],
                                      (T)sh[2], (T)a.L, mesh, fscale);
     }
     template <int W>
@@ -1395,7 +1463,7 @@ struct TileLaunch {
         size_t shm = q.ok ? sizeof(T) * (size_t)q.s[0] * q.s[1] * q.s[2] : sizeof(T);
         auto kern = k_tile_gather<T, W, O, M, FG>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-        kern<<<a.g.nt, gather_threads<T, W>(), shm, st>>>((const Entry<T> *)a.ent, a.start, a.cur, a.g, (T)sh[0], (T)sh[1], (T)sh[2],
+        kern<<<a.g.nt, gather_threads<T, W>(), shm, st>>>((const Entry<T> *)a.ent, a.start, a.gstart, a.cur, cap32(a), a.g, (T)sh[0], (T)sh[1], (T)sh[2],
                                         (T)a.L, (const T *)phi, (T)c[0], (T)c[1], (T)c[2], (T *)a.acc,
                                         (size_t)a.n * a.n * a.n, a.acc_by_entry);
     }
@@ -1408,7 +1476,8 @@ struct TileLaunch {
         auto kern = k_tile_gather_march<T, W, O, M>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         kern<<<a.g.nt / mm.G * mm.parts, gather_threads<T, W>(), shm, st>>>(
-            (const Entry<T> *)a.ent, a.start, a.cur, a.g, (T)sh[0], (T)sh[1], (T)sh[2], (T)a.L, (const T *)phi,
+            (const Entry<T> *)a.ent, a.start, a.gstart, a.cur, cap32(a), a.g, (T)sh[0], (T)sh[1], (T)sh[2], (T)a.L,
+            (const T *)phi,
             (T)c[0], (T)c[1], (T)c[2], (T *)a.acc, (size_t)a.n * a.n * a.n, a.acc_by_entry, mm);
     }
     template <int W, int O, int M>
@@ -1446,7 +1515,7 @@ static void kick_listed_l(const unsigned *own_at, const void *acc_list, void *ps
                           const KickArgs &k, hipStream_t st) {
     k_kick_listed<T><<<(unsigned)((np + 255) / 256), 256, 0, st>>>(own_at, (const T *)acc_list, (T *)psi, (T *)mom, np,
                                                                    (T)k.alpha, (T)k.beta, (T)k.dd2, (T)k.dd1_next,
-                                                                   k.has_next, k.nshifts);
+                                                                   k.has_next, k.nshifts, k.gate);
 }
 
 template <typename T> void tile_ops(TileOps &ops) {

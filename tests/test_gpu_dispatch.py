@@ -50,3 +50,89 @@ def test_spectra_over_runs_and_bins(N, bins, log):
     assert np.allclose(k, ko, rtol=1e-12, atol=0)
     ok = nmo > 0
     assert np.max(np.abs(pk[ok] / pko[ok] - 1)) < 1e-10 and np.all(pk[~ok] == 0)
+
+
+def _collapse(n, L, dt):
+    """Momenta that carry every particle close to the box centre at time 1, a little apart."""
+    q = np.arange(n) * (L / n)
+    q3 = np.stack([np.broadcast_to(v, (n, n, n)) for v in (q, q[:, None], q[:, None, None])])
+    return (0.97 * (L / 2 - q3)).astype(dt)
+
+
+@pytest.mark.parametrize("aa, prec, grad", [(0, 32, 2), (1, 32, 4), (1, 64, 2), (0, 64, 0)])
+def test_run_resumes_at_a_sort_that_overflows(aa, prec, grad):
+    """Particles that pile up in a few tiles between two steps of a run overflow the lists reserved from the
+    step before; the run goes back to that step.  The same steps one at a time, each call on a new solver
+    (whose first sort counts), give the same state: bit for bit in FP32, whose deposit sums in integers, to
+    1e-11 in FP64, whose atomics add in any order."""
+    n, res, L, steps = 32, 64, 100.0, 6
+    dt = np.float32 if prec == 32 else np.float64
+    psi, pi = 0.5 * _psi(n, 1.0, 5, dt), _collapse(n, L, dt)
+    cfg = D.PMConfig(res_pm=res, n_part=n, boxsize=L, grad_order=grad, antialias=aa)
+    dd1, dd2 = np.full(steps, 0.125), np.full(steps, 0.125)
+    alpha, beta = np.full(steps, 0.99), np.full(steps, 1e-3)
+    with D.PMSolverHIP(cfg, precision=prec) as S:
+        S.set_state(psi, pi)
+        S.run(dd1, alpha, beta, dd2)
+        got = S.get_state()
+        seen = []
+        S.set_state(psi, pi)
+        S.run(dd1, alpha, beta, dd2, want=[0, 0, 1, 0, 1, 0, 0], callback=lambda k: seen.append((k, S.get_state())))
+        again = S.get_state()
+    ref, refs = (psi, pi), []
+    for s in range(steps):
+        with D.PMSolverHIP(cfg, precision=prec) as S:
+            S.set_state(*ref)
+            S.step(dd1[s], alpha[s], beta[s], dd2[s])
+            ref = S.get_state()
+            refs.append(ref)
+    tol = 0 if prec == 32 else 1e-11
+    for a, b in ((got, ref), (again, ref), (seen[0][1], refs[1]), (seen[1][1], refs[3])):
+        assert G.rel(a[0], b[0]) <= tol and G.rel(a[1], b[1]) <= tol
+    assert [k for k, _ in seen] == [2, 4]
+
+
+@pytest.mark.parametrize("prec", [32, 64])
+def test_calls_after_a_state_that_does_not_fit_the_lists(prec):
+    """A force and a step of collapsed particles on a solver whose lists are reserved for uniform ones, against
+    a new solver's (bit for bit in FP32, 1e-11 in FP64)."""
+    n, res, L = 32, 64, 100.0
+    dt = np.float32 if prec == 32 else np.float64
+    psi = 0.5 * _psi(n, 1.0, 6, dt)
+    piled = (psi + _collapse(n, L, dt)).astype(dt)
+    pi = _psi(n, 0.1, 7, dt)
+    cfg = D.PMConfig(res_pm=res, n_part=n, boxsize=L)
+    with D.PMSolverHIP(cfg, precision=prec) as S:
+        S.pm_acceleration(psi)
+        acc = S.pm_acceleration(piled)
+        back = S.pm_acceleration(psi)
+        S.set_state(piled, pi)
+        S.step(0.0, 0.9, 0.1, 0.2)
+        st = S.get_state()
+    with D.PMSolverHIP(cfg, precision=prec) as S:
+        acc0 = S.pm_acceleration(piled)
+    with D.PMSolverHIP(cfg, precision=prec) as S:
+        back0 = S.pm_acceleration(psi)
+        S.set_state(piled, pi)
+    with D.PMSolverHIP(cfg, precision=prec) as S:
+        S.set_state(piled, pi)
+        S.step(0.0, 0.9, 0.1, 0.2)
+        st0 = S.get_state()
+    tol = 0 if prec == 32 else 1e-11
+    assert G.rel(acc, acc0) <= tol and G.rel(back, back0) <= tol
+    assert G.rel(st[0], st0[0]) <= tol and G.rel(st[1], st0[1]) <= tol
+
+
+@pytest.mark.parametrize("res, n, prec", [(256, 40, 32), (384, 40, 32), (192, 40, 64)])
+def test_sort_over_the_scan_rule(res, n, prec):
+    """Meshes on both sides of the one-workgroup scan (4096, 13824 and 1728 tiles): the deposit of two calls,
+    the second from reserved lists, against the oracle's in the same precision (an FP64 one would count the
+    rounding of the FP32 positions, up to 384 x 2^-23 of a cell)."""
+    L = 1.5 * res
+    dt = np.float32 if prec == 32 else np.float64
+    psi = _psi(n, 2.0, res, dt)
+    with D.PMSolverHIP(D.PMConfig(res_pm=res, n_part=n, boxsize=L), precision=prec) as S:
+        S.deposit(psi)
+        m = S.deposit(psi)
+    ref = O.pm_scatter(O.lagrangian_positions(psi, L), res, L, 2)
+    assert G.rel(m, ref) < (2e-5 if prec == 32 else 1e-12)
