@@ -29,9 +29,9 @@ namespace {
 
 thread_local std::string g_create_error;
 
-enum KernelId { K_ZERO = 0, K_SCATTER, K_XF, K_YF, K_ZM, K_YI, K_XI, K_GATHER, K_KICK, K_DRIFT, K_SORT,
+enum KernelId { K_SCATTER = 0, K_XF, K_YF, K_ZM, K_YI, K_XI, K_GATHER, K_KICK, K_DRIFT, K_SORT,
                 K_SORT_EXACT, K_RESAMPLE, K_NN, K_GATHER_LAST, K_KICK_LISTED, K_COUNT };
-const char *kernel_names[K_COUNT] = {"zero", "scatter", "fft_x_r2c", "fft_y_fwd", "fft_z_mult", "fft_y_inv",
+const char *kernel_names[K_COUNT] = {"scatter", "fft_x_r2c", "fft_y_fwd", "fft_z_mult", "fft_y_inv",
                                      "fft_x_c2r", "gather", "kick_drift", "drift", "bin",
                                      "bin_recount", "resample", "nn_correction", "gather_last", "kick_listed"};
 
@@ -372,7 +372,6 @@ void set_bytes(dj_ctx *c) {
     const double T = c->tsize, M = (double)c->M, HC = (double)c->HC, np = (double)c->np;
     // algorithmic bytes per launch: what the operation must read and write at least, with the
     // particle positions counted as 3 values per particle (the tile lists are this library's choice)
-    c->bytes[K_ZERO] = 3 * T * np;
     c->bytes[K_SCATTER] = 3 * T * np + M * (c->cfg.deposit == DJ_DEPOSIT_FIXED64 ? 8 : T);
     c->bytes[K_XF] = M * (c->cfg.deposit == DJ_DEPOSIT_FIXED64 ? 8 : T) + 2 * T * HC;
     c->bytes[K_YF] = 4 * T * HC;
@@ -569,31 +568,16 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
     const size_t mesh_bytes = c->M * (fixed ? 8 : c->tsize);
     void *dens = fixed ? c->meshfix : c->mesh;
     const double fscale = std::ldexp(1.0, -(cfg.fixed_frac_bits ? cfg.fixed_frac_bits : 32));
-    PartArgs pa{};
-    pa.psi = psi;
-    pa.mom = c->mom;
-    pa.acc = c->acc;
-    pa.q1 = c->q1;
-    pa.n = c->n;
-    pa.res = c->res;
-    pa.L = cfg.boxsize;
     const bool ik = cfg.grad_order == 0;
-    // the ik path accumulates the components into acc; the FD path assigns it in its first pass
-    if (ik) {
-        Prof p(c, K_ZERO);
-        c->part.zero(c->acc, (size_t)c->n3 * c->tsize, c->st);
-    }
     // the point sets of sheet resampling deposited together through their own tile lists (the particles'
-    // lists then serve only a finite-difference gather)
+    // lists then serve only the gather)
     const bool rs_tiled = cfg.n_resample > 1 && c->rs_tiled;
     // with interlacing the last pass adds its force into the list-ordered hand-over and the kick runs in
     // particle order (k_kick_listed), reading the sum through the own-list entry the bin records
     const bool listed_kick = mode == FORCE_KICK && ns > 1 && !ik;
     if (listed_kick && !c->own_at) HIPCHK(c, hipMalloc(&c->own_at, sizeof(unsigned) * (size_t)c->np));
-    if (!(rs_tiled && ik)) {
-        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
-        if (rs) return rs;
-    }
+    dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
+    if (rs) return rs;
     (void)mesh_bytes;
     // in a step the passes hand the acceleration over in tile-list order: both walk the same lists, so
     // the hand-over is read and written contiguously instead of at the particles' positions
@@ -605,9 +589,6 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
         c->acc_list_cap = c->tl.ent_cap;
     }
     for (int s = 0; s < ns; s++) {
-        pa.shift[0] = c->shifts[s][0];
-        pa.shift[1] = c->shifts[s][1];
-        pa.shift[2] = c->shifts[s][2];
         TileArgs ta = tile_args(c, psi, c->d_shifts, ns);
         if (lacc) {
             ta.acc = c->acc_list;
@@ -671,7 +652,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
                 { Prof p(c, K_YI); c->fft.yi(c->C, c->A, c->tw, c->st); }
                 { Prof p(c, K_XI); c->fft.xi(c->A, c->mesh, c->tw, c->st); }
                 Prof p(c, K_GATHER);
-                c->part.gather_comp(pa, cfg.worder, c->mesh, ax, c->st);
+                c->tiles.gather_comp(ta, cfg.worder, c->shifts[s], c->mesh, s == 0 ? GATHER_ASSIGN : GATHER_ACC, ax, c->st);
             }
         }
         dj_status r = check_launch(c, "force pass");
@@ -1181,19 +1162,14 @@ static dj_status deposit_mesh(dj_ctx *c, const void *psi, const double *shift, v
         HIPCHK(c, hipMemcpyAsync(c->psi_in, psi, (size_t)c->n3 * c->tsize, hipMemcpyHostToDevice, c->st));
         src = c->psi_in;
     }
-    PartArgs pa{};
-    pa.psi = src;
-    pa.q1 = c->q1;
-    pa.n = c->n;
-    pa.res = c->res;
-    pa.L = c->cfg.boxsize;
-    for (int a = 0; a < 3; a++) pa.shift[a] = shift ? shift[a] : 0.0;
+    double sh[3];
+    for (int k = 0; k < 3; k++) sh[k] = shift ? shift[k] : 0.0;
     void *dens = fixed ? c->meshfix : c->mesh;
-    HIPCHK(c, hipMemcpyAsync(c->d_shifts + 48, pa.shift, sizeof(double) * 3, hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, hipMemcpyAsync(c->d_shifts + 48, sh, sizeof(double) * 3, hipMemcpyHostToDevice, c->st));
     dj_status r = tile_sort(c, src, c->d_shifts + 48, 1, c->cfg.worder);
     if (r) return r;
     TileArgs ta = tile_args(c, src, c->d_shifts + 48, 1);
-    { Prof p(c, K_SCATTER); c->tiles.deposit(ta, c->cfg.worder, fixed, pa.shift, dens, fscale_dep(c->cfg), c->st); }
+    { Prof p(c, K_SCATTER); c->tiles.deposit(ta, c->cfg.worder, fixed, sh, dens, fscale_dep(c->cfg), c->st); }
     *dens_out = dens;
     return check_launch(c, "deposit");
 }
@@ -1880,12 +1856,6 @@ dj_status dj_power_spectrum(dj_ctx *c, const void *psi, int32_t W, int32_t nbins
         HIPCHK(c, hipMemcpyAsync(c->psi_in, psi, (size_t)c->n3 * c->tsize, hipMemcpyHostToDevice, c->st));
         src = c->psi_in;
     }
-    PartArgs pa{};
-    pa.psi = src;
-    pa.q1 = c->q1;
-    pa.n = c->n;
-    pa.res = c->res;
-    pa.L = c->cfg.boxsize;
     const double zero3[3] = {0, 0, 0};
     HIPCHK(c, hipMemcpyAsync(c->d_shifts + 48, zero3, sizeof(double) * 3, hipMemcpyHostToDevice, c->st));
     dj_status rs = tile_sort(c, src, c->d_shifts + 48, 1, dw);

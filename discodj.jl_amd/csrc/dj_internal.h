@@ -38,17 +38,6 @@ struct FftOps {
 template <typename T> bool fft_dispatch(int N, FftOps &ops);
 
 // particle-side kernels (particles.hip)
-struct PartArgs {
-    const void *psi;      // (3, Np) displacement, component-major
-    void *mom;            // (3, Np) momentum
-    void *acc;            // (3, Np) acceleration accumulator
-    const void *q1;       // (n) Lagrangian lattice coordinates (i * L/n in FP64, rounded to T)
-    int n;                // particles per side
-    int res;              // mesh cells per side
-    double L;             // box size
-    double shift[3];      // interlacing shift of this pass
-};
-
 enum { GATHER_ACC = 0, GATHER_ASSIGN = 1 };
 
 // The overflow flag of the sort that a step's force was made from, for the kernels that end the step while
@@ -76,8 +65,6 @@ struct KickArgs {
 };
 
 struct PartOps {
-    // gather one component of a mesh field at X into acc[comp] (+=)
-    void (*gather_comp)(const PartArgs &a, int W, const void *field, int comp, hipStream_t st);
     // psi += dd * mom
     void (*drift)(void *psi, const void *mom, int64_t n3, double dd, hipStream_t st);
     // out = psi + dd * mom (out may be psi); psi and mom also copied to ck_psi, ck_mom when both are non-null
@@ -133,6 +120,9 @@ struct TileOps {
                     hipStream_t st);
     void (*gather)(const TileArgs &a, int W, int order, const double *shift, const void *phi, const double *c,
                    int mode, hipStream_t st);
+    // acc[comp] at the particles = or += (mode) the interpolation of the mesh f
+    void (*gather_comp)(const TileArgs &a, int W, const double *shift, const void *f, int mode, int comp,
+                        hipStream_t st);
     // the kick and drifts of a step in particle order, the force summed over the ns passes in list order
     // (acc_list[3 e + c], e = own_at[p]): mom = alpha mom + beta acc / ns, psi += (dd2 + dd1n) steps of mom
     void (*kick_listed)(const unsigned *own_at, const void *acc_list, void *psi, void *mom, size_t np,

@@ -17,75 +17,13 @@
 #include <hip/hip_runtime.h>
 
 #include "dj_internal.h"
+#include "stencil.h"
 
 namespace dj {
 
 template <typename T> struct Entry;
 template <> struct alignas(16) Entry<float> { float x, y, z; int idx; };
 template <> struct alignas(16) Entry<double> { double x, y, z; int idx; int pad; };
-
-// Julia's float mod(x, L) for L > 0.  On [-L, 2L) it is computed without fmod: there fmod returns x,
-// x - L (exact, Sterbenz) or x (for -L < x < 0, then shifted by L), and every branch below gives
-// the same bits as the general rule (rem, then + L for a negative remainder, +0 for a zero one).
-// The three in-range cases are computed with the same operations and selected without branches;
-// only positions outside [-L, 2L) take the general path.
-template <typename T> __device__ __noinline__ T tjmod_general(T x, T L) {
-    T r = fmod(x, L);
-    if (r == (T)0) return copysign(r, L);
-    if ((r > (T)0) != (L > (T)0)) return r + L;
-    return r;
-}
-template <typename T> __device__ __forceinline__ T tjmod(T x, T L) {
-    T r = x + (T)0;            // [0, L): + 0 turns -0 into +0, as copysign(0, L) does
-    if (x >= L) r = x - L;     // [L, 2L)
-    if (x < (T)0) r = x + L;   // [-L, 0)
-    if (__builtin_expect(x < -L || x >= (T)2 * L, 0)) r = tjmod_general(x, L);
-    return r;
-}
-// a mod n for a in [-n, 2n)
-__device__ __forceinline__ int wrapn(int a, int n) { return a < 0 ? a + n : (a >= n ? a - n : a); }
-template <int W, typename T> __device__ __forceinline__ int twbase(T g) {
-    return (W % 2 == 0) ? (int)floor(g) : (int)rint(g);
-}
-template <int W> __device__ __forceinline__ constexpr int twlo() { return W == 2 ? 0 : -1; }
-__device__ __forceinline__ int timod(int a, int n) {
-    int r = a % n;
-    return r < 0 ? r + n : r;
-}
-// 1-D assignment weights (pm.jl:49-51).  Every piece is evaluated with the reference's operations
-// and the applicable one selected, so the code has no branches and the values are the same bits.
-template <int W, typename T> __device__ __forceinline__ T twk(T d) {
-    if constexpr (W == 2) {
-        const T a = (T)1 - d;
-        return d > (T)1 ? (T)0 : a;
-    } else if constexpr (W == 3) {
-        const T t = (T)1.5 - d;
-        const T outer = (T)0.5 * (t * t), inner = (T)0.75 - d * d;
-        return d > (T)1.5 ? (T)0 : (d > (T)0.5 ? outer : inner);
-    } else {
-        const T t = (T)2 - d;
-        const T outer = t * t * t / (T)6;
-        const T inner = ((T)4 - (T)6 * (d * d) + (T)3 * (d * d * d)) / (T)6;
-        return d > (T)2 ? (T)0 : (d > (T)1 ? outer : inner);
-    }
-}
-
-// The weight of stencil cell o (0 <= o < W) at d = |g - (b + lo + o)|, b the base cell of g.  Each
-// cell's d stays in one piece of the window, so only that piece is evaluated: TSC (b = round(g),
-// |g - b| <= 1/2) has d <= 1/2 at the centre (inner piece) and 1/2 <= d <= 3/2 at the sides (outer
-// piece; at d = 1/2 both pieces give 1/2 and at d = 3/2 the outer one gives the reference's 0); CIC
-// (b = floor(g)) has d <= 1, where the weight is 1 - d.  The values are the same bits as twk's.
-template <int W, typename T> __device__ __forceinline__ T twk_at(int o, T d) {
-    if constexpr (W == 3) {
-        if (o == 1) return (T)0.75 - d * d;
-        const T t = (T)1.5 - d;
-        return (T)0.5 * (t * t);
-    } else if constexpr (W == 2) {
-        return (T)1 - d;
-    } else {
-        return twk<W>(d);
-    }
-}
 
 // ------------------------------------------------------------------------------------ binning
 constexpr unsigned EMPTY = 0xffffffffu;
@@ -952,15 +890,32 @@ template <typename T, int W> constexpr int gather_threads() { return sizeof(T) =
 // waves per SIMD the register allocation must allow: two FP32 workgroups per CU (128 VGPRs)
 template <typename T, int W> constexpr int gather_min_waves() { return sizeof(T) == 4 && W <= 3 ? 4 : 1; }
 
-// a particle's tile entry and, when its gather adds to earlier passes, their sum
-template <typename T, int MODE>
+// The plain interpolation of a mesh (the spectral gradient's force meshes), summed over the cells in x, y, z order
+template <typename T, int W, typename LD>
+__device__ __forceinline__ T gather_sum(const LD &ld, const T (&w)[3][W]) {
+    T s = 0;
+#pragma unroll
+    for (int oz = 0; oz < W; oz++)
+#pragma unroll
+        for (int oy = 0; oy < W; oy++)
+#pragma unroll
+            for (int ox = 0; ox < W; ox++) s += ld(ox, oy, oz) * (w[0][ox] * w[1][oy] * w[2][oz]);
+    return s;
+}
+
+// What a gather of FD order ORDER makes per particle: the three components of -D phi, or for ORDER 0 the
+// interpolation of the mesh itself (one value)
+constexpr int gather_values(int order) { return order == 0 ? 1 : 3; }
+
+// a particle's tile entry and, when its gather adds to earlier passes, their sums
+template <typename T, int MODE, int NC>
 __device__ __forceinline__ void gather_fetch(const Entry<T> *__restrict__ ent, unsigned e, const T *__restrict__ acc,
-                                             size_t np, int lacc, Entry<T> &en, T (&a3)[3]) {
+                                             size_t np, int lacc, Entry<T> &en, T (&a3)[NC]) {
     en = ent[e];
     if constexpr (MODE == GATHER_ACC) {
-        const size_t ai = lacc ? 3 * (size_t)e : (size_t)en.idx, as = lacc ? 1 : np;
+        const size_t ai = lacc ? NC * (size_t)e : (size_t)en.idx, as = lacc ? 1 : np;
 #pragma unroll
-        for (int c = 0; c < 3; c++) a3[c] = acc[ai + c * as];
+        for (int c = 0; c < NC; c++) a3[c] = acc[ai + c * as];
     }
 }
 
@@ -1112,7 +1067,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
                                                       unsigned cap, TileGeom g, T sx, T sy, T sz, T L,
                                                       const T *__restrict__ phi, T c1, T c2, T c3,
                                                       T *__restrict__ acc, size_t np, int lacc) {
-    constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
+    constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>(), NC = gather_values(ORDER);
     extern __shared__ unsigned char smem[];
     T *ph = (T *)smem;
     int tx, ty, tz;
@@ -1130,8 +1085,8 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
     const unsigned e0 = start[t], e1 = e0 + list_len(own[t], e0, gstart[t], cap);
     unsigned e = e0 + threadIdx.x;
     Entry<T> en{};
-    T a3[3] = {0, 0, 0};
-    if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
+    T a3[NC] = {};
+    if (e < e1) gather_fetch<T, MODE, NC>(ent, e, acc, np, lacc, en, a3);
 
     if (region_ok) {
         const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1156,31 +1111,32 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
             lb[a] = wrapn(c0[a] - r0[a], N);
             staged &= lb[a] + Q <= S[a];
         }
-        T s1 = 0, s2 = 0, s3 = 0;
+        T f3[NC] = {};
         if (staged) {
             const int base = lb[0] + SX * lb[1] + SXY * lb[2];
             auto ld = [&](int x, int y, int z) { return ph[base + x + SX * y + SXY * z]; };
-            gather_sums_union<T, W, ORDER>(ld, w, c1, c2, c3, s1, s2, s3);
+            if constexpr (ORDER == 0) f3[0] = gather_sum<T, W>(ld, w);
+            else gather_sums_union<T, W, ORDER>(ld, w, c1, c2, c3, f3[0], f3[1], f3[2]);
         } else {
             auto ld = [&](int x, int y, int z) {
                 return phi[(size_t)wrapn(c0[0] + x, N) +
                            (size_t)N * ((size_t)wrapn(c0[1] + y, N) + (size_t)N * wrapn(c0[2] + z, N))];
             };
-            gather_sums<T, W, ORDER>(ld, w, c1, c2, c3, s1, s2, s3);
+            if constexpr (ORDER == 0) f3[0] = gather_sum<T, W>(ld, w);
+            else gather_sums<T, W, ORDER>(ld, w, c1, c2, c3, f3[0], f3[1], f3[2]);
         }
         const size_t p = (size_t)en.idx;
-        const T f3[3] = {s1, s2, s3};
         // acc of this particle: (3, Np) in particle order, or (entries, 3) in list order between the passes
-        const size_t ai = lacc ? 3 * (size_t)e : p, as = lacc ? 1 : np;
+        const size_t ai = lacc ? NC * (size_t)e : p, as = lacc ? 1 : np;
         if constexpr (MODE == GATHER_ACC) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) acc[ai + c * as] = a3[c] + f3[c];
+            for (int c = 0; c < NC; c++) acc[ai + c * as] = a3[c] + f3[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
+            for (int c = 0; c < NC; c++) acc[ai + c * as] = f3[c];
         }
         e += NT;
-        if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
+        if (e < e1) gather_fetch<T, MODE, NC>(ent, e, acc, np, lacc, en, a3);
     }
 }
 
@@ -1240,7 +1196,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
     const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start, const unsigned *__restrict__ gstart,
     const unsigned *__restrict__ own, unsigned cap, TileGeom g, T sx, T sy, T sz, T L, const T *__restrict__ phi, T c1, T c2, T c3, T *__restrict__ acc, size_t np, int lacc,
     MarchMap m) {
-    constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>();
+    constexpr int H = ORDER / 2, Q = W + 2 * H, NT = gather_threads<T, W>(), NC = gather_values(ORDER);
     extern __shared__ unsigned char smem[];
     T *ph = (T *)smem;
     const StageGeom q = gather_geom<T, W, true>(g, H);
@@ -1262,8 +1218,8 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
         const unsigned e0 = start[t], e1 = e0 + list_len(own[t], e0, gstart[t], cap);
         unsigned e = e0 + part * NT + threadIdx.x;
         Entry<T> en{};
-        T a3[3] = {0, 0, 0};
-        if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
+        T a3[NC] = {};
+        if (e < e1) gather_fetch<T, MODE, NC>(ent, e, acc, np, lacc, en, a3);
         // stage: the whole region for the first tile, else the TZ planes after the previous region,
         // into the ring slots (zg - zs0) mod R, split where the slots wrap
         {
@@ -1296,7 +1252,7 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
                 lb[a] = wrapn(c0[a] - r0[a], N);
                 staged &= lb[a] + Q <= S[a];
             }
-            T s1 = 0, s2 = 0, s3 = 0;
+            T f3[NC] = {};
             if (staged) {
                 // plane z of the stencil at ring slot sl0 + z, wrapping once, at plane zw: base A for the
                 // planes before it, B = A - R SXY after it, the rest an immediate offset
@@ -1304,26 +1260,27 @@ __global__ __launch_bounds__((gather_threads<T, W>()), (gather_min_waves<T, W>()
                 sl0 = sl0 >= R ? sl0 - R : sl0;
                 const int A = lb[0] + SX * lb[1] + sl0 * SXY, B = A - R * SXY, zw = R - sl0;
                 auto ld = [&](int x, int y, int z) { return ph[(z >= zw ? B : A) + x + SX * y + SXY * z]; };
-                gather_sums_union<T, W, ORDER>(ld, w, c1, c2, c3, s1, s2, s3);
+                if constexpr (ORDER == 0) f3[0] = gather_sum<T, W>(ld, w);
+            else gather_sums_union<T, W, ORDER>(ld, w, c1, c2, c3, f3[0], f3[1], f3[2]);
             } else {
                 auto ld = [&](int x, int y, int z) {
                     return phi[(size_t)wrapn(c0[0] + x, N) +
                                (size_t)N * ((size_t)wrapn(c0[1] + y, N) + (size_t)N * wrapn(c0[2] + z, N))];
                 };
-                gather_sums<T, W, ORDER>(ld, w, c1, c2, c3, s1, s2, s3);
+                if constexpr (ORDER == 0) f3[0] = gather_sum<T, W>(ld, w);
+            else gather_sums<T, W, ORDER>(ld, w, c1, c2, c3, f3[0], f3[1], f3[2]);
             }
             const size_t p = (size_t)en.idx;
-            const T f3[3] = {s1, s2, s3};
-            const size_t ai = lacc ? 3 * (size_t)e : p, as = lacc ? 1 : np;
+            const size_t ai = lacc ? NC * (size_t)e : p, as = lacc ? 1 : np;
             if constexpr (MODE == GATHER_ACC) {
 #pragma unroll
-                for (int c = 0; c < 3; c++) acc[ai + c * as] = a3[c] + f3[c];
+                for (int c = 0; c < NC; c++) acc[ai + c * as] = a3[c] + f3[c];
             } else {
 #pragma unroll
-                for (int c = 0; c < 3; c++) acc[ai + c * as] = f3[c];
+                for (int c = 0; c < NC; c++) acc[ai + c * as] = f3[c];
             }
             e += step;
-            if (e < e1) gather_fetch<T, MODE>(ent, e, acc, np, lacc, en, a3);
+            if (e < e1) gather_fetch<T, MODE, NC>(ent, e, acc, np, lacc, en, a3);
         }
         // every wave is done with this tile's first TZ planes before the next tile's staging overwrites them
         __syncthreads();
@@ -1502,6 +1459,16 @@ struct TileLaunch {
         else if (order == 4) gat_wo<W, 4>(a, sh, phi, c, mode, st);
         else gat_wo<W, 6>(a, sh, phi, c, mode, st);
     }
+    // ORDER 0 on the mesh f, into component comp of acc at the particles
+    static void gather_comp(const TileArgs &a, int W, const double *sh, const void *f, int mode, int comp,
+                            hipStream_t st) {
+        const double c[3] = {0, 0, 0};
+        TileArgs ac = a;
+        ac.acc = (T *)a.acc + (size_t)comp * a.n * a.n * a.n;
+        if (W == 2) gat_wo<2, 0>(ac, sh, f, c, mode, st);
+        else if (W == 3) gat_wo<3, 0>(ac, sh, f, c, mode, st);
+        else gat_wo<4, 0>(ac, sh, f, c, mode, st);
+    }
     static void gather(const TileArgs &a, int W, int order, const double *sh, const void *phi, const double *c,
                        int mode, hipStream_t st) {
         if (W == 2) gat_w<2>(a, order, sh, phi, c, mode, st);
@@ -1526,6 +1493,7 @@ template <typename T> void tile_ops(TileOps &ops) {
     ops.deposit = TileLaunch<T>::deposit;
     ops.deposit3 = TileLaunch<T>::deposit3;
     ops.gather = TileLaunch<T>::gather;
+    ops.gather_comp = TileLaunch<T>::gather_comp;
     ops.entry_bytes = sizeof(Entry<T>);
 }
 

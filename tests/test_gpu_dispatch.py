@@ -136,3 +136,20 @@ def test_sort_over_the_scan_rule(res, n, prec):
         m = S.deposit(psi)
     ref = O.pm_scatter(O.lagrangian_positions(psi, L), res, L, 2)
     assert G.rel(m, ref) < (2e-5 if prec == 32 else 1e-12)
+
+
+@pytest.mark.parametrize("W", [2, 3, 4])
+@pytest.mark.parametrize("res, n, aa, prec", [(16, 9, 0, 32), (64, 30, 1, 32), (96, 33, 2, 32), (64, 31, 1, 64),
+                                              (128, 32, 3, 32)])
+def test_spectral_force_over_tiles(W, res, n, aa, prec):
+    """The tiled interpolation of the spectral gradient's force meshes: regions as large as the mesh (16^3),
+    the compile-time regions of FP32, reaches they do not cover (antialias 3) and FP64, against the oracle."""
+    L = 2.0 * res
+    dt = np.float32 if prec == 32 else np.float64
+    psi = _psi(n, 3.0, res + W, dt)
+    acc = D.pm_acceleration(psi, D.PMConfig(res_pm=res, n_part=n, boxsize=L, worder=W, grad_order=0, antialias=aa),
+                            precision=prec)
+    # the oracle's force in the same precision's positions: FP32 rounds the weights' coordinates (res 2^-24 of a
+    # cell each), the meshes and the transforms
+    ref = O.pm_acceleration(psi, O.pm_config(res, n, L, worder=W, grad_order=0, antialias=aa), "solver")
+    assert G.rel(acc, ref) < (2e-5 if prec == 32 else 1e-12)
