@@ -561,6 +561,27 @@ dj_status resample_deposit(dj_ctx *c, const void *psi, const double *sh, void *d
                            void *pts = nullptr);
 void nn_forward_dev(dj_ctx *c, const void *dens, double a);
 
+// component ax of the spectral gradient's force mesh from zm_ik's two spectra (B and C): i k_x is applied by the
+// inverse x pass, i k_y by the inverse y pass
+void ik_force_mesh(dj_ctx *c, int ax, void *out) {
+    const void *gf, *gh;
+    if (c->tsize == 8) {
+        const KMult<double> &K = *(const KMult<double> *)c->kmult;
+        gf = K.gf; gh = K.gh;
+    } else {
+        const KMult<float> &K = *(const KMult<float> *)c->kmult;
+        gf = K.gf; gh = K.gh;
+    }
+    {
+        Prof p(c, K_YI);
+        if (ax == 1) c->fft.yi_mul(c->B, c->A, c->tw, gf, c->st);
+        else c->fft.yi(ax == 2 ? c->C : c->B, c->A, c->tw, c->st);
+    }
+    Prof p(c, K_XI);
+    if (ax == 0) c->fft.xi_mul(c->A, out, c->tw, gh, 1.0, c->st);
+    else c->fft.xi(c->A, out, c->tw, c->st);
+}
+
 dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool defer = false) {
     const dj_pm_config &cfg = c->cfg;
     const bool fixed = cfg.deposit == DJ_DEPOSIT_FIXED64;
@@ -598,7 +619,6 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
             const int nrn = cfg.n_resample * c->n;
             {
                 Prof p(c, K_RESAMPLE);
-                c->rs.shifted(psi, c->q1, c->n, c->shifts[s], cfg.n_resample, c->rl_pts, c->st);
                 dj_status rr = c->tsize == 8
                                    ? resample_deposit<double>(c, psi, c->shifts[s], dens, fixed, fscale_dep(cfg), c->rl_pts)
                                    : resample_deposit<float>(c, psi, c->shifts[s], dens, fixed, fscale_dep(cfg), c->rl_pts);
@@ -646,13 +666,12 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
                 c->tiles.kick_listed(c->own_at, c->acc_list, c->psi, c->mom, (size_t)c->np, kick, c->st);
             }
         } else {
-            { Prof p(c, K_ZM); c->fft.zm(ZM_NONE, true, false, c->B, c->B, c->tw, c->kmult, c->st); }
+            { Prof p(c, K_ZM); c->fft.zm_ik(c->B, c->B, c->C, c->tw, c->kmult, c->st); }
             for (int ax = 0; ax < 3; ax++) {
-                { Prof p(c, K_ZM); c->fft.zm(ZM_GRADX + ax, false, true, c->B, c->C, c->tw, c->kmult, c->st); }
-                { Prof p(c, K_YI); c->fft.yi(c->C, c->A, c->tw, c->st); }
-                { Prof p(c, K_XI); c->fft.xi(c->A, c->mesh, c->tw, c->st); }
+                ik_force_mesh(c, ax, c->mesh);
                 Prof p(c, K_GATHER);
-                c->tiles.gather_comp(ta, cfg.worder, c->shifts[s], c->mesh, s == 0 ? GATHER_ASSIGN : GATHER_ACC, ax, c->st);
+                c->tiles.gather_comp(ta, cfg.worder, c->shifts[s], c->mesh, s == 0 ? GATHER_ASSIGN : GATHER_ACC, ax,
+                                     c->st);
             }
         }
         dj_status r = check_launch(c, "force pass");
@@ -752,50 +771,94 @@ dj_status setup_resampling(dj_ctx *c) {
 
 // The extra point sets of one interlacing pass (shift sh) deposited into dens (pm.jl:471-483 with
 // _resample_prepare! / _resample_offset! for Fourier, _spawn for linear).
-// pts: instead of depositing, write each offset's positions into the point-set lattice pts (3, (nr n)^3)
+// pts: instead of depositing, write the particles' and every offset's positions into the point-set lattice
+// pts (3, (nr n)^3).  The phase of an offset (a, b, c) / nr is a product of one factor per axis, so the
+// inverse transforms share their passes: one z pass per a, one y pass per (a, b), one x pass per offset, each
+// multiplying by its axis's factor as it loads (nr = 2: 13 passes a component instead of 21 and 7 of phases).
 template <typename T>
 dj_status resample_deposit(dj_ctx *c, const void *psi, const double *sh, void *dens, bool fixed, double fscale,
                            void *pts) {
-    const int nr = pts ? c->cfg.n_resample : 1, o0[3] = {0, 0, 0};
-    const int n = c->n, H = n / 2 + 1;
+    const int nr = c->cfg.n_resample, o0[3] = {0, 0, 0};
+    const int n = c->n, H = n / 2 + 1, per = 2 * n + H;
     const double L = c->cfg.boxsize;
     const size_t n3 = (size_t)c->np, hc = (size_t)n * n * H;
     T *xr = (T *)c->rs_xr;
+    // the lattice shift d_c L / n of an offset's component c, rounded to T as the reference does
+    auto lattice = [&](int o) { return (double)(T)((double)o / nr * L / n); };
     if (c->cfg.resampling == 1) {
         T *w = (T *)c->rs_psi;
+        if (pts) c->rs.shifted(psi, c->q1, n, sh, nr, pts, c->st);
         for (int comp = 0; comp < 3; comp++)
             c->rs.wrap(psi, c->q1, n, comp, sh[comp], L, false, w + comp * n3, c->st);
         for (int o = 0; o < c->n_offsets; o++) {
-            const double *d = c->offsets[o];
             for (int comp = 0; comp < 3; comp++) {
-                c->rs.trilinear(w + comp * n3, n, d, w + 3 * n3, c->st);
-                c->rs.place(w + 3 * n3, c->q1, n, comp, (double)(T)(d[comp] * L / n), L, false, pts ? pts : xr, nr,
-                            pts ? c->ioffsets[o] : o0, c->st);
+                c->rs.trilinear(w + comp * n3, n, c->offsets[o], w + 3 * n3, c->st);
+                c->rs.place(w + 3 * n3, c->q1, n, comp, lattice(c->ioffsets[o][comp]), L, pts ? pts : xr,
+                            pts ? nr : 1, pts ? c->ioffsets[o] : o0, c->st);
             }
             if (!pts) c->rs.scatter(xr, n, c->cfg.worder, dens, c->res, L, fixed, fscale, c->st);
         }
         return check_launch(c, "linear sheet resampling");
     }
     cx<T> *hat = (cx<T> *)c->rs_hat;
-    for (int comp = 0; comp < 3; comp++) {
+    const double scale = (double)((T)1 / ((T)n * (T)n * (T)n));
+    auto forward = [&](int comp, cx<T> *out) {
         c->rs.wrap(psi, c->q1, n, comp, sh[comp], L, true, c->rs_psi, c->st);
         c->fftn.xf(c->rs_psi, false, c->rs_A, c->rs_tw, 1.0, c->st);
         c->fftn.yf(c->rs_A, c->rs_B, c->rs_tw, c->st);
-        c->fftn.zm(ZM_NONE, true, false, c->rs_B, hat + comp * hc, c->rs_tw, c->kmult, c->st);
+        c->fftn.zm(ZM_NONE, true, false, c->rs_B, out, c->rs_tw, c->kmult, c->st);
+    };
+    if (pts) {
+        // the factors of a, b and c, from the offsets (a, 0, 0), (0, b, 0) and (0, 0, c)
+        const cx<T> *ph = (const cx<T> *)c->rs_phase;
+        auto px = [&](int a) { return ph + (size_t)(a * nr * nr - 1) * per; };
+        auto py = [&](int b) { return ph + (size_t)(b * nr - 1) * per + n; };
+        auto pz = [&](int e) { return ph + (size_t)(e - 1) * per + 2 * n; };
+        cx<T> *Z[2] = {hat + hc, hat + 2 * hc};
+        void *Y[2] = {c->rs_A, c->rs_B};
+        for (int comp = 0; comp < 3; comp++) {
+            forward(comp, hat);
+            for (int a = 0; a < nr; a += 2) {
+                const int na = std::min(2, nr - a);
+                for (int q = 0; q < na; q++) {
+                    if (a + q) c->fftn.zi_mul(hat, Z[q], c->rs_tw, px(a + q), c->st);
+                    else c->fftn.zm(ZM_NONE, false, true, hat, Z[q], c->rs_tw, c->kmult, c->st);
+                }
+                for (int b = 0; b < nr; b++) {
+                    for (int q = 0; q < na; q++) {
+                        if (b) c->fftn.yi_mul(Z[q], Y[q], c->rs_tw, py(b), c->st);
+                        else c->fftn.yi(Z[q], Y[q], c->rs_tw, c->st);
+                    }
+                    for (int e = 0; e < nr; e++) {
+                        const int o[3] = {a, b, e};
+                        const bool own = a == 0 && b == 0 && e == 0;
+                        double shift[2];
+                        for (int q = 0; q < na; q++) {
+                            shift[q] = lattice(o[comp] + (comp == 0 ? q : 0));
+                            if (own && q == 0) continue;
+                            if (e) c->fftn.xi_mul(Y[q], xr + q * n3, c->rs_tw, pz(e), scale, c->st);
+                            else c->fftn.xi_scaled(Y[q], xr + q * n3, c->rs_tw, scale, c->st);
+                        }
+                        c->rs.place_t(own ? nullptr : xr, xr + n3, na, psi, c->q1, n, comp, sh[comp], shift, L, pts,
+                                      nr, o, c->st);
+                    }
+                }
+            }
+        }
+        return check_launch(c, "Fourier sheet resampling");
     }
-    const double scale = (double)((T)1 / ((T)n * (T)n * (T)n));
+    for (int comp = 0; comp < 3; comp++) forward(comp, hat + comp * hc);
     for (int o = 0; o < c->n_offsets; o++) {
-        const double *d = c->offsets[o];
-        const cx<T> *px = (const cx<T> *)c->rs_phase + (size_t)o * (2 * n + H), *py = px + n, *pz = px + 2 * n;
+        const cx<T> *px = (const cx<T> *)c->rs_phase + (size_t)o * per, *py = px + n, *pz = px + 2 * n;
         for (int comp = 0; comp < 3; comp++) {
             c->rs.phase(hat + comp * hc, c->rs_B, n, px, py, pz, scale, c->st);
             c->fftn.zm(ZM_NONE, false, true, c->rs_B, c->rs_B, c->rs_tw, c->kmult, c->st);
             c->fftn.yi(c->rs_B, c->rs_A, c->rs_tw, c->st);
             c->fftn.xi(c->rs_A, c->rs_psi, c->rs_tw, c->st);
-            c->rs.place(c->rs_psi, c->q1, n, comp, (double)(T)(d[comp] * L / n), L, true, pts ? pts : xr, nr,
-                        pts ? c->ioffsets[o] : o0, c->st);
+            const double shift = lattice(c->ioffsets[o][comp]);
+            c->rs.place_t(c->rs_psi, nullptr, 1, psi, c->q1, n, comp, sh[comp], &shift, L, xr, 1, o0, c->st);
         }
-        if (!pts) c->rs.scatter(xr, n, c->cfg.worder, dens, c->res, L, fixed, fscale, c->st);
+        c->rs.scatter(xr, n, c->cfg.worder, dens, c->res, L, fixed, fscale, c->st);
     }
     return check_launch(c, "Fourier sheet resampling");
 }
@@ -1263,7 +1326,6 @@ dj_status vjp_force(dj_ctx *c, const void *psi, void *abar, void *psibar, const 
         if (cfg.n_resample > 1) {
             // the forward's density: the particles and every offset's points through the point lattice
             const int nrn = cfg.n_resample * c->n;
-            c->rs.shifted(psi, c->q1, c->n, c->shifts[s], cfg.n_resample, c->rl_pts, c->st);
             r = c->tsize == 8 ? resample_deposit<double>(c, psi, c->shifts[s], dens, fixed, fscale_dep(cfg), c->rl_pts)
                               : resample_deposit<float>(c, psi, c->shifts[s], dens, fixed, fscale_dep(cfg), c->rl_pts);
             if (r) return r;
@@ -1283,12 +1345,8 @@ dj_status vjp_force(dj_ctx *c, const void *psi, void *abar, void *psibar, const 
             const size_t M = c->M;
             char *F = (char *)c->vb_fik, *Fb = (char *)c->vb_fbar;
             const size_t mb = M * c->tsize;
-            c->fft.zm(ZM_NONE, true, false, c->B, c->B, c->tw, c->kmult, c->st);
-            for (int ax = 0; ax < 3; ax++) {
-                c->fft.zm(ZM_GRADX + ax, false, true, c->B, c->C, c->tw, c->kmult, c->st);
-                c->fft.yi(c->C, c->A, c->tw, c->st);
-                c->fft.xi(c->A, F + ax * mb, c->tw, c->st);
-            }
+            c->fft.zm_ik(c->B, c->B, c->C, c->tw, c->kmult, c->st);
+            for (int ax = 0; ax < 3; ax++) ik_force_mesh(c, ax, F + ax * mb);
             if (!c->tiles.deposit3(ta, cfg.worder, c->shifts[s], abar, 1.0 / ns, c->vb_fbar, c->loss_work, c->st)) {
                 c->part.zero(c->vb_fbar, 3 * c->M * c->tsize, c->st);
                 c->adj.scatter3(psi, c->q1, c->n, N, cfg.boxsize, c->shifts[s], abar, 1.0 / ns, cfg.worder, c->vb_fbar,

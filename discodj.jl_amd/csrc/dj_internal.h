@@ -29,6 +29,13 @@ struct FftOps {
     void (*xi)(const void *A, void *mesh, const void *tw, hipStream_t st);
     // the same with the output multiplied by s as it is stored
     void (*xi_scaled)(const void *A, void *mesh, const void *tw, double s, hipStream_t st);
+    // inverse passes of the spectrum times a table along the pass's axis (N entries; N/2 + 1 for x, whose output is
+    // also multiplied by s)
+    void (*xi_mul)(const void *A, void *mesh, const void *tw, const void *tab, double s, hipStream_t st);
+    void (*yi_mul)(const void *B, void *A, const void *tw, const void *tab, hipStream_t st);
+    void (*zi_mul)(const void *in, void *out, const void *tw, const void *tab, hipStream_t st);
+    // the spectral gradient's z pass: out = inverse z of -K_phi (forward z of in), outz the same of i k_z times it
+    void (*zm_ik)(const void *in, void *out, void *outz, const void *tw, const void *kmult, hipStream_t st);
     void (*yf)(const void *A, void *B, const void *tw, hipStream_t st);
     void (*yi)(const void *B, void *A, const void *tw, hipStream_t st);
     void (*zm)(int mode, bool fwd, bool inv, const void *in, void *out, const void *tw, const void *K,
@@ -143,8 +150,12 @@ struct ResampleOps {
     void (*trilinear)(const void *f, int n, const double *d, void *out, hipStream_t st);
     // Xr_c = mod(q_c + npsi_c + shift + L, L), at point (nr i + o[0], nr j + o[1], nr k + o[2]) of the
     // (nr n)^3 point-set lattice xr (3 components); nr = 1, o = 0: the particle layout
-    void (*place)(const void *npsi, const void *q1, int n, int c, double shift, double L, bool transposed, void *xr,
-                  int nr, const int *o, hipStream_t st);
+    void (*place)(const void *npsi, const void *q1, int n, int c, double shift, double L, void *xr, int nr,
+                  const int *o, hipStream_t st);
+    // the same from transposed fields of na = 1 or 2 offsets that follow each other along x (x0 null: the
+    // particles, shifted by s, are the first set)
+    void (*place_t)(const void *x0, const void *x1, int na, const void *psi, const void *q1, int n, int c, double s,
+                    const double *shift, double L, void *xr, int nr, const int *o, hipStream_t st);
     // the particles' shifted positions (psi + q) + sh at points (nr i, nr j, nr k) of the point-set lattice
     void (*shifted)(const void *psi, const void *q1, int n, const double *sh, int nr, void *out, hipStream_t st);
     // unit-mass deposit of positions (3, n^3) with device atomics (float, or int64 fixed point)

@@ -122,10 +122,11 @@ struct PartnerSrc {
     __device__ cx<double> operator()(size_t g) const { return cx<double>{at(g), at(g + 1)}; }
 };
 
-// SC: the output multiplied by s as it is stored
-template <typename T, int N, bool SC = false>
+// SC: the output multiplied by s as it is stored; MUL: the spectrum multiplied by tab[kx] as it is loaded
+template <typename T, int N, bool SC = false, bool MUL = false>
 __global__ __launch_bounds__((FftShape<T, N>::NTXI)) void k_xi(const cx<T> *__restrict__ A, T *__restrict__ mesh,
-                                            const cx<T> *__restrict__ tw, T s = (T)1) {
+                                            const cx<T> *__restrict__ tw, T s = (T)1,
+                                            const cx<T> *__restrict__ tab = nullptr) {
     using S = FftShape<T, N>;
     using P = typename S::PXI;
     __shared__ cx<T> lds[P::EX::LDS_ELEMS];
@@ -140,9 +141,9 @@ __global__ __launch_bounds__((FftShape<T, N>::NTXI)) void k_xi(const cx<T> *__re
         P::xi_fetch(A, yb, z, threadIdx.x, va, vb);
         t = stage_twiddles<T, N, true>(tw, twl, threadIdx.x, S::NTXI);
         __syncthreads();
-        P::xi_pre(lds, t, threadIdx.x, va, vb);
+        P::template xi_pre<MUL>(lds, t, threadIdx.x, va, vb, tab);
     } else {
-        P::xi_load_pre(A, lds, tw, yb, z, threadIdx.x);
+        P::template xi_load_pre<MUL>(A, lds, tw, yb, z, threadIdx.x, tab);
     }
     __syncthreads();
     if constexpr (P::EX::wave_ok()) {
@@ -176,16 +177,18 @@ __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_yf(const cx<T> *__res
     P::y_store_b(lds, Bm, zb, kx, threadIdx.x);
 }
 
-template <typename T, int N>
+// MUL: the spectrum multiplied by tab[ky] as it is loaded
+template <typename T, int N, bool MUL = false>
 __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_yi(const cx<T> *__restrict__ Bm, cx<T> *__restrict__ A,
-                                                             const cx<T> *__restrict__ tw) {
+                                                             const cx<T> *__restrict__ tw,
+                                                             const cx<T> *__restrict__ tab = nullptr) {
     using S = FftShape<T, N>;
     using P = typename S::PY;
     __shared__ cx<T> lds[P::EF::LDS_ELEMS];
     __shared__ cx<T> twl[S::TWL ? N : 1];
     const int lb = xcd_block(blockIdx.x, gridDim.x), zb = lb % (N / S::B), kx = lb / (N / S::B);
     const cx<T> *t = stage_twiddles<T, N, S::TWL>(tw, twl, threadIdx.x, S::NTY);
-    P::y_load_b(Bm, lds, zb, kx, threadIdx.x);
+    P::template y_load_b<MUL>(Bm, lds, zb, kx, threadIdx.x, tab);
     __syncthreads();
     if constexpr (P::EF::wave_ok()) {
         P::EF::template run_wave<+1, 1>(lds, t, threadIdx.x);
@@ -229,6 +232,66 @@ __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zm(const cx<T> *in, c
     }
 }
 
+// The z pass of the spectral gradient: forward, times -K_phi, then two inverse transforms, of that product into
+// out (the x and y components are its transforms with i k_x and i k_y, which the inverse x and y passes apply)
+// and of i k_z times it into outz.  One read and two writes of the spectrum; a forward pass and three inverse
+// ones made four and four (512^3, FP32: 1.06 ms against 0.46).  in may equal out.
+template <typename T, int N>
+__global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zm_ik(const cx<T> *in, cx<T> *out, cx<T> *__restrict__ outz,
+                                                                const cx<T> *__restrict__ tw, KMult<T> K) {
+    using S = FftShape<T, N>;
+    using P = typename S::PY;
+    constexpr int H = N / 2 + 1, NT = S::NTY;
+    constexpr bool WV = P::EF::wave_ok();
+    // a thread's elements: its wave's lines in steps of 64, or the tile's in steps of the workgroup
+    constexpr int E = WV ? P::EF::LW * N : S::B * N, STEP = WV ? 64 : NT, CNT = (E + STEP - 1) / STEP;
+    __shared__ cx<T> lds[P::EF::LDS_ELEMS];
+    __shared__ cx<T> twl[S::TWL ? N : 1];
+    const int b = blockIdx.x, wave = threadIdx.x >> 6;
+    const int e0 = WV ? wave * E : 0, t0 = WV ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    const cx<T> *t = stage_twiddles<T, N, S::TWL>(tw, twl, threadIdx.x, NT);
+    auto sync = [&]() {
+        if constexpr (WV) P::EF::wave_sync();
+        else __syncthreads();
+    };
+    if constexpr (WV) P::z_load_w(in, lds, b, threadIdx.x);
+    else P::z_load(in, lds, b, threadIdx.x);
+    __syncthreads();
+    if constexpr (WV) P::EF::template run_wave<-1, 1>(lds, t, threadIdx.x);
+    else P::EF::template run<-1, 1>(lds, t, threadIdx.x);
+    cx<T> gz[CNT];
+#pragma unroll
+    for (int c = 0; c < CNT; c++) {
+        const int i = e0 + t0 + STEP * c, l = i / N, kz = i - l * N;
+        if (E % STEP != 0 && t0 + STEP * c >= E) continue;
+        const int L = b * S::B + l, ky = L / H, kx = L - ky * H;
+        const cx<T> v = scale(lds[P::EF::idx(l, kz)], -K.kphi(kx, ky, kz));
+        lds[P::EF::idx(l, kz)] = v;
+        const T k = K.gf[kz].y;  // i k_z, its Nyquist zeroed
+        gz[c] = {-(k * v.y), k * v.x};
+    }
+    sync();
+    auto inverse_to = [&](cx<T> *dst) {
+        if constexpr (WV) {
+            P::EF::template run_wave<+1, 1>(lds, t, threadIdx.x);
+            P::z_store_w(lds, dst, b, threadIdx.x);
+        } else {
+            P::EF::template run<+1, 1>(lds, t, threadIdx.x);
+            P::z_store(lds, dst, b, threadIdx.x);
+        }
+    };
+    inverse_to(out);
+    sync();
+#pragma unroll
+    for (int c = 0; c < CNT; c++) {
+        const int i = e0 + t0 + STEP * c, l = i / N;
+        if (E % STEP != 0 && t0 + STEP * c >= E) continue;
+        lds[P::EF::idx(l, i - l * N)] = gz[c];
+    }
+    sync();
+    inverse_to(outz);
+}
+
 // The z pass (forward or inverse) of lines read from src(e) and written to dst(e, v), e the B-layout index:
 // the FP64 2LPT derivative spectra formed as the pass loads them, or their cotangents cropped and added
 // into the n-grid spectrum as it stores them
@@ -255,6 +318,11 @@ __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zm_io(SRC src, DST ds
 template <typename T> struct StoreTo {
     cx<T> *out;
     __device__ void operator()(size_t e, cx<T> v) const { out[e] = v; }
+};
+// the z lines of in multiplied by tab[kz] as they are loaded
+template <typename T, int N> struct LoadMul {
+    const cx<T> *in, *tab;
+    __device__ cx<T> operator()(size_t e) const { return cmul(in[e], tab[(unsigned)(e % N)]); }
 };
 template <typename T> struct LoadFrom {
     const cx<T> *in;
@@ -418,6 +486,23 @@ struct FftN {
                     i, MultAccDst<IC_PSI2_ADJ, N>{(cx<T> *)acc, c, L, s}, t);
         }
     }
+    static void zm_ik(const void *in, void *out, void *outz, const void *tw, const void *Kp, hipStream_t st) {
+        k_zm_ik<T, N><<<P::ZBLOCKS(), S::NTY, 0, st>>>((const cx<T> *)in, (cx<T> *)out, (cx<T> *)outz, (const cx<T> *)tw,
+                                                       *(const KMult<T> *)Kp);
+    }
+    static void zi_mul(const void *in, void *out, const void *tw, const void *tab, hipStream_t st) {
+        k_zm_io<T, N, false, LoadMul<T, N>, StoreTo<T>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
+            LoadMul<T, N>{(const cx<T> *)in, (const cx<T> *)tab}, StoreTo<T>{(cx<T> *)out}, (const cx<T> *)tw);
+    }
+    static void yi_mul(const void *Bm, void *A, const void *tw, const void *tab, hipStream_t st) {
+        k_yi<T, N, true><<<P::YBLOCKS(), S::NTY, 0, st>>>((const cx<T> *)Bm, (cx<T> *)A, (const cx<T> *)tw,
+                                                          (const cx<T> *)tab);
+    }
+    static void xi_mul(const void *A, void *mesh, const void *tw, const void *tab, double s, hipStream_t st) {
+        using PX = typename S::PXI;
+        k_xi<T, N, true, true><<<PX::XBLOCKS(), S::NTXI, 0, st>>>((const cx<T> *)A, (T *)mesh, (const cx<T> *)tw, (T)s,
+                                                                  (const cx<T> *)tab);
+    }
     static void xi(const void *A, void *mesh, const void *tw, hipStream_t st) {
         using PX = typename S::PXI;
         k_xi<T, N><<<PX::XBLOCKS(), S::NTXI, 0, st>>>((const cx<T> *)A, (T *)mesh, (const cx<T> *)tw);
@@ -466,6 +551,10 @@ bool fft_dispatch(int N, FftOps &ops) {
         ops.xf = FftN<T, n>::xf;        \
         ops.xi = FftN<T, n>::xi;        \
         ops.xi_scaled = FftN<T, n>::xi_scaled; \
+        ops.xi_mul = FftN<T, n>::xi_mul; \
+        ops.yi_mul = FftN<T, n>::yi_mul; \
+        ops.zi_mul = FftN<T, n>::zi_mul; \
+        ops.zm_ik = FftN<T, n>::zm_ik; \
         ops.xf_partner = FftN<T, n>::xf_partner; \
         ops.zm_deriv_pad = FftN<T, n>::zm_deriv_pad; \
         ops.zm_deriv_adj = FftN<T, n>::zm_deriv_adj; \

@@ -198,8 +198,10 @@ struct Passes {
             }
         }
     }
+    // MUL: X[k] multiplied by tab[k] first
+    template <bool MUL = false>
     DJ_HD static void xi_pre(cx<T> *lds, const cx<T> *twN, int tid, const cx<T> (&va)[XI_CNT],
-                             const cx<T> (&vb)[XI_CNT]) {
+                             const cx<T> (&vb)[XI_CNT], const cx<T> *tab = nullptr) {
         constexpr int HP = NC / 2 + 1, TOTAL = B * HP;
 #pragma unroll
         for (int c = 0; c < XI_CNT; c++) {
@@ -207,6 +209,10 @@ struct Passes {
             if (!(TOTAL % NT == 0 || i < TOTAL)) continue;
             const int k = i / B, l = i - k * B;
             cx<T> a = va[c], b = vb[c];
+            if constexpr (MUL) {
+                a = cmul(a, tab[k]);
+                b = cmul(b, tab[NC - k]);
+            }
             if (k == 0) { a.y = 0; b.y = 0; }
             const cx<T> e = a + conj(b);
             const cx<T> o = cmulc(a - conj(b), twN[k]);
@@ -219,10 +225,12 @@ struct Passes {
         }
     }
     // all reads of a thread are issued before its first LDS write
-    DJ_HD static void xi_load_pre(const cx<T> *A, cx<T> *lds, const cx<T> *twN, int yb, int z, int tid) {
+    template <bool MUL = false>
+    DJ_HD static void xi_load_pre(const cx<T> *A, cx<T> *lds, const cx<T> *twN, int yb, int z, int tid,
+                                  const cx<T> *tab = nullptr) {
         cx<T> va[XI_CNT], vb[XI_CNT];
         xi_fetch(A, yb, z, tid, va, vb);
-        xi_pre(lds, twN, tid, va, vb);
+        xi_pre<MUL>(lds, twN, tid, va, vb, tab);
     }
     // SC: each value multiplied by s as it is stored (a normalisation that would otherwise be a pass of its own)
     template <bool SC = false>
@@ -256,10 +264,15 @@ struct Passes {
             tid, [&](int i) { const int ky = i / B, l = i - ky * B; return lds[EF::idx(l, ky)]; },
             [&](int i, cx<T> v) { const int ky = i / B, l = i - ky * B; Bm[b_at(zb * B + l, kx, ky)] = v; });
     }
-    DJ_HD static void y_load_b(const cx<T> *Bm, cx<T> *lds, int zb, int kx, int tid) {
+    // MUL: every value multiplied by tab[ky] as it is loaded
+    template <bool MUL = false>
+    DJ_HD static void y_load_b(const cx<T> *Bm, cx<T> *lds, int zb, int kx, int tid, const cx<T> *tab = nullptr) {
         copy_batched<cx<T>, B * N, NT>(
             tid, [&](int i) { const int ky = i / B, l = i - ky * B; return Bm[b_at(zb * B + l, kx, ky)]; },
-            [&](int i, cx<T> v) { const int ky = i / B, l = i - ky * B; lds[EF::idx(l, ky)] = v; });
+            [&](int i, cx<T> v) {
+                const int ky = i / B, l = i - ky * B;
+                lds[EF::idx(l, ky)] = MUL ? cmul(v, tab[ky]) : v;
+            });
     }
     DJ_HD static void y_store_a(const cx<T> *lds, cx<T> *A, int zb, int kx, int tid) {
         copy_batched<cx<T>, B * N, NT>(

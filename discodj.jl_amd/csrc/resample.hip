@@ -16,27 +16,43 @@
 
 #include "dj_complex.h"
 #include "dj_internal.h"
+#include "stencil.h"
 
 namespace dj {
 
-template <typename T> __device__ __forceinline__ T rs_jmod(T x, T L) {
-    T r = fmod(x, L);
-    if (r == (T)0) return copysign(r, L);
-    if ((r > (T)0) != (L > (T)0)) return r + L;
-    return r;
+// psi_c of particle (i, j, k) at X_s = (psi + q) + s_c, into the natural or the transposed layout (the latter
+// through a 32 x 32 tile in LDS: written straight, every lane's store is a line of its own, 182 us for 256^3
+// in FP32)
+template <typename T>
+__device__ __forceinline__ T rs_wrapped(const T *psi, const T *q1, size_t p, int ic, T sc, T L) {
+    const T qc = q1[ic], xs = (psi[p] + qc) + sc;
+    return tjmod(xs - qc + L / (T)2, L) - L / (T)2;
 }
-
-// psi_c of particle (i, j, k) at X_s = (psi + q) + s_c, into the natural or the transposed layout
-template <typename T, bool TRANSPOSED>
+template <typename T>
 __global__ __launch_bounds__(256) void k_rs_wrap(const T *__restrict__ psi, const T *__restrict__ q1, int n, int c, T sc,
                                                  T L, T *__restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
     if (i >= n) return;
     const size_t N = (size_t)n, p = (size_t)i + N * ((size_t)j + N * k);
-    const T qc = q1[c == 0 ? i : c == 1 ? j : k];
-    const T xs = (psi[p + (size_t)c * N * N * N] + qc) + sc;
-    const T v = rs_jmod(xs - qc + L / (T)2, L) - L / (T)2;
-    out[TRANSPOSED ? (size_t)k + N * ((size_t)j + N * i) : p] = v;
+    out[p] = rs_wrapped(psi + (size_t)c * N * N * N, q1, p, c == 0 ? i : c == 1 ? j : k, sc, L);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_rs_wrap_t(const T *__restrict__ psi, const T *__restrict__ q1, int n, int c, T sc,
+                                                   T L, T *__restrict__ out) {
+    __shared__ T sh[32][33];
+    const int i0 = blockIdx.x * 32, j = blockIdx.y, k0 = blockIdx.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const size_t N = (size_t)n;
+    for (int r = ty; r < 32; r += 8) {
+        const int i = i0 + tx, k = k0 + r;
+        if (i < n && k < n)
+            sh[r][tx] = rs_wrapped(psi + (size_t)c * N * N * N, q1, (size_t)i + N * ((size_t)j + N * k),
+                                   c == 0 ? i : c == 1 ? j : k, sc, L);
+    }
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8) {
+        const int i = i0 + r, k = k0 + tx;
+        if (i < n && k < n) out[(size_t)k + N * ((size_t)j + N * i)] = sh[tx][r];
+    }
 }
 
 // the phase of offset d on the transposed field's half spectrum, library layout B[w + n (h + H v)]:
@@ -73,19 +89,61 @@ __global__ __launch_bounds__(256) void k_rs_trilinear(const T *__restrict__ f, i
         F(i1, j1, k1) * dx * dy * dz;
 }
 
-// Xr_c = mod(q_c + npsi_c + shift + L, L); npsi in the natural or the transposed layout.  Written at
-// point (nr i + o0, nr j + o1, nr k + o2) of the (nr n)^3 lattice of all point sets of a pass (offset
-// (o0, o1, o2) / nr cells: the sets interleave into a finer lattice; nr = 1, o = 0 is the plain layout)
-template <typename T, bool TRANSPOSED>
+// Xr_c = mod(q_c + npsi_c + shift + L, L).  Written at point (nr i + o0, nr j + o1, nr k + o2) of the (nr n)^3
+// lattice of all point sets of a pass (offset (o0, o1, o2) / nr cells: the sets interleave into a finer
+// lattice; nr = 1, o = 0 is the plain layout)
+template <typename T>
 __global__ __launch_bounds__(256) void k_rs_place(const T *__restrict__ npsi, const T *__restrict__ q1, int n, int c,
                                                   T shift, T L, T *__restrict__ xr, int nr, int o0, int o1, int o2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
     if (i >= n) return;
     const size_t N = (size_t)n, p = (size_t)i + N * ((size_t)j + N * k), NR = (size_t)nr * n;
     const T qc = q1[c == 0 ? i : c == 1 ? j : k];
-    const T np_ = npsi[TRANSPOSED ? (size_t)k + N * ((size_t)j + N * i) : p];
     const size_t pr = ((size_t)nr * i + o0) + NR * (((size_t)nr * j + o1) + NR * ((size_t)nr * k + o2));
-    xr[pr + (size_t)c * NR * NR * NR] = rs_jmod(((qc + np_) + shift) + L, L);
+    xr[pr + (size_t)c * NR * NR * NR] = tjmod(((qc + npsi[p]) + shift) + L, L);
+}
+
+// The same from NA fields in the transposed layout, of the offsets (o0, o1, o2) and, NA = 2, (o0 + 1, o1, o2):
+// transposed through LDS, and two neighbours along x written together, so that lattice rows of nr = 2 are
+// written whole.  x0 null: the first set is the particles themselves, at (psi + q) + s (a store per lane at the
+// lattice's stride, of a value read along the other axis, took 95 us a component and offset at 256^3, FP32)
+template <typename T, int NA>
+__global__ __launch_bounds__(256) void k_rs_place_t(const T *__restrict__ x0, const T *__restrict__ x1,
+                                                    const T *__restrict__ psi, const T *__restrict__ q1, int n, int c,
+                                                    T s, T shift0, T shift1, T L, T *__restrict__ xr, int nr, int o0,
+                                                    int o1, int o2) {
+    __shared__ T sh[NA][32][33];
+    const int i0 = blockIdx.x * 32, j = blockIdx.y, k0 = blockIdx.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const size_t N = (size_t)n, NR = (size_t)nr * n;
+    for (int r = ty; r < 32; r += 8) {
+        const int i = i0 + r, k = k0 + tx;
+        if (i >= n || k >= n) continue;
+        const size_t at = (size_t)k + N * ((size_t)j + N * i);
+        if (x0) sh[0][r][tx] = x0[at];
+        if constexpr (NA == 2) sh[NA - 1][r][tx] = x1[at];
+    }
+    __syncthreads();
+    T *out = xr + (size_t)c * NR * NR * NR;
+    for (int r = ty; r < 32; r += 8) {
+        const int i = i0 + tx, k = k0 + r;
+        if (i >= n || k >= n) continue;
+        const T qc = q1[c == 0 ? i : c == 1 ? j : k];
+        const size_t pr = ((size_t)nr * i + o0) + NR * (((size_t)nr * j + o1) + NR * ((size_t)nr * k + o2));
+        T v0;
+        if (x0) v0 = tjmod(((qc + sh[0][tx][r]) + shift0) + L, L);
+        else v0 = (psi[(size_t)i + N * ((size_t)j + N * k) + (size_t)c * N * N * N] + qc) + s;
+        if constexpr (NA == 2) {
+            const T v1 = tjmod(((qc + sh[NA - 1][tx][r]) + shift1) + L, L);
+            if (nr == 2) {
+                *(cx<T> *)(out + pr) = cx<T>{v0, v1};  // o0 = 0: pr is even
+            } else {
+                out[pr] = v0;
+                out[pr + 1] = v1;
+            }
+        } else {
+            out[pr] = v0;
+        }
+    }
 }
 
 // the particles' own positions of the pass, X_c + s_c = (psi_c + q_c) + s_c (the deposit's arithmetic), at
@@ -102,23 +160,6 @@ __global__ __launch_bounds__(256) void k_rs_shifted(const T *__restrict__ psi, c
     out[pr + 2 * NR3] = (psi[p + 2 * N * N * N] + q1[k]) + s2;
 }
 
-// 1-D assignment weights and base cell (pm.jl:49-55), as in the particle kernels
-template <int W, typename T> __device__ __forceinline__ T rs_wk(T d) {
-    if constexpr (W == 2) {
-        const T a = (T)1 - d;
-        return d > (T)1 ? (T)0 : a;
-    } else if constexpr (W == 3) {
-        const T t = (T)1.5 - d;
-        const T outer = (T)0.5 * (t * t), inner = (T)0.75 - d * d;
-        return d > (T)1.5 ? (T)0 : (d > (T)0.5 ? outer : inner);
-    } else {
-        const T t = (T)2 - d;
-        const T outer = t * t * t / (T)6;
-        const T inner = ((T)4 - (T)6 * (d * d) + (T)3 * (d * d * d)) / (T)6;
-        return d > (T)2 ? (T)0 : (d > (T)1 ? outer : inner);
-    }
-}
-
 // unit-mass deposit of the positions X (3, n^3) with device atomics, added to a mesh that the tile
 // deposit has already written (float atomics, or int64 fixed point when FIXED)
 template <typename T, int W, bool FIXED>
@@ -131,13 +172,13 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const T *__restrict__ X, int
     int cell[3][W];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-        const T g = rs_jmod(X[p + a * np], L) / L * (T)res;
+        const T g = tjmod(X[p + a * np], L) / L * (T)res;
         const int b = (W % 2 == 0) ? (int)floor(g) : (int)rint(g);
         const int lo = W == 2 ? 0 : -1;
 #pragma unroll
         for (int o = 0; o < W; o++) {
             const int bo = b + lo + o;
-            w[a][o] = rs_wk<W>(fabs(g - (T)bo));
+            w[a][o] = twk<W>(fabs(g - (T)bo));
             int cc = bo % res;
             cell[a][o] = cc < 0 ? cc + res : cc;
         }
@@ -231,12 +272,13 @@ __global__ __launch_bounds__(256) void k_rs_trilinear_adj(const T *__restrict__ 
 template <typename T>
 struct RsLaunch {
     static dim3 pgrid(int n) { return dim3((n + 255) / 256, n, n); }
+    static dim3 tgrid(int n) { return dim3((n + 31) / 32, n, (n + 31) / 32); }
     static void wrap(const void *psi, const void *q1, int n, int c, double sc, double L, bool transposed, void *out,
                      hipStream_t st) {
         if (transposed)
-            k_rs_wrap<T, true><<<pgrid(n), 256, 0, st>>>((const T *)psi, (const T *)q1, n, c, (T)sc, (T)L, (T *)out);
+            k_rs_wrap_t<T><<<tgrid(n), 256, 0, st>>>((const T *)psi, (const T *)q1, n, c, (T)sc, (T)L, (T *)out);
         else
-            k_rs_wrap<T, false><<<pgrid(n), 256, 0, st>>>((const T *)psi, (const T *)q1, n, c, (T)sc, (T)L, (T *)out);
+            k_rs_wrap<T><<<pgrid(n), 256, 0, st>>>((const T *)psi, (const T *)q1, n, c, (T)sc, (T)L, (T *)out);
     }
     static void phase(const void *in, void *out, int n, const void *px, const void *py, const void *pz, double scale,
                       hipStream_t st) {
@@ -246,14 +288,20 @@ struct RsLaunch {
     static void trilinear(const void *f, int n, const double *d, void *out, hipStream_t st) {
         k_rs_trilinear<T><<<pgrid(n), 256, 0, st>>>((const T *)f, n, (T)d[0], (T)d[1], (T)d[2], (T *)out);
     }
-    static void place(const void *npsi, const void *q1, int n, int c, double shift, double L, bool transposed, void *xr,
-                      int nr, const int *o, hipStream_t st) {
-        if (transposed)
-            k_rs_place<T, true><<<pgrid(n), 256, 0, st>>>((const T *)npsi, (const T *)q1, n, c, (T)shift, (T)L, (T *)xr,
-                                                          nr, o[0], o[1], o[2]);
+    static void place(const void *npsi, const void *q1, int n, int c, double shift, double L, void *xr, int nr,
+                      const int *o, hipStream_t st) {
+        k_rs_place<T><<<pgrid(n), 256, 0, st>>>((const T *)npsi, (const T *)q1, n, c, (T)shift, (T)L, (T *)xr, nr,
+                                                o[0], o[1], o[2]);
+    }
+    static void place_t(const void *x0, const void *x1, int na, const void *psi, const void *q1, int n, int c, double s,
+                        const double *shift, double L, void *xr, int nr, const int *o, hipStream_t st) {
+        if (na == 2)
+            k_rs_place_t<T, 2><<<tgrid(n), 256, 0, st>>>((const T *)x0, (const T *)x1, (const T *)psi, (const T *)q1, n,
+                                                         c, (T)s, (T)shift[0], (T)shift[1], (T)L, (T *)xr, nr, o[0],
+                                                         o[1], o[2]);
         else
-            k_rs_place<T, false><<<pgrid(n), 256, 0, st>>>((const T *)npsi, (const T *)q1, n, c, (T)shift, (T)L, (T *)xr,
-                                                           nr, o[0], o[1], o[2]);
+            k_rs_place_t<T, 1><<<tgrid(n), 256, 0, st>>>((const T *)x0, nullptr, (const T *)psi, (const T *)q1, n, c,
+                                                         (T)s, (T)shift[0], (T)0, (T)L, (T *)xr, nr, o[0], o[1], o[2]);
     }
     static void extract(const void *pl, int n, int nr, const int *o, int c, bool transposed, void *out,
                         hipStream_t st) {
@@ -305,6 +353,7 @@ template <typename T> void resample_ops(ResampleOps &ops) {
     ops.phase = RsLaunch<T>::phase;
     ops.trilinear = RsLaunch<T>::trilinear;
     ops.place = RsLaunch<T>::place;
+    ops.place_t = RsLaunch<T>::place_t;
     ops.shifted = RsLaunch<T>::shifted;
     ops.scatter = RsLaunch<T>::scatter;
 }
