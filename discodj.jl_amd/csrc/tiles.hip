@@ -26,8 +26,6 @@ template <> struct alignas(16) Entry<float> { float x, y, z; int idx; };
 template <> struct alignas(16) Entry<double> { double x, y, z; int idx; int pad; };
 
 // ------------------------------------------------------------------------------------ binning
-constexpr unsigned EMPTY = 0xffffffffu;
-
 // Tiles of one particle.  The stencil cells of every shift along an axis lie within c0 + [rlo, rhi],
 // a span shorter than the tile, so the axis touches at most the two tiles {tile(c0 + rlo),
 // tile(c0 + rhi)}.  The particle's ghost tiles are the combinations of those per-axis tiles other
@@ -77,50 +75,104 @@ __device__ __forceinline__ int tdiff(int t, int b, int nt) {
     return d <= -((nt + 1) / 2) ? d + nt : d;
 }
 
-// list keys (tile * 2, + 1 for a ghost list) and window slots (-1: outside): index 8 is the own tile's,
-// c that of ghost combination c, or EMPTY when the combination does not exist or is the own tile.  The
-// per-axis parts (list index, window offset, in-window and own-tile tests of tl, th and to) are formed
-// once; each combination then selects and adds them (its selections are compile-time constants).
-struct AxisParts {
-    int k[3], sl[3];       // [tl, th, to]: tile index term, window slot term
-    bool in[3], eqo[2];    // [tl, th, to] inside the window; tl, th equal to the own tile's coordinate
-    bool two;              // th != tl
+// Per axis of a particle: the tile index and window slot terms of tl, th and to.  The lists a wave's particles
+// join are kept as 64-bit lane masks in scalar registers (BinMasks): combination c's mask is a few scalar ands,
+// and a combination that no lane joins (about half of them for 32 x 8 cells of a wave) costs nothing more.
+struct AxisTerms {
+    int k[3], sl[3];  // [tl, th, to]
+};
+struct BinMasks {
+    unsigned long long two[3];    // th != tl
+    unsigned long long eq[2][3];  // tl, th equal to the own tile's coordinate
+    unsigned long long in[3][3];  // tl, th, to inside the window
 };
 
-__device__ __forceinline__ void axis_parts(int tl, int th, int to, int tb, int nt, int wd, int mulk, int muls,
-                                           AxisParts &A) {
-    const int t3[3] = {tl, th, to};
-#pragma unroll
-    for (int h = 0; h < 3; h++) {
-        const int d = tdiff(t3[h], tb, nt) + wd / 2;
-        A.in[h] = (unsigned)d < (unsigned)wd;
-        A.k[h] = t3[h] * mulk;
-        A.sl[h] = d * muls;
+// Lists of a particle: combination C < 8 its ghost lists, 8 its own list
+constexpr int OWN = 8;
+template <int C, int AXIS> constexpr int axis_of() { return C == OWN ? 2 : (C >> AXIS) & 1; }
+template <int C> __device__ __forceinline__ unsigned long long joins(const BinMasks &M, unsigned long long ok) {
+    if constexpr (C < OWN) {
+        if (C & 1) ok &= M.two[0];
+        if (C & 2) ok &= M.two[1];
+        if (C & 4) ok &= M.two[2];
+        ok &= ~(M.eq[C & 1][0] & M.eq[(C >> 1) & 1][1] & M.eq[(C >> 2) & 1][2]);
     }
-    A.eqo[0] = tl == to;
-    A.eqo[1] = th == to;
-    A.two = th != tl;
+    return ok;
+}
+template <int C> __device__ __forceinline__ unsigned long long in_window(const BinMasks &M) {
+    return M.in[axis_of<C, 0>()][0] & M.in[axis_of<C, 1>()][1] & M.in[axis_of<C, 2>()][2];
+}
+template <int C> __device__ __forceinline__ int window_slot(const AxisTerms (&A)[3]) {
+    return 2 * (A[0].sl[axis_of<C, 0>()] + A[1].sl[axis_of<C, 1>()] + A[2].sl[axis_of<C, 2>()]) + (C < OWN ? 1 : 0);
+}
+template <int C> __device__ __forceinline__ unsigned tile_of(const AxisTerms (&A)[3]) {
+    return (unsigned)(A[0].k[axis_of<C, 0>()] + A[1].k[axis_of<C, 1>()] + A[2].k[axis_of<C, 2>()]);
 }
 
-template <int C>
-__device__ __forceinline__ void combo_key(const AxisParts (&A)[3], unsigned &key, int &slot) {
-    constexpr int sx = C & 1, sy = (C >> 1) & 1, sz = (C >> 2) & 1;
-    const bool exists = (!sx || A[0].two) && (!sy || A[1].two) && (!sz || A[2].two) &&
-                        !(A[0].eqo[sx] && A[1].eqo[sy] && A[2].eqo[sz]);
-    key = exists ? (unsigned)(A[0].k[sx] + A[1].k[sy] + A[2].k[sz]) * 2u + 1u : EMPTY;
-    slot = exists && A[0].in[sx] && A[1].in[sy] && A[2].in[sz] ? 2 * (A[0].sl[sx] + A[1].sl[sy] + A[2].sl[sz]) + 1
-                                                                : -1;
-}
-
+// Ranks within the workgroup's counters.  Where every active lane of the wave joins the same list (the common
+// case), one lane adds the group's size and each lane takes the group base plus its position, so a wave's
+// particles stay contiguous (in Lagrangian order) in their list; otherwise each lane makes its own LDS atomic.
 template <int C = 0>
-__device__ __forceinline__ void combo_keys(const AxisParts (&A)[3], unsigned (&key)[9], int (&slot)[9]) {
-    if constexpr (C < 8) {
-        combo_key<C>(A, key[C], slot[C]);
-        combo_keys<C + 1>(A, key, slot);
-    } else {
-        key[8] = (unsigned)(A[0].k[2] + A[1].k[2] + A[2].k[2]) * 2u;
-        slot[8] = A[0].in[2] && A[1].in[2] && A[2].in[2] ? 2 * (A[0].sl[2] + A[1].sl[2] + A[2].sl[2]) : -1;
+__device__ __forceinline__ void rank_lists(const BinMasks &M, unsigned long long ok, const AxisTerms (&A)[3],
+                                           unsigned *vals, int lane, unsigned (&rank)[9]) {
+    const unsigned long long w = joins<C>(M, ok) & in_window<C>(M);
+    rank[C] = 0;
+    if (w) {
+        const int sl = window_slot<C>(A), leader = __ffsll((long long)w) - 1;
+        const int ls = __builtin_amdgcn_readlane(sl, leader);
+        if ((__ballot(sl == ls) & w) == w) {
+            unsigned b = 0;
+            if (lane == leader) b = atomicAdd(&vals[ls], (unsigned)__popcll(w));
+            b = (unsigned)__builtin_amdgcn_readlane((int)b, leader);
+            rank[C] = __builtin_amdgcn_mbcnt_hi((unsigned)(w >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)w, b));
+        } else if (__builtin_amdgcn_inverse_ballot_w64(w)) {
+            rank[C] = atomicAdd(&vals[sl], 1u);
+        }
     }
+    if constexpr (C < OWN) rank_lists<C + 1>(M, ok, A, vals, lane, rank);
+}
+
+// lists outside the window count directly
+template <int C = 0>
+__device__ __forceinline__ void count_outside(const BinMasks &M, unsigned long long ok, const AxisTerms (&A)[3],
+                                              unsigned *cnt, int nt) {
+    const unsigned long long m = joins<C>(M, ok) & ~in_window<C>(M);
+    if (m && __builtin_amdgcn_inverse_ballot_w64(m)) atomicAdd(&cnt[(C < OWN ? nt : 0) + tile_of<C>(A)], 1u);
+    if constexpr (C < OWN) count_outside<C + 1>(M, ok, A, cnt, nt);
+}
+
+// the particle's entry into every list it joins; false when one of them has no room left
+template <typename T, int C = 0>
+__device__ __forceinline__ bool fill_lists(const BinMasks &M, unsigned long long ok, const AxisTerms (&A)[3],
+                                           const uint2 *room, const unsigned (&rank)[9], const Entry<T> &e,
+                                           Entry<T> *__restrict__ ent, unsigned cap, unsigned *own_at, unsigned *cur,
+                                           const unsigned *__restrict__ start, const unsigned *__restrict__ gstart,
+                                           int nt) {
+    bool fits = true;
+    const unsigned long long m = joins<C>(M, ok), w = m & in_window<C>(M);
+    if (m) {
+        unsigned at = 0, end = 0;
+        if (__builtin_amdgcn_inverse_ballot_w64(w)) {
+            const uint2 r = room[window_slot<C>(A)];
+            at = r.x + rank[C];
+            end = r.y;
+        }
+        if (m != w && __builtin_amdgcn_inverse_ballot_w64(m & ~w)) {  // a list outside the workgroup's window
+            const unsigned t = tile_of<C>(A), r = atomicAdd(&cur[(C < OWN ? nt : 0) + t], 1u);
+            at = (C < OWN ? gstart[t] : start[t]) + r;
+            end = min(C < OWN ? start[t + 1] : gstart[t], cap);
+        }
+        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+            fits = at < end;
+            if (fits) {
+                ent[at] = e;
+                if (C == OWN && own_at) own_at[e.idx] = at;
+            }
+        }
+    }
+    if constexpr (C < OWN)
+        fits &= fill_lists<T, C + 1>(M, ok, A, room, rank, e, ent, cap, own_at, cur, start, gstart, nt);
+    return fits;
 }
 
 template <typename T, int W, bool FILL>
@@ -128,23 +180,24 @@ __global__ __launch_bounds__(256) void k_tile_bin(const T *__restrict__ psi, con
                                                   const double *__restrict__ shifts, int ns, T L, TileGeom g,
                                                   unsigned *cnt, const unsigned *__restrict__ start,
                                                   const unsigned *__restrict__ gstart, unsigned *cur, unsigned *flag,
-                                                  Entry<T> *__restrict__ ent, size_t ent_cap, unsigned *own_at) {
-    __shared__ unsigned vals[BSLOTS], base[BSLOTS], lend[BSLOTS];
+                                                  Entry<T> *__restrict__ ent, unsigned cap, unsigned *own_at) {
+    __shared__ unsigned vals[BSLOTS];
+    __shared__ uint2 room[FILL ? BSLOTS : 1];  // per window list: the group's first entry, the list's end
     __shared__ int tbs[3];
     for (int s = threadIdx.x; s < BSLOTS; s += 256) vals[s] = 0;
     // 16 x 4 x 4 Lagrangian block of particles per workgroup (thread 0's particle always exists)
     const int i = blockIdx.x * 16 + (threadIdx.x & 15), j = blockIdx.y * 4 + ((threadIdx.x >> 4) & 3),
               k = blockIdx.z * 4 + (threadIdx.x >> 6);
     const bool ok = i < n && j < n && k < n;
-    T X[3] = {0, 0, 0};
-    size_t p = 0;
+    Entry<T> e{};
     PartTiles P{};
     if (ok) {
-        const size_t np = (size_t)n * n * n;
-        p = (size_t)i + (size_t)n * ((size_t)j + (size_t)n * k);
-        X[0] = psi[p] + q1[i];
-        X[1] = psi[p + np] + q1[j];
-        X[2] = psi[p + 2 * np] + q1[k];
+        const size_t np = (size_t)n * n * n, p = (size_t)i + (size_t)n * ((size_t)j + (size_t)n * k);
+        const T X[3] = {psi[p] + q1[i], psi[p + np] + q1[j], psi[p + 2 * np] + q1[k]};
+        e.x = X[0];
+        e.y = X[1];
+        e.z = X[2];
+        e.idx = (int)p;
         P = particle_tiles<T, W>(X, g, shifts, ns, L);
     }
     if (threadIdx.x == 0) {
@@ -154,51 +207,30 @@ __global__ __launch_bounds__(256) void k_tile_bin(const T *__restrict__ psi, con
     }
     __syncthreads();
     const int tb[3] = {tbs[0], tbs[1], tbs[2]};
-    // the particle's list keys and window slots (every index below is a compile-time constant once the
-    // loops are unrolled, so the arrays stay in registers without indexed selects)
-    unsigned key[9];
-    int slot[9], rank[9];
-    if (ok) {
-        AxisParts A[3];
-        axis_parts(P.tl[0], P.th[0], P.to[0], tb[0], g.ntx, BWX, 1, 1, A[0]);
-        axis_parts(P.tl[1], P.th[1], P.to[1], tb[1], g.nty, BWY, g.ntx, BWX, A[1]);
-        axis_parts(P.tl[2], P.th[2], P.to[2], tb[2], g.ntz, BWZ, g.ntx * g.nty, BWX * BWY, A[2]);
-        combo_keys(A, key, slot);
-    } else {
+    const int wd[3] = {BWX, BWY, BWZ}, mulk[3] = {1, g.ntx, g.ntx * g.nty}, muls[3] = {1, BWX, BWX * BWY},
+              ntl[3] = {g.ntx, g.nty, g.ntz}, lane = __lane_id();
+    AxisTerms A[3];
+    BinMasks M;
+    const unsigned long long okm = __ballot(ok);
 #pragma unroll
-        for (int c = 0; c < 9; c++) {
-            key[c] = EMPTY;
-            slot[c] = -1;
-        }
-    }
-    // Ranks within the workgroup's counters.  Where every active lane of the wave joins the same list
-    // (the common case), one lane adds the group's size and each lane takes the group base plus its
-    // position, so a wave's particles stay contiguous (in Lagrangian order) in their list; otherwise each
-    // lane makes its own LDS atomic.
-    const int lane = __lane_id();
-    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int a = 0; a < 3; a++) {
+        const int t3[3] = {P.tl[a], P.th[a], P.to[a]};
 #pragma unroll
-    for (int c = 0; c < 9; c++) {
-        rank[c] = -1;
-        const bool act = key[c] != EMPTY && slot[c] >= 0;
-        const unsigned long long am = __ballot(act);
-        if (am) {
-            const int leader = __ffsll((long long)am) - 1;
-            const int ls = __builtin_amdgcn_readlane(slot[c], leader);
-            const unsigned long long sm = __ballot(act && slot[c] == ls);
-            if (sm == am) {
-                unsigned b = 0;
-                if (lane == leader) b = atomicAdd(&vals[ls], (unsigned)__popcll(am));
-                b = (unsigned)__builtin_amdgcn_readlane((int)b, leader);
-                if (act) rank[c] = (int)(b + (unsigned)__popcll(am & below));
-            } else if (act) {
-                rank[c] = (int)atomicAdd(&vals[slot[c]], 1u);
-            }
+        for (int h = 0; h < 3; h++) {
+            const int d = tdiff(t3[h], tb[a], ntl[a]) + wd[a] / 2;
+            M.in[h][a] = __ballot((unsigned)d < (unsigned)wd[a]);
+            A[a].k[h] = t3[h] * mulk[a];
+            A[a].sl[h] = d * muls[a];
         }
+        M.two[a] = __ballot(P.th[a] != P.tl[a]);
+        M.eq[0][a] = __ballot(P.tl[a] == P.to[a]);
+        M.eq[1][a] = __ballot(P.th[a] == P.to[a]);
     }
+    unsigned rank[9];
+    rank_lists(M, okm, A, vals, lane, rank);
     __syncthreads();
     // one global atomic per window list in use; the fill also records the group's first entry and its
-    // list's end (own list [start[t], gstart[t]), ghost list [gstart[t], start[t + 1]))
+    // list's end (own list [start[t], gstart[t]), ghost list [gstart[t], start[t + 1]), within the buffer)
     for (int s = threadIdx.x; s < BSLOTS; s += 256) {
         const unsigned v = vals[s];
         if (!v) continue;
@@ -207,52 +239,22 @@ __global__ __launch_bounds__(256) void k_tile_bin(const T *__restrict__ psi, con
         const int tx = timod(tb[0] + r % BWX - BWX / 2, g.ntx), ty = timod(tb[1] + (r / BWX) % BWY - BWY / 2, g.nty),
                   tz = timod(tb[2] + r / (BWX * BWY) - BWZ / 2, g.ntz);
         const unsigned t = (unsigned)(tx + g.ntx * (ty + g.nty * tz));
-        if (!FILL) {
+        if constexpr (!FILL) {
             atomicAdd(&cnt[gh * g.nt + t], v);
         } else {
             const unsigned b = atomicAdd(&cur[gh * g.nt + t], v);
-            base[s] = (gh ? gstart[t] : start[t]) + b;
-            lend[s] = gh ? start[t + 1] : gstart[t];
+            room[s] = make_uint2((gh ? gstart[t] : start[t]) + b, min(gh ? start[t + 1] : gstart[t], cap));
         }
     }
-    if (!FILL) {
-        // lists outside the window count directly
-#pragma unroll
-        for (int c = 0; c < 9; c++)
-            if (key[c] != EMPTY && slot[c] < 0) atomicAdd(&cnt[(key[c] & 1u) * g.nt + (key[c] >> 1)], 1u);
-        return;
+    if constexpr (!FILL) {
+        count_outside(M, okm, A, cnt, g.nt);
+    } else {
+        __syncthreads();
+        const bool fits = fill_lists<T>(M, okm, A, room, rank, e, ent, cap, own_at, cur, start, gstart, g.nt);
+        // capacity exceeded: the host repeats the sort with exact counts (one flag atomic per wave; a
+        // buffer that is much too small would otherwise have every lane hit the one flag word)
+        if (__any(!fits) && lane == 0) atomicOr(flag, 1u);
     }
-    __syncthreads();
-    bool over = false;
-#pragma unroll
-    for (int c = 0; c < 9; c++) {
-        if (key[c] == EMPTY) continue;
-        const unsigned t = key[c] >> 1;
-        const bool gh = key[c] & 1u;
-        unsigned at, end;
-        if (slot[c] >= 0) {
-            at = base[slot[c]] + (unsigned)rank[c];
-            end = lend[slot[c]];
-        } else {  // a list outside the workgroup's window
-            const unsigned r = atomicAdd(&cur[(gh ? g.nt : 0) + t], 1u);
-            at = (gh ? gstart[t] : start[t]) + r;
-            end = gh ? start[t + 1] : gstart[t];
-        }
-        if (at < end && at < ent_cap) {
-            Entry<T> e;
-            e.x = X[0];
-            e.y = X[1];
-            e.z = X[2];
-            e.idx = (int)p;
-            ent[at] = e;
-            if (c == 8 && own_at) own_at[p] = at;
-        } else {
-            over = true;
-        }
-    }
-    // capacity exceeded: the host repeats the sort with exact counts (one flag atomic per wave; a
-    // buffer that is much too small would otherwise have every lane hit the one flag word)
-    if (__any(over) && __lane_id() == 0) atomicOr(flag, 1u);
 }
 
 // List capacities of every tile from counts src (own, then ghost; src may be the fill cursors of
@@ -1319,14 +1321,14 @@ struct TileLaunch {
         dim3 grid((a.n + 15) / 16, (a.n + 3) / 4, (a.n + 3) / 4);
         k_tile_bin<T, W, false><<<grid, 256, 0, st>>>((const T *)a.psi, (const T *)a.q1, a.n, a.shifts, a.ns, (T)a.L,
                                                       a.g, a.cnt, a.start, a.gstart, a.cur, a.flag, (Entry<T> *)a.ent,
-                                                      a.ent_cap, a.own_at);
+                                                      cap32(a), a.own_at);
     }
     template <int W>
     static void fill_w(const TileArgs &a, hipStream_t st) {
         dim3 grid((a.n + 15) / 16, (a.n + 3) / 4, (a.n + 3) / 4);
         k_tile_bin<T, W, true><<<grid, 256, 0, st>>>((const T *)a.psi, (const T *)a.q1, a.n, a.shifts, a.ns, (T)a.L,
                                                      a.g, a.cnt, a.start, a.gstart, a.cur, a.flag, (Entry<T> *)a.ent,
-                                                     a.ent_cap, a.own_at);
+                                                     cap32(a), a.own_at);
     }
     static void count(const TileArgs &a, int W, hipStream_t st) {
         if (W == 2) bin_w<2>(a, st); else if (W == 3) bin_w<3>(a, st); else bin_w<4>(a, st);
