@@ -15,6 +15,8 @@
 // convolution of the backward pass is the same kernel with the flipped, transposed taps.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dj_internal.h"
 
 namespace dj {
@@ -22,12 +24,10 @@ namespace dj {
 typedef short s4v __attribute__((ext_vector_type(4)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-// FP32 -> BF16 round to nearest even (finite values); BF16 -> FP32 exact
-__device__ __forceinline__ unsigned short f2bf(float x) {
-    unsigned u = __float_as_uint(x);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
+// FP32 -> BF16 round to nearest even (the conversion instruction); BF16 -> FP32 exact
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ unsigned short f2bf(float x) { return __builtin_bit_cast(unsigned short, (__bf16)x); }
+__device__ __forceinline__ s4v f2bf4(f4v x) { return __builtin_bit_cast(s4v, __builtin_convertvector(x, bf4)); }
 __device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
 
 __device__ __forceinline__ float nn_input(float dens, float inv_rho) {
@@ -39,67 +39,72 @@ __device__ __forceinline__ int nn_wrap(int v, int N) { return v < 0 ? v + N : (v
 
 enum { NN_IN_H = 0, NN_IN_FIELD = 1, NN_IN_GRAD = 2 };  // B: 16-channel tensor / density field / 1-channel float
 enum { NN_EPI_HIDDEN = 0, NN_EPI_OUT = 1, NN_EPI_BWD = 2 };
+enum { NN_RES_NONE = 0, NN_RES_INPUT = 1, NN_RES_TENSOR = 2 };  // the residual: none, the layer's input, another tensor
 
-// B operand of one tap: channels 4 (l/16) .. +3 of voxel v
-template <int IN>
-__device__ __forceinline__ s4v nn_bop(const unsigned short *hin, const float *fin, float inv_rho, float cval, size_t v,
-                                      int cg) {
-    s4v b = {0, 0, 0, 0};
-    if constexpr (IN == NN_IN_H) {
-        b = *(const s4v *)(hin + v * 16 + cg);
-    } else if (cg == 0) {
-        // density field: the net's input transform; gradient field: scaled by inv_rho
-        const float f = IN == NN_IN_FIELD ? nn_input(fin[v], inv_rho) : fin[v] * inv_rho;
-        b[0] = (short)f2bf(f);
-        b[1] = (short)f2bf(cval);
-    }
-    return b;
-}
+// One block marches along z over a 64 (x) x 8 (y) footprint: the input planes z-1, z, z+1 (with a one-voxel x-y
+// halo, 66 x 10 voxels) sit in a three-slot LDS ring, so each input voxel is read from memory about 1.3 times
+// instead of once per tap.  Two blocks share a CU (63 KB of LDS each).  Wave w computes y rows 2w, 2w+1 of the
+// plane (8 segments of 16 voxels), per tap one MFMA per segment.  The taps' weights (A) stay in registers for
+// the whole march; an input row (B) is read from LDS once for the two output rows that use it (48 reads of 8
+// bytes a lane and input plane instead of 72); and the plane after the next is loaded into registers while the
+// current one is computed, so a plane costs its MFMAs (16 cycles each, 216 a wave) and not the loads' latency.
+// Every output adds its taps in the order dz, dy, dx.  Hidden layer at 256^3: 0.34 ms (matrix cores 62 % busy),
+// against 0.56 with A in LDS, every tap its own read and the loads before the barrier; first layer 0.17 (0.35),
+// last 0.27 (0.41).
+constexpr int NN_TX = 64, NN_TY = 8, NN_PX = NN_TX + 2, NN_PY = NN_TY + 2, NN_PV = NN_PX * NN_PY;
+// A 16-channel plane in LDS is four planes of 8-byte units (4 channels), NN_PVP units apart: a wave's read of 16
+// neighbouring voxels' units in each is 4 x 128 contiguous bytes that meet no bank twice (NN_PVP = 16 mod 32
+// puts neighbouring channel groups on the two halves of the 64 banks).  Channel-last voxels, 32 bytes apart,
+// made 30 LDS cycles of every 8.
+constexpr int NN_PVP = 688;
+static_assert(NN_PVP >= NN_PV && NN_PVP % 32 == 16, "channel planes on alternating bank halves");
 
-// One block marches along z over a 64 (x) x 8 (y) footprint, 16 planes: the input planes z-1, z, z+1
-// (with a one-voxel x-y halo, 66 x 10 voxels) sit in a three-slot LDS ring, so each input voxel is
-// read from memory about 1.3 times instead of once per tap.  Two blocks share a CU (77 KB of LDS
-// each), so one stages while the other computes.  Wave w computes y rows 2w, 2w+1 of the plane (8
-// segments of 16 voxels), per tap one MFMA per segment with B read from LDS (8 bytes per lane,
-// conflict-free) and A (the tap's weights) from LDS.
-constexpr int NN_TX = 64, NN_TY = 8, NN_TZ = 16, NN_PX = NN_TX + 2, NN_PY = NN_TY + 2, NN_PV = NN_PX * NN_PY;
-constexpr int NN_CHUNKS = NN_PV * 2;                       // 16-byte chunks of a 16-channel plane
-constexpr int NN_PER = (NN_CHUNKS + 255) / 256;            // chunks per thread
-
-// stage input plane zz (wrapped) of the block's footprint into an LDS slot as 16-channel BF16; a field
-// input becomes (bf16(input), bf16(cval), 0, ...)
-template <int IN>
-__device__ __forceinline__ void nn_plane_stage(unsigned short *slot, const unsigned short *hin, const float *fin, int N,
-                                               int x0, int y0, int zz, float inv_rho, float cval) {
-    const size_t zb = (size_t)N * N * nn_wrap(zz, N);
-    if constexpr (IN == NN_IN_H) {
+// This thread's part of an input plane of the footprint: PER units in registers between load() and store().
+// 16-channel tensors move in 16-byte halves of a voxel; a field becomes one 4-byte pair (bf16(input),
+// bf16(cval)) per voxel (gradient field: scaled by inv_rho).
+template <int IN> struct PlaneStage {
+    static constexpr bool H = IN == NN_IN_H;
+    static constexpr int UNITS = H ? 2 * NN_PV : NN_PV, PER = (UNITS + 255) / 256;
+    using Unit = typename std::conditional<H, uint4, float>::type;
+    unsigned off[PER];  // of the unit in the plane (units of 8 channels, or voxels)
+    Unit v[PER];
+    __device__ __forceinline__ void init(int N, int x0, int y0) {
 #pragma unroll
-        for (int k = 0; k < NN_PER; k++) {
-            const int ch = threadIdx.x + 256 * k;
-            if (ch < NN_CHUNKS) {
-                const int vox = ch >> 1, xi = vox % NN_PX, yi = vox / NN_PX;
-                const size_t v = zb + (size_t)nn_wrap(x0 - 1 + xi, N) + (size_t)N * nn_wrap(y0 - 1 + yi, N);
-                *(uint4 *)(slot + ch * 8) = *(const uint4 *)(hin + v * 16 + (ch & 1) * 8);
-            }
-        }
-    } else {
-        // a field input has two channels, (input, cval): one 4-byte pair per voxel
-        const unsigned c1 = (unsigned)f2bf(cval) << 16;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const int vox = threadIdx.x + 256 * k;
-            if (vox < NN_PV) {
-                const int xi = vox % NN_PX, yi = vox / NN_PX;
-                const float fv = fin[zb + (size_t)nn_wrap(x0 - 1 + xi, N) + (size_t)N * nn_wrap(y0 - 1 + yi, N)];
-                const float x = IN == NN_IN_FIELD ? nn_input(fv, inv_rho) : fv * inv_rho;
-                ((unsigned *)slot)[vox] = (unsigned)f2bf(x) | c1;
-            }
+        for (int k = 0; k < PER; k++) {
+            const int u = min((int)threadIdx.x + 256 * k, UNITS - 1), vox = H ? u >> 1 : u;
+            const int xi = vox % NN_PX, yi = vox / NN_PX;
+            const unsigned p = (unsigned)nn_wrap(x0 - 1 + xi, N) + (unsigned)N * (unsigned)nn_wrap(y0 - 1 + yi, N);
+            off[k] = H ? 2 * p + (u & 1) : p;
         }
     }
-}
+    __device__ __forceinline__ void load(const unsigned short *hin, const float *fin, int N, int z) {
+        const size_t zb = (size_t)N * N * nn_wrap(z, N);
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            if constexpr (H) v[k] = ((const uint4 *)hin)[2 * zb + off[k]];
+            else v[k] = fin[zb + off[k]];
+        }
+    }
+    __device__ __forceinline__ void store(unsigned short *slot, float inv_rho, unsigned c1) const {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int u = threadIdx.x + 256 * k;
+            if (u >= UNITS) continue;
+            if constexpr (H) {
+                uint2 *d = (uint2 *)slot + (u & 1) * (2 * NN_PVP) + (u >> 1);
+                d[0] = make_uint2(v[k].x, v[k].y);
+                d[NN_PVP] = make_uint2(v[k].z, v[k].w);
+            } else {
+                const float x = IN == NN_IN_FIELD ? nn_input(v[k], inv_rho) : v[k] * inv_rho;
+                ((unsigned *)slot)[u] = (unsigned)f2bf(x) | c1;
+            }
+        }
+    }
+};
+template <int IN> constexpr size_t nn_conv_lds() { return 3 * (IN == NN_IN_H ? (size_t)NN_PVP * 32 : (size_t)NN_PV * 4); }
 
-template <int IN, int EPI>
-__global__ __launch_bounds__(256, 2) void k_nn_conv(int N, const unsigned short *__restrict__ hin,
+template <int IN, int EPI, int RES>
+__global__ __launch_bounds__(256, 2) void k_nn_conv(int N, int tz, const unsigned short *__restrict__ hin,
                                                     const float *__restrict__ fin, float inv_rho, float cval,
                                                     const s4v *__restrict__ wsw, const float *__restrict__ bias,
                                                     const unsigned short *__restrict__ res,
@@ -107,95 +112,128 @@ __global__ __launch_bounds__(256, 2) void k_nn_conv(int N, const unsigned short 
                                                     unsigned short *__restrict__ out_z, unsigned short *__restrict__ out_h,
                                                     float *__restrict__ out_f, float oscale) {
     extern __shared__ unsigned char nn_smem[];
-    s4v *wl = (s4v *)nn_smem;                                           // 27 x 64 lane-ordered A operands
-    unsigned short *ring = (unsigned short *)(nn_smem + 27 * 64 * 8);   // 3 x NN_PV x 16 BF16
+    constexpr int SLOT = IN == NN_IN_H ? NN_PVP * 16 : NN_PV * 2, NA = IN == NN_IN_H ? 27 : 4;
+    unsigned short *ring = (unsigned short *)nn_smem;  // 3 planes
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cg = 4 * (lane >> 4), lx = lane & 15;
     const int nbx = N / NN_TX, nby = N / NN_TY;
     const int x0 = (blockIdx.x % nbx) * NN_TX, y0 = ((blockIdx.x / nbx) % nby) * NN_TY,
-              z0 = (blockIdx.x / (nbx * nby)) * NN_TZ;
-    for (int i = threadIdx.x; i < (IN == NN_IN_H ? 27 : 4) * 64; i += 256) wl[i] = wsw[i];
-    auto slot = [&](int z) { return ring + (size_t)(((z % 3) + 3) % 3) * NN_PV * 16; };
-    nn_plane_stage<IN>(slot(z0 - 1), hin, fin, N, x0, y0, z0 - 1, inv_rho, cval);
-    nn_plane_stage<IN>(slot(z0), hin, fin, N, x0, y0, z0, inv_rho, cval);
-    for (int z = z0; z < z0 + NN_TZ; z++) {
-        nn_plane_stage<IN>(slot(z + 1), hin, fin, N, x0, y0, z + 1, inv_rho, cval);
-        __syncthreads();  // planes z-1, z, z+1 (and the weights) in LDS
+              z0 = (blockIdx.x / (nbx * nby)) * tz;
+    s4v a[NA];
+#pragma unroll
+    for (int t = 0; t < NA; t++) a[t] = wsw[t * 64 + lane];
+    float bs[4] = {0, 0, 0, 0};
+    if constexpr (EPI == NN_EPI_HIDDEN) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) bs[j] = bias[cg + j];
+    } else if constexpr (EPI == NN_EPI_OUT) {
+        bs[0] = bias[0];
+    }
+    const unsigned c1 = (unsigned)f2bf(cval) << 16;
+    PlaneStage<IN> st;
+    st.init(N, x0, y0);
+    // slots of planes z-1, z, z+1
+    unsigned short *s0 = ring, *s1 = ring + SLOT, *s2 = ring + 2 * SLOT;
+    st.load(hin, fin, N, z0 - 1);
+    st.store(s0, inv_rho, c1);
+    st.load(hin, fin, N, z0);
+    st.store(s1, inv_rho, c1);
+    st.load(hin, fin, N, z0 + 1);
+    for (int z = z0; z < z0 + tz; z++) {
+        st.store(s2, inv_rho, c1);
+        if (z + 1 < z0 + tz) st.load(hin, fin, N, z + 2);
+        __syncthreads();  // planes z-1, z, z+1 in LDS
         f4v acc[8];
 #pragma unroll
         for (int sg = 0; sg < 8; sg++) acc[sg] = {0, 0, 0, 0};
         if constexpr (IN == NN_IN_H) {
-#pragma unroll 1
-        for (int dz = -1; dz <= 1; dz++) {
-            const unsigned short *sh = slot(z + dz);
 #pragma unroll
-            for (int dy = -1; dy <= 1; dy++)
+            for (int dz = 0; dz < 3; dz++) {
+                const s4v *sh = (const s4v *)(dz == 0 ? s0 : dz == 1 ? s1 : s2) + (lane >> 4) * NN_PVP +
+                                2 * wave * NN_PX + lx;
 #pragma unroll
-                for (int dx = -1; dx <= 1; dx++) {
-                    const s4v a = wl[((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1)) * 64 + lane];
+                for (int yr = 0; yr < 4; yr++)  // input rows 2w - 1 + yr: dy = yr of row 2w, yr - 1 of row 2w + 1
 #pragma unroll
-                    for (int sg = 0; sg < 8; sg++) {
-                        const int yi = 2 * wave + (sg >> 2) + dy + 1, xi = (sg & 3) * 16 + lx + dx + 1;
-                        const s4v b = *(const s4v *)(sh + (yi * NN_PX + xi) * 16 + cg);
-                        acc[sg] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[sg], 0, 0, 0);
+                    for (int dx = 0; dx < 3; dx++) {
+                        s4v b[4];
+#pragma unroll
+                        for (int sg = 0; sg < 4; sg++) b[sg] = sh[yr * NN_PX + sg * 16 + dx];
+                        if (yr < 3)
+#pragma unroll
+                            for (int sg = 0; sg < 4; sg++)
+                                acc[sg] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[dz * 9 + yr * 3 + dx], b[sg],
+                                                                                   acc[sg], 0, 0, 0);
+                        if (yr > 0)
+#pragma unroll
+                            for (int sg = 0; sg < 4; sg++)
+                                acc[4 + sg] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[dz * 9 + (yr - 1) * 3 + dx],
+                                                                                       b[sg], acc[4 + sg], 0, 0, 0);
                     }
-                }
-        }
+            }
         } else {
             // two input channels: one MFMA takes 8 taps x 2 channels (K = 16), 4 MFMAs for the 27 taps
             // (the 5 extra taps have zero weights); lane k-group 4 (lane / 16) + j reads taps
             // 8 q + 2 (lane / 16) + j / 2, channel j % 2
+            auto slot = [&](int dz) { return (const unsigned *)(dz == 0 ? s0 : dz == 1 ? s1 : s2); };
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const s4v a = wl[q * 64 + lane];
                 const int t1 = min(8 * q + 2 * (lane >> 4), 26), t2 = min(t1 + 1, 26);
-                const unsigned *s1 = (const unsigned *)slot(z + t1 / 9 - 1), *s2 = (const unsigned *)slot(z + t2 / 9 - 1);
-                const int d1 = ((t1 / 3) % 3) * NN_PX + t1 % 3, d2 = ((t2 / 3) % 3) * NN_PX + t2 % 3;
+                const unsigned *p1 = slot(t1 / 9) + ((t1 / 3) % 3) * NN_PX + t1 % 3 + 2 * wave * NN_PX + lx,
+                               *p2 = slot(t2 / 9) + ((t2 / 3) % 3) * NN_PX + t2 % 3 + 2 * wave * NN_PX + lx;
 #pragma unroll
                 for (int sg = 0; sg < 8; sg++) {
-                    const int v0 = (2 * wave + (sg >> 2)) * NN_PX + (sg & 3) * 16 + lx;  // the (-1,-1) corner cell
-                    const unsigned u1 = s1[v0 + d1], u2 = s2[v0 + d2];
+                    const int v0 = (sg >> 2) * NN_PX + (sg & 3) * 16;
+                    const unsigned u1 = p1[v0], u2 = p2[v0];
                     const s4v b = {(short)(u1 & 0xffffu), (short)(u1 >> 16), (short)(u2 & 0xffffu), (short)(u2 >> 16)};
-                    acc[sg] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[sg], 0, 0, 0);
+                    acc[sg] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[q], b, acc[sg], 0, 0, 0);
                 }
             }
         }
-        // epilogue: lane holds D[cg + j][lx] of each segment: channels cg..cg+3 of one voxel
+        // epilogue: lane holds D[cg + j][lx] of each segment: channels cg..cg+3 of one voxel.  What it reads from
+        // memory is read for all segments before the first store (a wait for a load waits for earlier stores).
+        auto voxel = [&](int sg) {
+            return (size_t)(x0 + (sg & 3) * 16 + lx) +
+                   (size_t)N * ((size_t)(y0 + 2 * wave + (sg >> 2)) + (size_t)N * z);
+        };
+        if constexpr (EPI == NN_EPI_OUT) {
+            if (cg == 0)
 #pragma unroll
-        for (int sg = 0; sg < 8; sg++) {
-            const int y = y0 + 2 * wave + (sg >> 2), x = x0 + (sg & 3) * 16 + lx;
-            const size_t v = (size_t)x + (size_t)N * ((size_t)y + (size_t)N * z);
-            if constexpr (EPI == NN_EPI_OUT) {
-                if (cg == 0) out_f[v] = oscale * (acc[sg][0] + bias[0]);
-            } else {
-                s4v zo, ho;
-                s4v rr = {0, 0, 0, 0}, m = {0, 0, 0, 0};
-                if constexpr (IN == NN_IN_H) {
-                    if (res == hin)  // the residual is the layer's input: its centre cell is in the LDS ring
-                        rr = *(const s4v *)(slot(z) + ((2 * wave + (sg >> 2) + 1) * NN_PX + (sg & 3) * 16 + lx + 1) * 16 + cg);
-                    else if (res)
-                        rr = *(const s4v *)(res + v * 16 + cg);
-                } else if (res) {
-                    rr = *(const s4v *)(res + v * 16 + cg);
-                }
-                if constexpr (EPI == NN_EPI_BWD) m = *(const s4v *)(zmask + v * 16 + cg);
+                for (int sg = 0; sg < 8; sg++) out_f[voxel(sg)] = oscale * (acc[sg][0] + bs[0]);
+        } else {
+            s4v rr[8], m[8];
+#pragma unroll
+            for (int sg = 0; sg < 8; sg++) {
+                if constexpr (RES == NN_RES_INPUT)  // its centre cell is in the LDS ring
+                    rr[sg] = ((const s4v *)s1)[(lane >> 4) * NN_PVP + (2 * wave + (sg >> 2) + 1) * NN_PX +
+                                               (sg & 3) * 16 + lx + 1];
+                else if constexpr (RES == NN_RES_TENSOR) rr[sg] = *(const s4v *)(res + voxel(sg) * 16 + cg);
+                else rr[sg] = {0, 0, 0, 0};
+                if constexpr (EPI == NN_EPI_BWD) m[sg] = *(const s4v *)(zmask + voxel(sg) * 16 + cg);
+            }
+#pragma unroll
+            for (int sg = 0; sg < 8; sg++) {
+                f4v zo, ho;
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const float rv = bf2f((unsigned short)rr[j]);
+                    const float rv = bf2f((unsigned short)rr[sg][j]);
                     if constexpr (EPI == NN_EPI_HIDDEN) {
-                        const float zz = acc[sg][j] + bias[cg + j];
-                        zo[j] = (short)f2bf(zz);
-                        ho[j] = (short)f2bf(rv + fmaxf(zz, 0.0f));
+                        const float zz = acc[sg][j] + bs[j];
+                        zo[j] = zz;
+                        ho[j] = rv + fmaxf(zz, 0.0f);
                     } else {
                         const float g = rv + acc[sg][j];
-                        ho[j] = (short)f2bf(g);
-                        zo[j] = (short)f2bf(bf2f((unsigned short)m[j]) > 0.0f ? g : 0.0f);
+                        ho[j] = g;
+                        zo[j] = bf2f((unsigned short)m[sg][j]) > 0.0f ? g : 0.0f;
                     }
                 }
-                if (out_z) *(s4v *)(out_z + v * 16 + cg) = zo;  // pre-activations: kept for training only
-                *(s4v *)(out_h + v * 16 + cg) = ho;
+                if (out_z) *(s4v *)(out_z + voxel(sg) * 16 + cg) = f2bf4(zo);  // pre-activations: kept for training only
+                *(s4v *)(out_h + voxel(sg) * 16 + cg) = f2bf4(ho);
             }
         }
-        __syncthreads();  // slot (z - 1) is overwritten by plane z + 2 next
+        __syncthreads();  // plane z - 1's slot takes plane z + 2 next
+        unsigned short *t = s0;
+        s0 = s1;
+        s1 = s2;
+        s2 = t;
     }
 }
 
@@ -401,26 +439,36 @@ __global__ __launch_bounds__(256) void k_nn_loss_total(double *sum) {
     if (threadIdx.x == 0) sum[NN_LOSS_BLOCKS] = red[0];
 }
 
+#ifndef NNMB
+#define NNMB 256
+#endif
+constexpr int NN_MIN_BLOCKS = NNMB;
 static unsigned ngrid(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 struct NnLaunch {
     static void conv(int in, int epi, int N, const void *hin, const void *fin, double inv_rho, double cval,
                      const void *wsw, const void *bias, const void *res, const void *zmask, void *out_z, void *out_h,
                      void *out_f, double oscale, hipStream_t st) {
-        const dim3 g((N / NN_TX) * (N / NN_TY) * (N / NN_TZ));
-        const size_t shm = (size_t)27 * 64 * 8 + (size_t)3 * NN_PV * 16 * 2;
-#define NN_C(I, E)                                                                                                   \
+        // planes per block: 16, fewer where that leaves the chip's 512 block slots half empty (a 64^3 mesh in
+        // segments of 16 runs on 32 blocks)
+        const int cols = (N / NN_TX) * (N / NN_TY);
+        int tz = 16;
+        while (tz > 1 && cols * (N / tz) < NN_MIN_BLOCKS) tz /= 2;
+        const dim3 g(cols * (N / tz));
+#define NN_C(I, E, R)                                                                                                \
     do {                                                                                                             \
-    (void)hipFuncSetAttribute((const void *)k_nn_conv<I, E>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);   \
-    k_nn_conv<I, E><<<g, 256, shm, st>>>(N, (const unsigned short *)hin, (const float *)fin, (float)inv_rho, (float)cval, \
-                                       (const s4v *)wsw, (const float *)bias, (const unsigned short *)res,              \
-                                       (const unsigned short *)zmask, (unsigned short *)out_z, (unsigned short *)out_h, \
-                                       (float *)out_f, (float)oscale); } while (0)
-        if (in == NN_IN_FIELD && epi == NN_EPI_HIDDEN) NN_C(NN_IN_FIELD, NN_EPI_HIDDEN);
-        else if (in == NN_IN_H && epi == NN_EPI_HIDDEN) NN_C(NN_IN_H, NN_EPI_HIDDEN);
-        else if (in == NN_IN_H && epi == NN_EPI_OUT) NN_C(NN_IN_H, NN_EPI_OUT);
-        else if (in == NN_IN_GRAD && epi == NN_EPI_BWD) NN_C(NN_IN_GRAD, NN_EPI_BWD);
-        else NN_C(NN_IN_H, NN_EPI_BWD);
+        (void)hipFuncSetAttribute((const void *)k_nn_conv<I, E, R>, hipFuncAttributeMaxDynamicSharedMemorySize,       \
+                                  (int)nn_conv_lds<I>());                                                             \
+        k_nn_conv<I, E, R><<<g, 256, nn_conv_lds<I>(), st>>>(                                                          \
+            N, tz, (const unsigned short *)hin, (const float *)fin, (float)inv_rho, (float)cval, (const s4v *)wsw,     \
+            (const float *)bias, (const unsigned short *)res, (const unsigned short *)zmask, (unsigned short *)out_z,  \
+            (unsigned short *)out_h, (float *)out_f, (float)oscale);                                                   \
+    } while (0)
+        if (in == NN_IN_FIELD) NN_C(NN_IN_FIELD, NN_EPI_HIDDEN, NN_RES_NONE);
+        else if (in == NN_IN_GRAD) NN_C(NN_IN_GRAD, NN_EPI_BWD, NN_RES_NONE);
+        else if (epi == NN_EPI_HIDDEN) NN_C(NN_IN_H, NN_EPI_HIDDEN, NN_RES_INPUT);
+        else if (epi == NN_EPI_OUT) NN_C(NN_IN_H, NN_EPI_OUT, NN_RES_NONE);
+        else NN_C(NN_IN_H, NN_EPI_BWD, NN_RES_TENSOR);
 #undef NN_C
     }
     static void wgrad(int in, int ga, int N, const void *hin, const void *fin, double inv_rho, double cval, const void *gz,
