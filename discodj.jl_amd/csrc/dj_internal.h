@@ -12,20 +12,6 @@ namespace dj {
 // FFT passes of one mesh size and precision (fft.hip)
 struct FftOps {
     void (*xf)(const void *mesh, bool fixed, void *A, const void *tw, double fscale, hipStream_t st);
-    // FP64: xf of the real field -(mub a) (neg) or mub (a + b) (b nullable), formed as the pass loads it
-    void (*xf_partner)(const double *mub, const double *a, const double *b, int neg, void *A, const void *tw,
-                       hipStream_t st);
-    // FP64, on the ext grid of the 2LPT source: the inverse z pass of A_ik formed from phi (F, n grid) as it
-    // is loaded, and the forward z pass of an A_ik cotangent whose output is added into Fb (n grid)
-    void (*zm_deriv_pad)(const void *F, void *Be, int n, double L, int i, int k, double s, const void *tw,
-                         hipStream_t st);
-    void (*zm_deriv_adj)(const void *Be, void *Fb, int n, double L, int i, int k, double sme, double s,
-                         const void *tw, hipStream_t st);
-    // FP64 IC spectra (mode: IC_PSI1 / IC_PSI2, and IC_DERIV / IC_PSI2_ADJ of ic_modes.h): the inverse z pass
-    // of the multiplied spectrum, and the forward z pass whose output is weighted, multiplied, accumulated
-    void (*zm_mult_inv)(int mode, const void *in, void *out, int c, double L, const void *tw, hipStream_t st);
-    void (*zm_fwd_mult_acc)(int mode, const void *in, void *acc, int c, double L, double s, const void *tw,
-                            hipStream_t st);
     void (*xi)(const void *A, void *mesh, const void *tw, hipStream_t st);
     // the same with the output multiplied by s as it is stored
     void (*xi_scaled)(const void *A, void *mesh, const void *tw, double s, hipStream_t st);
@@ -274,19 +260,21 @@ void ngenic_seed_table(uint32_t seed, int res, uint32_t *tab);
 // complex, element (i, j, k) at i + res (j + res k), into device memory d_field; returns a HIP error code
 int ngenic_field_device(uint32_t seed, int res, double *d_field, hipStream_t st);
 // Device buffers of the IC pipeline and its reverse for one (n, order), kept between calls (the 2LPT
-// transforms at 3n/2 need about 20 n^3 doubles: 5.3 GB at n = 256, 42 GB at n = 512); freed by
+// transforms at 3n/2 need about 26 n^3 doubles: 3.4 GB at n = 256, 27 GB at n = 512); freed by
 // ic_work_free or when a call needs another size
 struct IcWork {
     int n = 0, order = 0, ntab = 0;
     std::vector<void *> bufs;
     void *twn = nullptr, *twe = nullptr, *kt = nullptr, *pt = nullptr;
-    void *A = nullptr, *Bm = nullptr, *F = nullptr, *Fb = nullptr, *fLb = nullptr;
-    void *w = nullptr, *p1 = nullptr, *p2 = nullptr;
-    void *Ae = nullptr, *Be = nullptr, *mu = nullptr, *fld[3] = {nullptr, nullptr, nullptr};
-    // The nine second-order fields A_ik of the last forward (ext grid), kept for the reverse pass of the
-    // same ICs, and what they were computed from: n, L, order, the P(k) table, and the seed or (wkey) a
-    // copy of the white noise.  fk_room: 0 not tried, 1 allocated, -1 no room (the forward then uses fld).
-    void *fk[9] = {}, *wkey = nullptr, *flag = nullptr;
+    void *F = nullptr, *Fb = nullptr, *G = nullptr;  // phi(k), its cotangent, the source's fL(k) / k^2 (or its cotangent)
+    void *w = nullptr, *mu = nullptr;
+    // spectra between the passes (ic_fft.hip): lines along z; working sets after the y pass; the six second
+    // derivatives of phi.  W has buffers of its own where the device has room for them (fk_room 1), and A then holds
+    // the last forward's for the reverse pass of the same ICs; without (-1; 0 not tried) W is A, and every pass
+    // computes A again.
+    void *Z[3] = {}, *W[6] = {}, *A[6] = {};
+    // what A was computed from: n, L, order, the P(k) table, and the seed or (wkey) a copy of the white noise
+    void *wkey = nullptr, *flag = nullptr;
     int fk_room = 0;
     bool fk_valid = false, fk_seeded = false;
     int fk_n = 0, fk_order = 0;
@@ -295,6 +283,26 @@ struct IcWork {
     std::vector<double> fk_kt, fk_pt;
 };
 void ic_work_free(IcWork &ws);
+// The passes of the IC pipeline on the buffers of an IcWork, for one n (ic_fft.hip).  second: the de-aliased grid of
+// the second order (3 n / 2) is built
+struct IcPasses {
+    // F = phi(k) from Z[0], the white noise after its y pass (B layout)
+    void (*phi)(const IcWork &w, double L, int ntab, hipStream_t st);
+    // A from F: the spectra of the second derivatives; G from A: the 2LPT source mu's spectrum over k^2
+    void (*second)(const IcWork &w, double L, hipStream_t st);
+    void (*source)(const IcWork &w, double L, hipStream_t st);
+    // Psi = D psi1 + D^2 psi2, Pi = psi1 + 2 D psi2 from F and (two) G
+    void (*combine)(const IcWork &w, double L, double D, bool two, int prec, void *psi, void *pi, hipStream_t st);
+    // reverse: Fb and (two) G, the cotangents of F and of fL; mu = mubar; Fb += F's cotangent through A (A is
+    // overwritten where it is W); Z[0] = the white noise's cotangent before its inverse y pass
+    void (*combine_adj)(const IcWork &w, double L, double D, bool two, int prec, const void *psibar, const void *pibar,
+                        hipStream_t st);
+    void (*mu_adj)(const IcWork &w, double L, hipStream_t st);
+    void (*source_adj)(const IcWork &w, double L, hipStream_t st);
+    void (*phi_adj)(const IcWork &w, double L, int ntab, hipStream_t st);
+    bool has_second;
+};
+bool ic_passes(int n, IcPasses &ops);
 // White noise: `white` (n^3 real values, on the host, or on the device when white_on_device), or else
 // (NULL) the N-GenIC field of seed generated on the device.  The reverse writes the white-noise cotangent
 // to wbar (host, or device when wbar_on_device).  Both return a HIP error code.

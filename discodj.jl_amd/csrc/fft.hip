@@ -2,34 +2,9 @@
 #include <hip/hip_runtime.h>
 
 #include "dj_internal.h"
-#include "fft_passes.h"
-#include "ic_modes.h"
+#include "fft_shape.h"
 
 namespace dj {
-
-template <typename T, int N> struct FftShape {
-    // lines per workgroup: about 64 KiB of LDS for the y/z tiles, at most 16, dividing N
-    static constexpr int target = 65536 / (N * (int)sizeof(cx<T>));
-    static constexpr int B = (N % 16 == 0 && target >= 16) ? 16
-                           : (N % 8 == 0 && target >= 8) ? 8
-                           : (N % 4 == 0 && target >= 4) ? 4
-                           : (N % 2 == 0 && target >= 2) ? 2 : 1;
-    // x passes (half-length packed lines, about 32 KiB of LDS) run 256 threads; the y/z passes run
-    // 512 once a radix-16 pass has at least that many butterflies, so that the two workgroups their
-    // LDS tile allows per CU still hold 16 waves
-    static constexpr int NT = 256;
-    static constexpr int NTY = (B * N / 16 >= 512) ? 512 : 256;
-    using P = Passes<T, N, B, NT>;
-    using PY = Passes<T, N, B, NTY>;
-    // the N-entry twiddle table moves into LDS when two workgroups of the y/z tile plus table
-    // still fit a CU (160 KiB); otherwise the passes read it through the caches
-    static constexpr bool TWL = (PY::EF::LDS_ELEMS + N) * sizeof(cx<T>) <= 80 * 1024;
-    // the c2r x pass at 1024^3 (FP32): 16 lines per workgroup and 512 threads, so that its transposed
-    // loads read whole 128-byte lines of a block's own (1.99 against 2.12 ms with 8 lines and 256)
-    static constexpr int BXI = (sizeof(T) == 4 && N == 1024) ? 16 : B;
-    static constexpr int NTXI = BXI == B ? NT : 512;
-    using PXI = Passes<T, N, BXI, NTXI>;
-};
 
 // Shape of the persistent z pass (k_zm_pipe): 4 waves of one line-group each, 1024 points per wave
 // (4096 / N lines per workgroup), about 43 KiB of LDS with the twiddle table, three workgroups per CU
@@ -39,23 +14,6 @@ template <typename T, int N> struct ZPipeShape {
     using P = Passes<T, N, B, NT>;
     static constexpr int GROUPS_PER_CU = 3;
 };
-
-// The hardware hands workgroup b to XCD b % 8.  Logical block (b % 8) (nb / 8) + b / 8 puts runs of
-// consecutive logical blocks on one XCD, where they run close in time: neighbouring line groups
-// whose transposed loads and stores share 128-byte lines then meet in that XCD's L2 instead of
-// fetching each line twice from HBM.
-__device__ __forceinline__ int xcd_block(int b, int nb) { return (nb & 7) ? b : (b & 7) * (nb >> 3) + (b >> 3); }
-
-// the twiddle table for a workgroup: a copy in LDS, or the global table
-template <typename T, int N, bool TWL>
-__device__ __forceinline__ const cx<T> *stage_twiddles(const cx<T> *__restrict__ tw, cx<T> *twl, int tid, int nt) {
-    if constexpr (TWL) {
-        for (int i = tid; i < N; i += nt) twl[i] = tw[i];
-        return twl;  // the caller's barrier after the tile load covers this copy
-    } else {
-        return tw;
-    }
-}
 
 // Each kernel runs its line FFTs wave by wave (run_wave) when the engine's pass shapes allow it,
 // with workgroup barriers only around the twiddle table and the transposed (strided) side of a pass;
@@ -85,42 +43,6 @@ __global__ __launch_bounds__(256) void k_xf(const IN *__restrict__ mesh, cx<T> *
     }
     P::xf_store(lds, t, A, yb, z, threadIdx.x);
 }
-
-// The r2c x pass of a real field computed as it is loaded (src(g): the reals g, g + 1 as a complex)
-template <typename T, int N, typename SRC>
-__global__ __launch_bounds__(256) void k_xf_src(SRC src, cx<T> *__restrict__ A, const cx<T> *__restrict__ tw) {
-    using S = FftShape<T, N>;
-    using P = typename S::P;
-    __shared__ cx<T> lds[P::EX::LDS_ELEMS];
-    constexpr bool TWX = sizeof(T) == 4;
-    __shared__ cx<T> twl[TWX ? N : 1];
-    const cx<T> *t = stage_twiddles<T, N, TWX>(tw, twl, threadIdx.x, 256);
-    const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / S::B), z = lb / (N / S::B);
-    if constexpr (P::EX::wave_ok()) {
-        P::xf_load_src_w(src, lds, yb, z, threadIdx.x);
-        if constexpr (TWX) __syncthreads();
-        else P::EX::wave_sync();
-        P::EX::template run_wave<-1, 2>(lds, t, threadIdx.x);
-        __syncthreads();
-    } else {
-        P::xf_load_src(src, lds, yb, z, threadIdx.x);
-        __syncthreads();
-        P::EX::template run<-1, 2>(lds, t, threadIdx.x);
-    }
-    P::xf_store(lds, t, A, yb, z, threadIdx.x);
-}
-
-// The 2LPT source's partner product of the IC reverse pass, -(mubar a) (neg) or mubar (a + b) (b non-null),
-// as a source of k_xf_src: the values k_ic_partner writes, without the field in memory
-struct PartnerSrc {
-    const double *mub, *a, *b;
-    int neg;
-    __device__ double at(size_t i) const {
-        const double p = b ? a[i] + b[i] : a[i];
-        return neg ? -(mub[i] * p) : mub[i] * p;
-    }
-    __device__ cx<double> operator()(size_t g) const { return cx<double>{at(g), at(g + 1)}; }
-};
 
 // SC: the output multiplied by s as it is stored; MUL: the spectrum multiplied by tab[kx] as it is loaded
 template <typename T, int N, bool SC = false, bool MUL = false>
@@ -292,42 +214,30 @@ __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zm_ik(const cx<T> *in
     inverse_to(outz);
 }
 
-// The z pass (forward or inverse) of lines read from src(e) and written to dst(e, v), e the B-layout index:
-// the FP64 2LPT derivative spectra formed as the pass loads them, or their cotangents cropped and added
-// into the n-grid spectrum as it stores them
-template <typename T, int N, bool FWD, typename SRC, typename DST>
-__global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zm_io(SRC src, DST dst, const cx<T> *__restrict__ tw) {
+// The inverse z pass of lines multiplied by tab[kz] as they are loaded
+template <typename T, int N>
+__global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zi_mul(const cx<T> *__restrict__ in, cx<T> *__restrict__ out,
+                                                                 const cx<T> *__restrict__ tw,
+                                                                 const cx<T> *__restrict__ tab) {
     using S = FftShape<T, N>;
     using P = typename S::PY;
     __shared__ cx<T> lds[P::EF::LDS_ELEMS];
     __shared__ cx<T> twl[S::TWL ? N : 1];
     const int b = blockIdx.x;
     const cx<T> *t = stage_twiddles<T, N, S::TWL>(tw, twl, threadIdx.x, S::NTY);
+    const auto src = [&](size_t e) { return cmul(in[e], tab[(unsigned)(e % N)]); };
     if constexpr (P::EF::wave_ok()) {
         P::z_load_src_w(src, lds, b, threadIdx.x);
         __syncthreads();  // the twiddle table; from here on every wave works on its own lines
-        P::EF::template run_wave<FWD ? -1 : +1, 1>(lds, t, threadIdx.x);
-        P::z_store_dst_w(lds, dst, b, threadIdx.x);
+        P::EF::template run_wave<+1, 1>(lds, t, threadIdx.x);
+        P::z_store_w(lds, out, b, threadIdx.x);
     } else {
         P::z_load_src(src, lds, b, threadIdx.x);
         __syncthreads();
-        P::EF::template run<FWD ? -1 : +1, 1>(lds, t, threadIdx.x);
-        P::z_store_dst(lds, dst, b, threadIdx.x);
+        P::EF::template run<+1, 1>(lds, t, threadIdx.x);
+        P::z_store(lds, out, b, threadIdx.x);
     }
 }
-template <typename T> struct StoreTo {
-    cx<T> *out;
-    __device__ void operator()(size_t e, cx<T> v) const { out[e] = v; }
-};
-// the z lines of in multiplied by tab[kz] as they are loaded
-template <typename T, int N> struct LoadMul {
-    const cx<T> *in, *tab;
-    __device__ cx<T> operator()(size_t e) const { return cmul(in[e], tab[(unsigned)(e % N)]); }
-};
-template <typename T> struct LoadFrom {
-    const cx<T> *in;
-    __device__ cx<T> operator()(size_t e) const { return in[e]; }
-};
 
 // The z pass as a persistent kernel (three workgroups per CU, block b, b + G, b + 2G, ... for G
 // workgroups): each wave holds the next block's lines in registers while it transforms and stores
@@ -439,60 +349,13 @@ struct FftN {
         else
             k_xf<T, N, T><<<P::XBLOCKS(), 256, 0, st>>>((const T *)mesh, (cx<T> *)A, (const cx<T> *)tw, fscale);
     }
-    static void xf_partner(const double *mub, const double *a, const double *b, int neg, void *A, const void *tw,
-                           hipStream_t st) {
-        if constexpr (sizeof(T) == 8)
-            k_xf_src<T, N, PartnerSrc><<<P::XBLOCKS(), 256, 0, st>>>(PartnerSrc{mub, a, b, neg}, (cx<T> *)A,
-                                                                     (const cx<T> *)tw);
-    }
-    // inverse z pass of the A_ik spectrum (ext grid N) formed from phi (F, n grid) as it is loaded, into Be
-    static void zm_deriv_pad(const void *F, void *Be, int n, double L, int i, int k, double s, const void *tw,
-                             hipStream_t st) {
-        if constexpr (sizeof(T) == 8)
-            k_zm_io<T, N, false, DerivPadSrc<N>, StoreTo<T>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                DerivPadSrc<N>{(const cx<double> *)F, i, k, L, s}, StoreTo<T>{(cx<T> *)Be}, (const cx<T> *)tw);
-    }
-    // forward z pass of Be (ext grid N) whose output is cropped, multiplied and added into Fb (n grid)
-    static void zm_deriv_adj(const void *Be, void *Fb, int n, double L, int i, int k, double sme, double s,
-                             const void *tw, hipStream_t st) {
-        if constexpr (sizeof(T) == 8)
-            k_zm_io<T, N, true, LoadFrom<T>, DerivAdjDst<N>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                LoadFrom<T>{(const cx<T> *)Be}, DerivAdjDst<N>{(cx<double> *)Fb, i, k, L, sme, s}, (const cx<T> *)tw);
-    }
-    // FP64 IC spectra on this grid: the inverse z pass of mult<mode>(in) into out, and the forward z pass of
-    // in whose output is weighted (s), multiplied by mult<mode> and added into acc
-    static void zm_mult_inv(int mode, const void *in, void *out, int c, double L, const void *tw, hipStream_t st) {
-        if constexpr (sizeof(T) == 8) {
-            const cx<T> *i = (const cx<T> *)in, *t = (const cx<T> *)tw;
-            StoreTo<T> o{(cx<T> *)out};
-            if (mode == IC_PSI1)
-                k_zm_io<T, N, false, MultSrc<IC_PSI1, N>, StoreTo<T>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                    MultSrc<IC_PSI1, N>{i, c, L}, o, t);
-            else
-                k_zm_io<T, N, false, MultSrc<IC_PSI2, N>, StoreTo<T>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                    MultSrc<IC_PSI2, N>{i, c, L}, o, t);
-        }
-    }
-    static void zm_fwd_mult_acc(int mode, const void *in, void *acc, int c, double L, double s, const void *tw,
-                                hipStream_t st) {
-        if constexpr (sizeof(T) == 8) {
-            const cx<T> *t = (const cx<T> *)tw;
-            LoadFrom<T> i{(const cx<T> *)in};
-            if (mode == IC_DERIV)
-                k_zm_io<T, N, true, LoadFrom<T>, MultAccDst<IC_DERIV, N>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                    i, MultAccDst<IC_DERIV, N>{(cx<T> *)acc, c, L, s}, t);
-            else
-                k_zm_io<T, N, true, LoadFrom<T>, MultAccDst<IC_PSI2_ADJ, N>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-                    i, MultAccDst<IC_PSI2_ADJ, N>{(cx<T> *)acc, c, L, s}, t);
-        }
-    }
     static void zm_ik(const void *in, void *out, void *outz, const void *tw, const void *Kp, hipStream_t st) {
         k_zm_ik<T, N><<<P::ZBLOCKS(), S::NTY, 0, st>>>((const cx<T> *)in, (cx<T> *)out, (cx<T> *)outz, (const cx<T> *)tw,
                                                        *(const KMult<T> *)Kp);
     }
     static void zi_mul(const void *in, void *out, const void *tw, const void *tab, hipStream_t st) {
-        k_zm_io<T, N, false, LoadMul<T, N>, StoreTo<T>><<<P::ZBLOCKS(), S::NTY, 0, st>>>(
-            LoadMul<T, N>{(const cx<T> *)in, (const cx<T> *)tab}, StoreTo<T>{(cx<T> *)out}, (const cx<T> *)tw);
+        k_zi_mul<T, N><<<P::ZBLOCKS(), S::NTY, 0, st>>>((const cx<T> *)in, (cx<T> *)out, (const cx<T> *)tw,
+                                                        (const cx<T> *)tab);
     }
     static void yi_mul(const void *Bm, void *A, const void *tw, const void *tab, hipStream_t st) {
         k_yi<T, N, true><<<P::YBLOCKS(), S::NTY, 0, st>>>((const cx<T> *)Bm, (cx<T> *)A, (const cx<T> *)tw,
@@ -555,11 +418,6 @@ bool fft_dispatch(int N, FftOps &ops) {
         ops.yi_mul = FftN<T, n>::yi_mul; \
         ops.zi_mul = FftN<T, n>::zi_mul; \
         ops.zm_ik = FftN<T, n>::zm_ik; \
-        ops.xf_partner = FftN<T, n>::xf_partner; \
-        ops.zm_deriv_pad = FftN<T, n>::zm_deriv_pad; \
-        ops.zm_deriv_adj = FftN<T, n>::zm_deriv_adj; \
-        ops.zm_mult_inv = FftN<T, n>::zm_mult_inv; \
-        ops.zm_fwd_mult_acc = FftN<T, n>::zm_fwd_mult_acc; \
         ops.yf = FftN<T, n>::yf;        \
         ops.yi = FftN<T, n>::yi;        \
         ops.zm = FftN<T, n>::zm;        \

@@ -131,35 +131,6 @@ struct Passes {
                 lds[EX::idx(l, m)] = v;
             });
     }
-    // the same loads from a computed real field: src(g) returns the pair of reals (g, g + 1) as a complex
-    template <typename SRC>
-    DJ_HD static void xf_load_src(const SRC &src, cx<T> *lds, int yb, int z, int tid) {
-        const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
-        copy_batched<cx<T>, B * NC, NT>(
-            tid,
-            [&](int i) {
-                const int l = i / NC, m = i - l * NC;
-                return src(base + (size_t)N * l + 2 * m);
-            },
-            [&](int i, cx<T> v) {
-                const int l = i / NC, m = i - l * NC;
-                lds[EX::idx(l, m)] = v;
-            });
-    }
-    template <typename SRC>
-    DJ_HD static void xf_load_src_w(const SRC &src, cx<T> *lds, int yb, int z, int tid) {
-        const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
-        copy_wave<cx<T>, EX::LW * NC>(
-            tid >> 6, tid & 63,
-            [&](int i) {
-                const int l = i / NC, m = i - l * NC;
-                return src(base + (size_t)N * l + 2 * m);
-            },
-            [&](int i, cx<T> v) {
-                const int l = i / NC, m = i - l * NC;
-                lds[EX::idx(l, m)] = v;
-            });
-    }
     // X[k] = E[k] + W_N^k O[k], E = (Z[k] + conj Z[NC-k]) / 2, O = (Z[k] - conj Z[NC-k]) / 2i
     DJ_HD static void xf_store(const cx<T> *lds, const cx<T> *twN, cx<T> *A, int yb, int z, int tid) {
         copy_batched<cx<T>, B * H, NT>(
@@ -315,7 +286,7 @@ struct Passes {
             if ((B * N) % NT == 0 || i < B * N) z_mult_one<MODE>(lds, K, b, i);
         }
     }
-    // the z lines of block b from / to functors of the B-layout entry index (src(e), dst(e, v))
+    // the z lines of block b from a functor of the B-layout entry index (src(e))
     template <typename SRC>
     DJ_HD static void z_load_src(const SRC &src, cx<T> *lds, int b, int tid) {
         const size_t base = (size_t)N * B * b;
@@ -323,26 +294,12 @@ struct Passes {
             tid, [&](int i) { return src(base + i); },
             [&](int i, cx<T> v) { const int l = i / N, zz = i - l * N; lds[EF::idx(l, zz)] = v; });
     }
-    template <typename DST>
-    DJ_HD static void z_store_dst(const cx<T> *lds, const DST &dst, int b, int tid) {
-        const size_t base = (size_t)N * B * b;
-        copy_batched<cx<T>, B * N, NT>(
-            tid, [&](int i) { const int l = i / N, zz = i - l * N; return lds[EF::idx(l, zz)]; },
-            [&](int i, cx<T> v) { dst(base + i, v); });
-    }
     template <typename SRC>
     DJ_HD static void z_load_src_w(const SRC &src, cx<T> *lds, int b, int tid) {
         const size_t base = (size_t)N * B * b;
         copy_wave<cx<T>, EF::LW * N>(
             tid >> 6, tid & 63, [&](int i) { return src(base + i); },
             [&](int i, cx<T> v) { const int l = i / N, zz = i - l * N; lds[EF::idx(l, zz)] = v; });
-    }
-    template <typename DST>
-    DJ_HD static void z_store_dst_w(const cx<T> *lds, const DST &dst, int b, int tid) {
-        const size_t base = (size_t)N * B * b;
-        copy_wave<cx<T>, EF::LW * N>(
-            tid >> 6, tid & 63, [&](int i) { const int l = i / N, zz = i - l * N; return lds[EF::idx(l, zz)]; },
-            [&](int i, cx<T> v) { dst(base + i, v); });
     }
     DJ_HD static void z_store(const cx<T> *lds, cx<T> *Bm, int b, int tid) {
         cx<T> *dst = Bm + (size_t)N * B * b;

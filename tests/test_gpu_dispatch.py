@@ -153,3 +153,35 @@ def test_spectral_force_over_tiles(W, res, n, aa, prec):
     # cell each), the meshes and the transforms
     ref = O.pm_acceleration(psi, O.pm_config(res, n, L, worder=W, grad_order=0, antialias=aa), "solver")
     assert G.rel(acc, ref) < (2e-5 if prec == 32 else 1e-12)
+
+
+@pytest.mark.parametrize("n, order, prec", [(16, 2, 32), (24, 1, 64), (48, 1, 32), (96, 1, 64), (128, 2, 64), (192, 1, 64)])
+def test_ics_over_the_transform_sizes(n, order, prec):
+    """Displacements and momenta of the ICs at sizes whose line groups differ (1e-12, or FP32's rounding of the
+    results), and the reverse pass as their transpose: a central difference along one direction is exact up to
+    rounding, the ICs being quadratic in the noise."""
+    L, a, eps = 2.0 * n, 0.05, 1e-3
+    rng = np.random.default_rng(n)
+    white, v = rng.normal(size=(n, n, n)), rng.normal(size=(n, n, n))
+    pb, mb = rng.normal(size=(3, n, n, n)), rng.normal(size=(3, n, n, n))
+    oc = O.Cosmology(0.2621, 0.049, 0.6766, 0.8102, 0.9665)
+    k, pk = O.linear_power_spectrum(oc)
+    psi1, psi2 = O.compute_core2(O.white_noise_to_fphi(O.ic_operator(n, L, k, pk), white), L)
+    psi_ref, pi_ref = O.nbody_ics_lpt2(oc, psi1, psi2 if order == 2 else np.zeros_like(psi2), a)
+    Dg = oc.Dplus(a)
+    with D.PMSolverHIP(D.PMConfig(res_pm=max(n, 32), n_part=n, boxsize=L), precision=prec) as S:
+        S.ics_lpt(k, pk, Dg, order=order, white=white)
+        psi, pi = S.get_state()
+        tol = 1e-12 if prec == 64 else 2e-7
+        assert G.rel(psi, psi_ref) < tol and G.rel(pi, pi_ref) < tol
+        if prec == 32:
+            return
+        f = []
+        for e in (eps, -eps):
+            S.ics_lpt(k, pk, Dg, order=order, white=white + e * v)
+            p, m = S.get_state()
+            f.append(float(np.vdot(pb, p) + np.vdot(mb, m)))
+        wb = S.vjp_ics_lpt(k, pk, Dg, pb, mb, order=order, white=white)
+    # the sum's own scale: its two dot products' norms times the direction's
+    scale = np.linalg.norm(wb) * np.linalg.norm(v)
+    assert abs(float(np.vdot(wb, v)) - (f[0] - f[1]) / (2 * eps)) < 1e-9 * scale
