@@ -134,13 +134,37 @@ template <int DIR, typename T> DJ_HD void dft16(cx<T> *a) {
     }
 }
 
+// 3 Q, Q a power of two, without inner twiddles (the prime-factor map: n = 3 n1 + Q n2, k = 3 u k1 + Q v k2 mod 3 Q
+// with 3 u = 1 mod Q and Q v = 1 mod 3)
+template <int Q, int DIR, typename T> DJ_HD void dft_3q(cx<T> *a);
+
 template <int R, int DIR, typename T> DJ_HD void dft(cx<T> *a) {
     if constexpr (R == 2) dft2<DIR>(a);
     else if constexpr (R == 3) dft3<DIR>(a);
     else if constexpr (R == 4) dft4<DIR>(a);
     else if constexpr (R == 8) dft8<DIR>(a);
     else if constexpr (R == 16) dft16<DIR>(a);
+    else if constexpr (R % 3 == 0) dft_3q<R / 3, DIR>(a);
     else static_assert(R == 2, "unsupported radix");
+}
+
+template <int Q, int DIR, typename T> DJ_HD void dft_3q(cx<T> *a) {
+    constexpr int N = 3 * Q, u = Q % 3 == 2 ? (Q + 1) / 3 : (2 * Q + 1) / 3, v = Q % 3;
+    static_assert((3 * u) % Q == 1 % Q && (Q * v) % 3 == 1, "3 and Q are coprime");
+    cx<T> y[3][Q];
+#pragma unroll
+    for (int n1 = 0; n1 < Q; n1++) {
+        cx<T> t[3] = {a[3 * n1], a[(3 * n1 + Q) % N], a[(3 * n1 + 2 * Q) % N]};
+        dft3<DIR>(t);
+#pragma unroll
+        for (int k2 = 0; k2 < 3; k2++) y[k2][n1] = t[k2];
+    }
+#pragma unroll
+    for (int k2 = 0; k2 < 3; k2++) {
+        dft<Q, DIR>(y[k2]);
+#pragma unroll
+        for (int k1 = 0; k1 < Q; k1++) a[(3 * u * k1 + Q * v * k2) % N] = y[k2][k1];
+    }
 }
 
 }  // namespace dj

@@ -7,12 +7,13 @@
 namespace dj {
 
 // Shape of the persistent z pass (k_zm_pipe): 4 waves of one line-group each, 1024 points per wave
-// (4096 / N lines per workgroup), about 43 KiB of LDS with the twiddle table, three workgroups per CU
+// (4096 / N lines per workgroup), about 43 KiB of LDS with the twiddle table, three workgroups per CU;
+// 384: four lines per wave, which its passes need (wave_ok), two workgroups
 template <typename T, int N> struct ZPipeShape {
-    static constexpr bool ok = sizeof(T) == 4 && (N == 256 || N == 512 || N == 1024);
-    static constexpr int B = ok ? 4096 / N : 1, NT = 256;
+    static constexpr bool ok = sizeof(T) == 4 && (N == 256 || N == 384 || N == 512 || N == 1024);
+    static constexpr int B = !ok ? 1 : N == 384 ? 16 : 4096 / N, NT = 256;
     using P = Passes<T, N, B, NT>;
-    static constexpr int GROUPS_PER_CU = 3;
+    static constexpr int GROUPS_PER_CU = N == 384 ? 2 : 3;
 };
 
 // Each kernel runs its line FFTs wave by wave (run_wave) when the engine's pass shapes allow it,
@@ -246,7 +247,8 @@ __global__ __launch_bounds__((FftShape<T, N>::NTY)) void k_zi_mul(const cx<T> *_
 // are the same for every block and are read once; the per-line ones (kx, ky) are read before the
 // next block's loads are issued, so that waiting for them does not wait for those loads.  The
 // arithmetic of the multiplier is KMult::kphi's, in its order.  FP32 on 256^3 to 1024^3 meshes (a
-// lane's elements keep one kz per step), the potential multiplier without window deconvolution or
+// lane's elements keep one kz per step; 384^3: 179 -> 100 us; in FP64 the held lines take the registers of a
+// wave's transforms: 192^3 37 -> 46 us, 512^3 613 -> 657), the potential multiplier without window deconvolution or
 // transfer function.
 template <typename T, int N, int MODE, bool FWD, bool INV>
 __global__ __launch_bounds__((ZPipeShape<T, N>::NT), (ZPipeShape<T, N>::GROUPS_PER_CU)) void k_zm_pipe(

@@ -1,6 +1,6 @@
 // Batched line FFT over an LDS tile: B lines of N complex points, NT threads.
 //
-// Stockham autosort passes (radix 16/8/4/2, then 3): every pass reads each thread's butterfly
+// Stockham autosort passes (radix 16/8/4/2, then 3 times a power of two): every pass reads each thread's butterfly
 // inputs from LDS into registers, synchronises, applies twiddles and the in-register DFT, and
 // writes the outputs back in place, so one LDS tile serves all passes and the result is in natural
 // order.  Element e of line l lives at l*LS + e + (e >> PS): one pad slot per 2^PS elements breaks
@@ -14,7 +14,8 @@
 // and every pass maps that wave's butterflies onto its own 64 lanes, so the phases only need the
 // wave's own ordering (LDS operations of one wave execute in issue order) and no workgroup barrier;
 // waves of a workgroup then run their lines independently.  It applies when every pass has a
-// multiple of 64 butterflies per wave (wave_ok()).
+// multiple of 64 butterflies per wave (wave_ok()), in FP32 also when three quarters of a pass's lanes
+// have one (384^3: y passes 91 -> 87 us; the FP64 x pass at 192^3 loses, 25 -> 29).
 #pragma once
 
 #include "dj_complex.h"
@@ -26,16 +27,26 @@ struct RadixPlan {
     int r[10];
 };
 
-// largest radices first; factors of 3 last
+// Largest radices first.  A length 3 2^a from 96 to 384 ends in one radix 12 or 24: a pass of its own for the 3 moves
+// the whole tile through LDS and twiddles it once more (FP32 192^3: forward and inverse z 26 -> 21 us; FP64 384^3: 373 ->
+// 323).  24 and 48 keep the 3, whose pass has more butterflies for the threads (48^3: 3.6 against 4.0 us); 768 takes
+// three passes either way.
 constexpr RadixPlan make_plan(int N) {
     RadixPlan p{0, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
     int m = N, threes = 0;
     while (m % 3 == 0) { threes++; m /= 3; }
+    int last = 3;
+    if (threes == 1 && m >= 32 && m <= 128) {
+        const int q = m == 128 ? 8 : 4;
+        last = 3 * q;
+        m /= q;
+    }
     while (m % 16 == 0 && m > 0) { p.r[p.n++] = 16; m /= 16; }
     if (m == 8) { p.r[p.n++] = 8; m = 1; }
     if (m == 4) { p.r[p.n++] = 4; m = 1; }
     if (m == 2) { p.r[p.n++] = 2; m = 1; }
-    for (int i = 0; i < threes; i++) p.r[p.n++] = 3;
+    if (threes == 1) p.r[p.n++] = last;
+    else for (int i = 0; i < threes; i++) p.r[p.n++] = 3;
     if (m != 1) p.n = -1;  // unsupported length
     return p;
 }
@@ -114,13 +125,15 @@ struct LineFFT {
         static constexpr int R = P.r[p];
         static constexpr int S = plan_stride(P, p);
         static constexpr int M = N / R;
-        static constexpr int CW = LW * M / 64;  // butterflies per lane
+        static constexpr int NBW = LW * M;              // the wave's butterflies
+        static constexpr int CW = (NBW + 63) / 64;     // per lane, the last round's up to NBW
         static constexpr int STEP = N / (S * R);
 
         DJ_HD static void load(const cx<T> *lds, cx<T> (&reg)[CW][R], int wave, int lane) {
 #pragma unroll
             for (int c = 0; c < CW; c++) {
                 const int u = lane + 64 * c, l = wave * LW + u / M, j = u % M;
+                if (!(NBW % 64 == 0 || u < NBW)) continue;
 #pragma unroll
                 for (int r = 0; r < R; r++) reg[c][r] = lds[idx(l, j + r * M)];
             }
@@ -131,6 +144,7 @@ struct LineFFT {
 #pragma unroll
             for (int c = 0; c < CW; c++) {
                 const int u = lane + 64 * c, l = wave * LW + u / M, j = u % M;
+                if (!(NBW % 64 == 0 || u < NBW)) continue;
                 const int k = j % S;
                 if (S > 1 && k != 0) {
 #pragma unroll
@@ -146,8 +160,10 @@ struct LineFFT {
 
     template <int p = 0>
     static constexpr bool wave_ok() {
-        if constexpr (p >= P.n) return LW > 0;
-        else return LW > 0 && (LW * (N / P.r[p])) % 64 == 0 && wave_ok<p + 1>();
+        if constexpr (p >= P.n || LW == 0) return LW > 0;
+        else
+            return (sizeof(T) == 4 ? 4 * WPass<p>::NBW >= 3 * 64 * WPass<p>::CW : WPass<p>::NBW % 64 == 0) &&
+                   wave_ok<p + 1>();
     }
 
 #if defined(__HIPCC__)

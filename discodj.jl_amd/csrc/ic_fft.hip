@@ -284,7 +284,7 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 4) void k_ic_xf(SRC src,
 // rows are its own): inverse x of the three (s times their transforms), mubar (A_jj + A_kk) each (DIAG: in =
 // A11, A22, A33) or -2 mubar A_ik (in = A12, A13, A23), forward x
 template <int N, int HX, bool DIAG>
-__global__ __launch_bounds__((FftShape<double, N>::NT), 3) void k_ic_x_adj(IcIn in, IcOut out, double s,
+__global__ __launch_bounds__((FftShape<double, N>::NT), DIAG ? 2 : 3) void k_ic_x_adj(IcIn in, IcOut out, double s,
                                                                           const double *__restrict__ mub,
                                                                           const cd *__restrict__ tw, double dk) {
     using S = FftShape<double, N>;

@@ -15,10 +15,10 @@ def _psi(n, scale, seed, dt):
 
 
 @pytest.mark.parametrize("res, n, prec", [(16, 7, 32), (64, 33, 32), (96, 50, 32), (128, 40, 32), (192, 64, 32),
-                                          (256, 65, 32), (64, 33, 64)])
+                                          (256, 65, 32), (64, 33, 64), (192, 40, 64), (384, 48, 32)])
 def test_step_over_the_gather_segment_rule(res, n, prec):
     """One pass, kicked in particle order, on meshes of 8 (tiles shared by workgroups) to 4096 tiles (segments
-    of several tiles): Psi and Pi after a step against the oracle's force at the drifted positions.  The
+    of several tiles), and transforms of every plan: Psi and Pi after a step against the oracle's force at the drifted positions.  The
     bounds are the force's (2e-5 FP32, 1e-12 FP64); beta makes the kick the momentum's own size."""
     L = 2.0 * res
     dt = np.float32 if prec == 32 else np.float64
