@@ -439,6 +439,33 @@ __device__ __forceinline__ void dep_add(Acc *a, T wx, T wy, T wz, T wyz, double 
     }
 }
 
+// Accumulators set to zero, 16 bytes a thread and turn (a tile holds a multiple of 64 of them)
+template <typename Acc> __device__ __forceinline__ void zero_acc(Acc *acc, int cells) {
+    uint4 *q = (uint4 *)acc;
+    for (int c = threadIdx.x; c < cells * (int)sizeof(Acc) / 16; c += blockDim.x) q[c] = uint4{0, 0, 0, 0};
+}
+
+// The tile's cells to the mesh, 16 bytes a thread and turn: a cell a turn spent more instructions on a tile of 512
+// particles than their entries did (TSC at 1024^3: 2.23 ms a pass, 2.05 so).  cell(i): the value of accumulator i
+template <typename O, typename F>
+__device__ __forceinline__ void store_tile(O *mesh, const TileGeom &g, const int (&o3)[3], int pad, int sxd, const F &cell) {
+    constexpr int V = 16 / (int)sizeof(O), LV = V == 4 ? 2 : 1;
+    struct alignas(16) Vec {
+        O v[V];
+    };
+    const int lgx = g.lT[0] - LV, gx = (threadIdx.x & ((1 << lgx) - 1)) * V;
+    const unsigned N = (unsigned)g.N;
+    for (int r = threadIdx.x >> lgx; r < g.TY * g.TZ; r += blockDim.x >> lgx) {
+        const unsigned ly = r & (g.TY - 1), lz = r >> g.lT[1];
+        const unsigned gi = (o3[0] + gx) + N * ((o3[1] + ly) + N * (o3[2] + lz));  // cell indices < N^3 <= 2^30
+        const int li = gx + pad + sxd * r;
+        Vec o;
+#pragma unroll
+        for (int k = 0; k < V; k++) o.v[k] = cell(li + k);
+        *(Vec *)(mesh + gi) = o;
+    }
+}
+
 // Padded accumulator (PAD, every axis of the mesh holds at least two tiles): rows of SXD = TX + 2 (W-1)
 // cells, the tile's x cells at [W-1, W-1+TX), for the TY TZ rows of the tile.  An entry's stencil starts at local x cell l0 in
 // [-(W-1), TX) whenever it overlaps the tile, so its W x cells are always in the row (cells outside
@@ -459,7 +486,7 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
     constexpr int P = W - 1;
     const int t = blockIdx.x, TV = g.TX * g.TY * g.TZ;
     const int SXD = PAD ? g.TX + 2 * P : g.TX, ROWS = g.TY * g.TZ, CELLS = PAD ? SXD * ROWS : TV;
-    for (int c = threadIdx.x; c < CELLS; c += blockDim.x) acc[c] = 0;
+    zero_acc(acc, CELLS);
     const int tx = t % g.ntx, ty = (t / g.ntx) % g.nty, tz = t / (g.ntx * g.nty);
     const int ox = tx << g.lT[0], oy = ty << g.lT[1], oz = tz << g.lT[2];
     __syncthreads();
@@ -549,15 +576,14 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
         }
     }
     __syncthreads();
-    // one x row of the tile per TX threads (the block size is a multiple of TX); cell indices < N^3 <= 2^30
-    const unsigned N = (unsigned)g.N, lx = threadIdx.x & (g.TX - 1);
-    for (int r = threadIdx.x >> g.lT[0]; r < ROWS; r += blockDim.x >> g.lT[0]) {
-        const unsigned ly = r & (g.TY - 1), lz = r >> g.lT[1];
-        const unsigned gi = (ox + lx) + N * ((oy + ly) + N * (oz + lz));
-        const Acc v = acc[(PAD ? lx + P : lx) + SXD * r];
-        if constexpr (ACC == ACC_Q31) ((T *)mesh)[gi] = (T)((double)v * 0x1p-31);
-        else if constexpr (ACC == ACC_Q32) ((T *)mesh)[gi] = (T)ldexp((double)v, -qbits);
-        else ((Acc *)mesh)[gi] = v;
+    const int pad = PAD ? P : 0;
+    if constexpr (ACC == ACC_Q31) {
+        store_tile((T *)mesh, g, o3, pad, SXD, [&](int i) { return (T)((double)acc[i] * 0x1p-31); });
+    } else if constexpr (ACC == ACC_Q32) {
+        const T inv = (T)ldexpf(1.0f, -qbits);  // the cell's sum rounds once, in its conversion
+        store_tile((T *)mesh, g, o3, pad, SXD, [&](int i) { return (T)acc[i] * inv; });
+    } else {
+        store_tile((Acc *)mesh, g, o3, pad, SXD, [&](int i) { return acc[i]; });
     }
 }
 
@@ -659,7 +685,8 @@ __global__ __launch_bounds__(512) void k_tile_deposit3(const Entry<T> *__restric
 // integer (|term| <= 2^30, so the sum of up to 2^33 terms fits in 64 bits) and summed by 64-bit LDS integer
 // atomics, which run several times faster than float ones; the store divides by s_c.  The sum is
 // independent of the order of the additions; each term carries its float product's rounding plus at most
-// 2^-31 max_c.  Block (tile, component): one 64-bit accumulator per padded cell (the layout above).
+// 2^-31 max_c.  Block (tile, component): one 64-bit accumulator per padded cell (the layout above); a block for all
+// three components shares an entry's weights but leaves one block to a CU (256^3, CIC: 376 against 350 us).
 __global__ __launch_bounds__(256) void k_absmax3(const float *__restrict__ vals, size_t np, float vscale,
                                                  unsigned *__restrict__ mx) {
     __shared__ float red[3][256];
@@ -703,7 +730,7 @@ __global__ __launch_bounds__(512) void k_tile_deposit3q(const Entry<float> *__re
     const int t = blockIdx.x, comp = blockIdx.y;
     const int SXD = g.TX + 2 * P, ROWS = g.TY * g.TZ, CELLS = SXD * ROWS;
     const int SZ = SXD * g.TY, END = SXD * ROWS;
-    for (int c = threadIdx.x; c < CELLS; c += blockDim.x) acc[c] = 0ull;
+    zero_acc(acc, CELLS);
     const int tx = t % g.ntx, ty = (t / g.ntx) % g.nty, tz = t / (g.ntx * g.nty);
     const int o3[3] = {tx << g.lT[0], ty << g.lT[1], tz << g.lT[2]};
     const float s = fx_scale(mx[comp]);
@@ -753,15 +780,9 @@ __global__ __launch_bounds__(512) void k_tile_deposit3q(const Entry<float> *__re
             }
     }
     __syncthreads();
-    const unsigned N = (unsigned)g.N, lx = threadIdx.x & (g.TX - 1);
-    const size_t M = (size_t)N * N * N;
+    const size_t M = (size_t)g.N * g.N * g.N;
     const double inv = s > 0.f ? 1.0 / (double)s : 0.0;
-    float *oc = out + (size_t)comp * M;
-    for (int r = threadIdx.x >> g.lT[0]; r < ROWS; r += blockDim.x >> g.lT[0]) {
-        const unsigned ly = r & (g.TY - 1), lz = r >> g.lT[1];
-        const unsigned gi = (o3[0] + lx) + N * ((o3[1] + ly) + N * (o3[2] + lz));
-        oc[gi] = (float)((double)(long long)acc[(int)lx + P + SXD * r] * inv);
-    }
+    store_tile(out + (size_t)comp * M, g, o3, P, SXD, [&](int i) { return (float)((double)(long long)acc[i] * inv); });
 }
 
 // ------------------------------------------------------------------------------------ gather
