@@ -265,7 +265,7 @@ int ngenic_field_device(uint32_t seed, int res, double *d_field, hipStream_t st)
 struct IcWork {
     int n = 0, order = 0, ntab = 0;
     std::vector<void *> bufs;
-    void *twn = nullptr, *twe = nullptr, *kt = nullptr, *pt = nullptr;
+    void *twn = nullptr, *twe = nullptr, *kt = nullptr, *pt = nullptr, *amp = nullptr;
     void *F = nullptr, *Fb = nullptr, *G = nullptr;  // phi(k), its cotangent, the source's fL(k) / k^2 (or its cotangent)
     void *w = nullptr, *mu = nullptr;
     // spectra between the passes (ic_fft.hip): lines along z; working sets after the y pass; the six second
@@ -287,7 +287,7 @@ void ic_work_free(IcWork &ws);
 // the second order (3 n / 2) is built
 struct IcPasses {
     // F = phi(k) from Z[0], the white noise after its y pass (B layout)
-    void (*phi)(const IcWork &w, double L, int ntab, hipStream_t st);
+    void (*phi)(const IcWork &w, double L, hipStream_t st);
     // A from F: the spectra of the second derivatives; G from A: the 2LPT source mu's spectrum over k^2
     void (*second)(const IcWork &w, double L, hipStream_t st);
     void (*source)(const IcWork &w, double L, hipStream_t st);
@@ -299,7 +299,7 @@ struct IcPasses {
                         hipStream_t st);
     void (*mu_adj)(const IcWork &w, double L, hipStream_t st);
     void (*source_adj)(const IcWork &w, double L, hipStream_t st);
-    void (*phi_adj)(const IcWork &w, double L, int ntab, hipStream_t st);
+    void (*phi_adj)(const IcWork &w, double L, hipStream_t st);
     bool has_second;
 };
 bool ic_passes(int n, IcPasses &ops);

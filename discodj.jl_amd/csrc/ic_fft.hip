@@ -7,7 +7,7 @@
 // and the fields share their passes: for the A_ik one z pass writes three spectra (k_z^0, k_z^1, k_z^2), their
 // y passes write six, and one x pass forms the source mu from the six real lines that its workgroup holds
 // (all ICs at n = 256: 8.2 ms with nine stored fields of three passes each over the whole padded spectrum,
-// 3.9 so).  The reverse runs the same tree backwards, each pass adding the spectra that the forward split.
+// 3.4 so).  The reverse runs the same tree backwards, each pass adding the spectra that the forward split.
 //
 // A pad has non-zero modes only for |k| < n/2: the spectra between the passes are stored without the rest.
 //   line spectra  S[z + N line], line = kx + HX ky': HX = n/2 (pad) or n/2 + 1, ky' the n grid's index
@@ -38,7 +38,8 @@ __device__ __forceinline__ int second_power(int f) { return f == 0 ? 2 : f == 3 
 // The thread's index, opaque to the compiler: what a round of a kernel's loop derives from it (indexes, twiddles) is
 // computed in that round.  Taken out of the loop as invariant it costs up to 150 registers, and with them all but
 // one workgroup of a CU (the x pass of mu at n = 256, then with the fields
-// stored: 2.4 ms against 1.6).
+// stored: 2.4 ms against 1.6).  The x kernels keep the twiddles in LDS: through the caches, four twiddle loads to one of
+// data, that pass took 1.15 ms, 1.01 so, and the x passes of its reverse 2.3, 1.75.
 __device__ __forceinline__ int round_tid() {
     int t = threadIdx.x;
     asm volatile("" : "+v"(t));
@@ -176,10 +177,13 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 4) void k_ic_xi(const cd
     using EX = typename S::P::EX;
     constexpr int B = S::B, NC = N / 2, TOTAL = B * NC;
     __shared__ cd lds[EX::LDS_ELEMS];
+    __shared__ cd twl[N];
+    const cd *t = stage_twiddles<double, N, true>(tw, twl, threadIdx.x, S::NT);
+    __syncthreads();
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / B), z = lb / (N / B);
     const int tid = threadIdx.x;
-    x_load<N, HX>(in, lds, tw, yb, z, r, dk, tid);
-    x_lines<N, +1>(lds, tw, tid);
+    x_load<N, HX>(in, lds, t, yb, z, r, dk, tid);
+    x_lines<N, +1>(lds, t, tid);
     const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
     for (int i = threadIdx.x; i < TOTAL; i += S::NT) {
         const cd v = lds[EX::idx(i / NC, i % NC)];
@@ -189,7 +193,7 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 4) void k_ic_xi(const cd
 
 // Inverse x pass of the six spectra of A11, A22, A33, A12, A13, A23 (k_x powers 2, 0, 0, 1, 1, 0; each field s times
 // its transform) and the 2LPT source from them, mu = (A11 A22 + A11 A33 + A22 A33 - A12^2 - A13^2 - A23^2) smu.
-// The fields are not stored (1.6 ms with, 1.3 without, at n = 256): the reverse forms them again from the kept spectra,
+// The fields are not stored (at n = 256 that took 0.35 ms): the reverse forms them again from the kept spectra,
 // which it reads in less time than the fields, in the pass that needs them.
 template <int N, int HX>
 __global__ __launch_bounds__((FftShape<double, N>::NT), 3) void k_ic_xi_mu(IcIn in, double s, double smu,
@@ -199,26 +203,29 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 3) void k_ic_xi_mu(IcIn 
     using EX = typename S::P::EX;
     constexpr int B = S::B, NC = N / 2, TOTAL = B * NC, CNT = (TOTAL + S::NT - 1) / S::NT;
     __shared__ cd lds[EX::LDS_ELEMS];
+    __shared__ cd twl[N];
+    const cd *t = stage_twiddles<double, N, true>(tw, twl, threadIdx.x, S::NT);
+    __syncthreads();
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / B), z = lb / (N / B);
     const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
-    // one field's code six times over (unrolled it takes twice the registers): t = A11, A11 + A22 meets the next
+    // one field's code six times over (unrolled it takes twice the registers): g = A11, A11 + A22 meets the next
     // diagonal field in m
-    cd t[CNT], m[CNT];
+    cd g[CNT], m[CNT];
 #pragma unroll
-    for (int c = 0; c < CNT; c++) t[c] = m[c] = cd{0, 0};
+    for (int c = 0; c < CNT; c++) g[c] = m[c] = cd{0, 0};
 #pragma unroll 1
     for (int f = 0; f < 6; f++) {
         const int tid = round_tid();
-        x_load<N, HX>(in.p[f], lds, tw, yb, z, second_power(f), dk, tid);
-        x_lines<N, +1>(lds, tw, tid);
+        x_load<N, HX>(in.p[f], lds, t, yb, z, second_power(f), dk, tid);
+        x_lines<N, +1>(lds, t, tid);
 #pragma unroll
         for (int c = 0; c < CNT; c++) {
             const int i = tid + c * S::NT;
             if (!(TOTAL % S::NT == 0 || i < TOTAL)) continue;
             const cd v = scale(lds[EX::idx(i / NC, i % NC)], s);
             if (f < 3) {
-                m[c] = cd{m[c].x + t[c].x * v.x, m[c].y + t[c].y * v.y};
-                t[c] = t[c] + v;
+                m[c] = cd{m[c].x + g[c].x * v.x, m[c].y + g[c].y * v.y};
+                g[c] = g[c] + v;
             } else {
                 m[c] = cd{m[c].x - v.x * v.x, m[c].y - v.y * v.y};
             }
@@ -258,6 +265,9 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 4) void k_ic_xf(SRC src,
     using EX = typename S::P::EX;
     constexpr int B = S::B, NC = N / 2, TOTAL = B * NC, CNT = (TOTAL + S::NT - 1) / S::NT;
     __shared__ cd lds[EX::LDS_ELEMS];
+    __shared__ cd twl[N];
+    const cd *t = stage_twiddles<double, N, true>(tw, twl, threadIdx.x, S::NT);
+    __syncthreads();
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / B), z = lb / (N / B);
     const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
 #pragma unroll 1
@@ -274,8 +284,8 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), 4) void k_ic_xf(SRC src,
             const int i = tid + c * S::NT;
             if (TOTAL % S::NT == 0 || i < TOTAL) lds[EX::idx(i / NC, i % NC)] = v[c];
         }
-        x_lines<N, -1>(lds, tw, tid);
-        x_store<N, HX>(lds, out.p[f], tw, yb, z, pw.r[f], dk, tid);
+        x_lines<N, -1>(lds, t, tid);
+        x_store<N, HX>(lds, out.p[f], t, yb, z, pw.r[f], dk, tid);
         __syncthreads();
     }
 }
@@ -291,6 +301,9 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), DIAG ? 2 : 3) void k_ic_
     using EX = typename S::P::EX;
     constexpr int B = S::B, NC = N / 2, TOTAL = B * NC, CNT = (TOTAL + S::NT - 1) / S::NT;
     __shared__ cd lds[EX::LDS_ELEMS];
+    __shared__ cd twl[N];
+    const cd *t = stage_twiddles<double, N, true>(tw, twl, threadIdx.x, S::NT);
+    __syncthreads();
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / B), z = lb / (N / B);
     const size_t base = (size_t)N * N * z + (size_t)N * yb * B;
     constexpr int F0 = DIAG ? 0 : 3;
@@ -304,8 +317,8 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), DIAG ? 2 : 3) void k_ic_
 #pragma unroll 1
         for (int f = 0; f < 3; f++) {  // a = the fields, the last one in a[2]
             const int tid = round_tid();
-            x_load<N, HX>(in.p[f], lds, tw, yb, z, second_power(F0 + f), dk, tid);
-            x_lines<N, +1>(lds, tw, tid);
+            x_load<N, HX>(in.p[f], lds, t, yb, z, second_power(F0 + f), dk, tid);
+            x_lines<N, +1>(lds, t, tid);
 #pragma unroll
             for (int c = 0; c < CNT; c++) {
                 const int i = tid + c * S::NT;
@@ -320,8 +333,8 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), DIAG ? 2 : 3) void k_ic_
     for (int f = 0; f < 3; f++) {
         const int tid = round_tid();
         if constexpr (!DIAG) {
-            x_load<N, HX>(in.p[f], lds, tw, yb, z, second_power(F0 + f), dk, tid);
-            x_lines<N, +1>(lds, tw, tid);
+            x_load<N, HX>(in.p[f], lds, t, yb, z, second_power(F0 + f), dk, tid);
+            x_lines<N, +1>(lds, t, tid);
         }
 #pragma unroll
         for (int c = 0; c < CNT; c++) {
@@ -339,8 +352,8 @@ __global__ __launch_bounds__((FftShape<double, N>::NT), DIAG ? 2 : 3) void k_ic_
                 v = cd{-2.0 * (m[c].x * x.x), -2.0 * (m[c].y * x.y)};
             }
         }
-        x_lines<N, -1>(lds, tw, tid);
-        x_store<N, HX>(lds, out.p[f], tw, yb, z, second_power(F0 + f), dk, tid);
+        x_lines<N, -1>(lds, t, tid);
+        x_store<N, HX>(lds, out.p[f], t, yb, z, second_power(F0 + f), dk, tid);
         __syncthreads();
     }
 }
@@ -606,8 +619,8 @@ struct IcN {
         }
     }
 
-    static void phi(const IcWork &w, double L, int ntab, hipStream_t st) {
-        const IcAmplitude amp{(const double *)w.kt, (const double *)w.pt, ntab, L};
+    static void phi(const IcWork &w, double L, hipStream_t st) {
+        const IcAmplitude amp{(const double *)w.amp};
         k_ic_zf<n, 1><<<n * H / S::B, S::NTY, 0, st>>>(IcIn{{(const cd *)w.Z[0]}}, PhiDst<n>{(cd *)w.F, amp},
                                                       (const cd *)w.twn, 2 * M_PI / L);
     }
@@ -672,8 +685,8 @@ struct IcN {
             k_ic_zf<ext, 3><<<bz, E::NTY, 0, st>>>(IcIn{{Z[0], Z[1], Z[2]}}, PadAdjDst<n>{(cd *)w.Fb, pad * s}, tw, dk);
         }
     }
-    static void phi_adj(const IcWork &w, double L, int ntab, hipStream_t st) {
-        const IcAmplitude amp{(const double *)w.kt, (const double *)w.pt, ntab, L};
+    static void phi_adj(const IcWork &w, double L, hipStream_t st) {
+        const IcAmplitude amp{(const double *)w.amp};
         zi<1>(w, PhiAdjSrc<n>{(const cd *)w.Fb, amp}, IcOut{{(cd *)w.Z[0]}}, 2 * M_PI / L, st);
     }
 };

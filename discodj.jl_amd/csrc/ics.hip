@@ -186,6 +186,7 @@ static hipError_t ic_work_ensure(IcWork &ws, int n, int order, int ntab) {
     ws.twn = twiddles(n);
     ws.kt = alloc((size_t)cap * 8);
     ws.pt = alloc((size_t)cap * 8);
+    ws.amp = alloc(ic_amplitudes(n) * 8);
     ws.F = alloc(HC * 16);
     ws.Fb = alloc(HC * 16);
     ws.w = alloc(M * 8);
@@ -260,16 +261,28 @@ static hipError_t ic_white(IcWork &ws, FftOps &fn, int n, const double *white, b
     return hipGetLastError();
 }
 
-static hipError_t ic_tables(IcWork &ws, const double *kt, const double *pt, int ntab, hipStream_t st) {
+__global__ void k_ic_amplitudes(double *amp, size_t cnt, int n, double L, const double *kt, const double *pt, int ntab) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < cnt) amp[i] = ic_amplitude_entry(i, n, L, kt, pt, ntab);
+}
+
+// the P(k) table, and the amplitude of every mode length from it (searched once per length instead of once per mode:
+// the z pass that applies it took AMP0 us at n = 256, AMP1 so)
+static hipError_t ic_tables(IcWork &ws, int n, double L, const double *kt, const double *pt, int ntab, hipStream_t st) {
     hipError_t err = hipMemcpyAsync(ws.kt, kt, ntab * 8, hipMemcpyHostToDevice, st);
-    return err == hipSuccess ? hipMemcpyAsync(ws.pt, pt, ntab * 8, hipMemcpyHostToDevice, st) : err;
+    if (err == hipSuccess) err = hipMemcpyAsync(ws.pt, pt, ntab * 8, hipMemcpyHostToDevice, st);
+    if (err != hipSuccess) return err;
+    const size_t cnt = ic_amplitudes(n);
+    k_ic_amplitudes<<<g1(cnt), 256, 0, st>>>((double *)ws.amp, cnt, n, L, (const double *)ws.kt, (const double *)ws.pt,
+                                             ntab);
+    return hipGetLastError();
 }
 
 // phi(k) of the white noise w
-static void ic_phi(IcWork &ws, FftOps &fn, const IcPasses &ic, const double *w, double L, int ntab, hipStream_t st) {
+static void ic_phi(IcWork &ws, FftOps &fn, const IcPasses &ic, const double *w, double L, hipStream_t st) {
     fn.xf(w, false, ws.W[0], ws.twn, 1.0, st);
     fn.yf(ws.W[0], ws.Z[0], ws.twn, st);
-    ic.phi(ws, L, ntab, st);
+    ic.phi(ws, L, st);
 }
 
 // host orchestration; returns a HIP error code (0 = success)
@@ -281,13 +294,13 @@ int ics_lpt_device(IcWork &ws, int n, double L, int order, const double *white, 
     if (!fft_dispatch<double>(n, fn) || !ic_passes(n, ic) || (order >= 2 && !ic.has_second)) return (int)hipErrorInvalidValue;
     hipError_t err = ic_work_ensure(ws, n, order, ntab);
     if (err != hipSuccess) return (int)err;
-    err = ic_tables(ws, kt_h, pt_h, ntab, st);
+    err = ic_tables(ws, n, L, kt_h, pt_h, ntab, st);
     const bool two = order >= 2, keep = two && ic_keep_ensure(ws, n);
     ws.fk_valid = false;
     double *w = (double *)(keep && white ? ws.wkey : ws.w);  // the key of the kept fields
     if (err == hipSuccess) err = ic_white(ws, fn, n, white, white_on_device, seed, w, st);
     if (err == hipSuccess) {
-        ic_phi(ws, fn, ic, w, L, ntab, st);
+        ic_phi(ws, fn, ic, w, L, st);
         if (two) {
             ic.second(ws, L, st);
             ic.source(ws, L, st);
@@ -325,7 +338,7 @@ int ics_lpt_vjp_device(IcWork &ws, int n, double L, int order, const double *whi
     const size_t M = (size_t)n * n * n;
     hipError_t err = ic_work_ensure(ws, n, order, ntab);
     if (err != hipSuccess) return (int)err;
-    err = ic_tables(ws, kt_h, pt_h, ntab, st);
+    err = ic_tables(ws, n, L, kt_h, pt_h, ntab, st);
     const bool two = order >= 2;
     // The spectra of the last forward serve when they were computed from the same inputs: n, L, order, the
     // same P(k) table values, and the same seed or white-noise values (compared bit for bit on the device)
@@ -345,7 +358,7 @@ int ics_lpt_vjp_device(IcWork &ws, int n, double L, int order, const double *whi
         if (err == hipSuccess) err = hipStreamSynchronize(st);
         hit = err == hipSuccess && !differs;
     }
-    if (err == hipSuccess && two && !hit) ic_phi(ws, fn, ic, w, L, ntab, st);
+    if (err == hipSuccess && two && !hit) ic_phi(ws, fn, ic, w, L, st);
     if (err == hipSuccess) {
         ic.combine_adj(ws, L, D, two, prec, psibar, pibar, st);
         if (two) {
@@ -357,7 +370,7 @@ int ics_lpt_vjp_device(IcWork &ws, int n, double L, int order, const double *whi
             ic.source_adj(ws, L, st);
         }
         // phi = r2c(w) s(k):  wbar = c2r(phibar s / w)
-        ic.phi_adj(ws, L, ntab, st);
+        ic.phi_adj(ws, L, st);
         fn.yi(ws.Z[0], ws.W[0], ws.twn, st);
         fn.xi(ws.W[0], w, ws.twn, st);
         err = hipGetLastError();
