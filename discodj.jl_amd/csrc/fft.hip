@@ -25,16 +25,15 @@ __global__ __launch_bounds__(256) void k_xf(const IN *__restrict__ mesh, cx<T> *
     using S = FftShape<T, N>;
     using P = typename S::P;
     __shared__ cx<T> lds[P::EX::LDS_ELEMS];
-    // FP32: the twiddle table in LDS (read by the transforms and the post-processing; through the caches
-    // the pass took 1.92 against 1.62 ms at 1024^3, at three workgroups per CU instead of four)
-    constexpr bool TWX = sizeof(T) == 4;
-    __shared__ cx<T> twl[TWX ? N : 1];
-    const cx<T> *t = stage_twiddles<T, N, TWX>(tw, twl, threadIdx.x, 256);
+    // the twiddle table in LDS (read by the transforms and the post-processing; through the caches the pass took
+    // 1.92 against 1.62 ms at 1024^3 in FP32, at three workgroups per CU instead of four, and 25 against 21 us at
+    // 192^3, 432 against 400 us at 512^3 in FP64)
+    __shared__ cx<T> twl[N];
+    const cx<T> *t = stage_twiddles<T, N, true>(tw, twl, threadIdx.x, 256);
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / S::B), z = lb / (N / S::B);
     if constexpr (P::EX::wave_ok()) {
         P::xf_load_w(mesh, lds, yb, z, threadIdx.x, fixed_scale);
-        if constexpr (TWX) __syncthreads();
-        else P::EX::wave_sync();
+        __syncthreads();
         P::EX::template run_wave<-1, 2>(lds, t, threadIdx.x);
         __syncthreads();
     } else {
@@ -53,21 +52,15 @@ __global__ __launch_bounds__((FftShape<T, N>::NTXI)) void k_xi(const cx<T> *__re
     using S = FftShape<T, N>;
     using P = typename S::PXI;
     __shared__ cx<T> lds[P::EX::LDS_ELEMS];
-    // FP32: the twiddle table in LDS, staged while the block's loads are in flight (1.99 against 1.56 ms
-    // at 1024^3)
-    constexpr bool TWX = sizeof(T) == 4;
-    __shared__ cx<T> twl[TWX ? N : 1];
+    // the twiddle table in LDS, staged while the block's loads are in flight (1.99 against 1.56 ms at 1024^3 in
+    // FP32, 426 against 374 us at 512^3 in FP64)
+    __shared__ cx<T> twl[N];
     const int lb = xcd_block(blockIdx.x, gridDim.x), yb = lb % (N / S::BXI), z = lb / (N / S::BXI);
-    const cx<T> *t = tw;
-    if constexpr (TWX) {
-        cx<T> va[P::XI_CNT], vb[P::XI_CNT];
-        P::xi_fetch(A, yb, z, threadIdx.x, va, vb);
-        t = stage_twiddles<T, N, true>(tw, twl, threadIdx.x, S::NTXI);
-        __syncthreads();
-        P::template xi_pre<MUL>(lds, t, threadIdx.x, va, vb, tab);
-    } else {
-        P::template xi_load_pre<MUL>(A, lds, tw, yb, z, threadIdx.x, tab);
-    }
+    cx<T> va[P::XI_CNT], vb[P::XI_CNT];
+    P::xi_fetch(A, yb, z, threadIdx.x, va, vb);
+    const cx<T> *t = stage_twiddles<T, N, true>(tw, twl, threadIdx.x, S::NTXI);
+    __syncthreads();
+    P::template xi_pre<MUL>(lds, t, threadIdx.x, va, vb, tab);
     __syncthreads();
     if constexpr (P::EX::wave_ok()) {
         P::EX::template run_wave<+1, 2>(lds, t, threadIdx.x);
