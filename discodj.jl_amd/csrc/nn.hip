@@ -439,10 +439,9 @@ __global__ __launch_bounds__(256) void k_nn_loss_total(double *sum) {
     if (threadIdx.x == 0) sum[NN_LOSS_BLOCKS] = red[0];
 }
 
-#ifndef NNMB
-#define NNMB 256
-#endif
-constexpr int NN_MIN_BLOCKS = NNMB;
+// convolution blocks below which a block takes fewer planes (one to a CU; a training step at 64^3: 1.27 ms with 128,
+// 1.15 with 256 and 512)
+constexpr int NN_MIN_BLOCKS = 256;
 static unsigned ngrid(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 struct NnLaunch {

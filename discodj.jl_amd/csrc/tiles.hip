@@ -448,14 +448,15 @@ template <typename Acc> __device__ __forceinline__ void zero_acc(Acc *acc, int c
 // The tile's cells to the mesh, 16 bytes a thread and turn: a cell a turn spent more instructions on a tile of 512
 // particles than their entries did (TSC at 1024^3: 2.23 ms a pass, 2.05 so).  cell(i): the value of accumulator i
 template <typename O, typename F>
-__device__ __forceinline__ void store_tile(O *mesh, const TileGeom &g, const int (&o3)[3], int pad, int sxd, const F &cell) {
+__device__ __forceinline__ void store_tile(O *mesh, const TileGeom &g, const int (&o3)[3], int rows, int pad, int sxd,
+                                           const F &cell) {
     constexpr int V = 16 / (int)sizeof(O), LV = V == 4 ? 2 : 1;
     struct alignas(16) Vec {
         O v[V];
     };
     const int lgx = g.lT[0] - LV, gx = (threadIdx.x & ((1 << lgx) - 1)) * V;
     const unsigned N = (unsigned)g.N;
-    for (int r = threadIdx.x >> lgx; r < g.TY * g.TZ; r += blockDim.x >> lgx) {
+    for (int r = threadIdx.x >> lgx; r < rows; r += blockDim.x >> lgx) {
         const unsigned ly = r & (g.TY - 1), lz = r >> g.lT[1];
         const unsigned gi = (o3[0] + gx) + N * ((o3[1] + ly) + N * (o3[2] + lz));  // cell indices < N^3 <= 2^30
         const int li = gx + pad + sxd * r;
@@ -478,24 +479,29 @@ template <typename T, int W, int ACC, bool PAD>
 __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
                                              const unsigned *__restrict__ gstart, const unsigned *__restrict__ cnt,
                                              unsigned cap, const TileGeom &g, T sx, T sy, T sz, T L, void *mesh,
-                                             double fscale, int qbits) {
+                                             double fscale, int qbits, int parts) {
     using Acc = typename std::conditional<ACC == ACC_T, T,
                                           typename std::conditional<ACC == ACC_Q32, unsigned, unsigned long long>::type>::type;
     extern __shared__ unsigned char smem[];
     Acc *acc = (Acc *)smem;
     constexpr int P = W - 1;
-    const int t = blockIdx.x, TV = g.TX * g.TY * g.TZ;
-    const int SXD = PAD ? g.TX + 2 * P : g.TX, ROWS = g.TY * g.TZ, CELLS = PAD ? SXD * ROWS : TV;
+    const int t = blockIdx.x / parts, TZ = g.TZ / parts, TV = g.TX * g.TY * TZ;
+    const int SXD = PAD ? g.TX + 2 * P : g.TX, ROWS = g.TY * TZ, CELLS = PAD ? SXD * ROWS : TV;
     zero_acc(acc, CELLS);
     const int tx = t % g.ntx, ty = (t / g.ntx) % g.nty, tz = t / (g.ntx * g.nty);
-    const int ox = tx << g.lT[0], oy = ty << g.lT[1], oz = tz << g.lT[2];
+    const int ox = tx << g.lT[0], oy = ty << g.lT[1], oz = (tz << g.lT[2]) + (int)(blockIdx.x % parts) * TZ;
     __syncthreads();
     // the tile's own list, then its ghost list
     const unsigned s_own = start[t], g0 = gstart[t], n_own = list_len(cnt[t], s_own, g0, cap),
                    n_all = n_own + list_len(cnt[g.nt + t], g0, start[t + 1], cap), s_gh = g0 - n_own;
-    const int o3[3] = {ox, oy, oz}, T3[3] = {g.TX, g.TY, g.TZ};
-    for (unsigned i = threadIdx.x; i < n_all; i += blockDim.x) {
-        const Entry<T> en = ent[i < n_own ? s_own + i : s_gh + i];
+    const int o3[3] = {ox, oy, oz}, T3[3] = {g.TX, g.TY, TZ};
+    unsigned i = threadIdx.x;
+    Entry<T> nx{};
+    if (i < n_all) nx = ent[i < n_own ? s_own + i : s_gh + i];
+    while (i < n_all) {
+        const Entry<T> en = nx;
+        i += blockDim.x;
+        if (i < n_all) nx = ent[i < n_own ? s_own + i : s_gh + i];  // in flight during this entry's atomics
         const T xs[3] = {en.x + sx, en.y + sy, en.z + sz};
         T w[3][W];
         int b0[3];
@@ -534,7 +540,7 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
             for (int o = 0; o < W; o++) {
                 const int y = l0[1] + o, z = l0[2] + o;
                 ly[o] = (unsigned)y < (unsigned)g.TY ? __mul24(y, SXD) : BIG;
-                lz[o] = (okx && (unsigned)z < (unsigned)g.TZ) ? __mul24(z, SZ) : BIG;
+                lz[o] = (okx && (unsigned)z < (unsigned)TZ) ? __mul24(z, SZ) : BIG;
             }
             // rows outside the tile are skipped (their lanes sit out the row's atomics); sending them to a
             // shared discard row instead made every lane's atomics meet on one row
@@ -578,31 +584,36 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
     __syncthreads();
     const int pad = PAD ? P : 0;
     if constexpr (ACC == ACC_Q31) {
-        store_tile((T *)mesh, g, o3, pad, SXD, [&](int i) { return (T)((double)acc[i] * 0x1p-31); });
+        store_tile((T *)mesh, g, o3, ROWS, pad, SXD, [&](int i) { return (T)((double)acc[i] * 0x1p-31); });
     } else if constexpr (ACC == ACC_Q32) {
         const T inv = (T)ldexpf(1.0f, -qbits);  // the cell's sum rounds once, in its conversion
-        store_tile((T *)mesh, g, o3, pad, SXD, [&](int i) { return (T)acc[i] * inv; });
+        store_tile((T *)mesh, g, o3, ROWS, pad, SXD, [&](int i) { return (T)acc[i] * inv; });
     } else {
-        store_tile((Acc *)mesh, g, o3, pad, SXD, [&](int i) { return acc[i]; });
+        store_tile((Acc *)mesh, g, o3, ROWS, pad, SXD, [&](int i) { return acc[i]; });
     }
 }
 
+// Workgroup (tile, part): on a mesh of few tiles, each tile's z planes are shared by several workgroups, which all read
+// its lists (rows outside a part are skipped, the sums are the same; ten steps at 64^3: 0.70 against 0.69 ms, and 0.67
+// with each entry loaded during the one before it).
+inline int deposit_parts(const TileGeom &g) { return g.nt <= 128 ? 4 : g.nt <= 256 ? 2 : 1; }
 // FP32 tiles (ACC_Q31) with fewer than 2^12 entries sum in 32 bits (ACC_Q32); the LDS holds 64-bit
 // accumulators either way
 template <typename T, int W, int ACC, bool PAD>
 __global__ __launch_bounds__(512) void k_tile_deposit(const Entry<T> *__restrict__ ent, const unsigned *__restrict__ start,
                                                       const unsigned *__restrict__ gstart, const unsigned *__restrict__ cnt,
                                                       unsigned cap, TileGeom g, T sx, T sy, T sz, T L, void *mesh,
-                                                      double fscale) {
+                                                      double fscale, int parts) {
     if constexpr (ACC == ACC_Q31) {
-        const unsigned t = blockIdx.x, e = cnt[t] + cnt[g.nt + t];
+        const unsigned t = blockIdx.x / parts, e = cnt[t] + cnt[g.nt + t];
         const int qbits = 32 - (32 - __clz(e));  // 32 - bits(e): e 2^qbits < 2^32
         if (qbits >= Q32_MIN_BITS) {
-            tile_deposit<T, W, ACC_Q32, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, min(qbits, 31));
+            tile_deposit<T, W, ACC_Q32, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, min(qbits, 31),
+                                          parts);
             return;
         }
     }
-    tile_deposit<T, W, ACC, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, 31);
+    tile_deposit<T, W, ACC, PAD>(ent, start, gstart, cnt, cap, g, sx, sy, sz, L, mesh, fscale, 31, parts);
 }
 
 // Vector deposit (reverse mode): out_c(cell) = sum_p W(X_p + s - cell) vals[p + c np] scale for c = 0, 1, 2,
@@ -782,7 +793,7 @@ __global__ __launch_bounds__(512) void k_tile_deposit3q(const Entry<float> *__re
     __syncthreads();
     const size_t M = (size_t)g.N * g.N * g.N;
     const double inv = s > 0.f ? 1.0 / (double)s : 0.0;
-    store_tile(out + (size_t)comp * M, g, o3, P, SXD, [&](int i) { return (float)((double)(long long)acc[i] * inv); });
+    store_tile(out + (size_t)comp * M, g, o3, ROWS, P, SXD, [&](int i) { return (float)((double)(long long)acc[i] * inv); });
 }
 
 // ------------------------------------------------------------------------------------ gather
@@ -1186,7 +1197,7 @@ struct MarchMap {
 // Segments are as long as leaves MARCH_WGS workgroups (four per CU; 16 tiles at most, where a tile stages
 // TZ of S2 planes and longer ones gain nothing).  A mesh of too few tiles for that gives every tile up to
 // four workgroups, each of which stages the tile and takes its part of the list.  16 tiles everywhere left
-// a 64^3 mesh with 8 workgroups (97 us; 20 us with 256) and a 256^3 mesh with one per CU (279 us a pass,
+// a 64^3 mesh with 8 workgroups (97 us; 9 us with 256) and a 256^3 mesh with one per CU (279 us a pass,
 // CIC, order 4; 204 us with four).
 constexpr int MARCH_WGS = 1024;
 inline MarchMap march_map(const TileGeom &g) {
@@ -1373,15 +1384,16 @@ struct TileLaunch {
     static void dep_w(const TileArgs &a, const double *sh, void *mesh, double fscale, hipStream_t st) {
         const TileGeom &g = a.g;
         const bool pad = g.ntx >= 2 && g.nty >= 2 && g.ntz >= 2;
-        const size_t cells = pad ? (size_t)(g.TX + 2 * (W - 1)) * (g.TY * g.TZ) : (size_t)g.TX * g.TY * g.TZ;
+        const int parts = deposit_parts(g);
+        const size_t cells = (size_t)(pad ? g.TX + 2 * (W - 1) : g.TX) * g.TY * (g.TZ / parts);
         const size_t shm = cells * (ACC == ACC_T ? sizeof(T) : 8);
         auto kern = pad ? k_tile_deposit<T, W, ACC, true> : k_tile_deposit<T, W, ACC, false>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         // 512 threads: the four workgroups that the accumulators' LDS allows per CU then hold the
         // CU's full 32 waves, twice as many LDS atomics in flight as with 256 (2.97 -> 2.56 ms at
         // 512^3 on 1024^3, TSC)
-        kern<<<g.nt, 512, shm, st>>>((const Entry<T> *)a.ent, a.start, a.gstart, a.cur, cap32(a), g, (T)sh[0], (T)sh[1],
-                                     (T)sh[2], (T)a.L, mesh, fscale);
+        kern<<<g.nt * parts, 512, shm, st>>>((const Entry<T> *)a.ent, a.start, a.gstart, a.cur, cap32(a), g, (T)sh[0],
+                                             (T)sh[1], (T)sh[2], (T)a.L, mesh, fscale, parts);
     }
     template <int W>
     static void dep_sel(const TileArgs &a, bool fixed, const double *sh, void *mesh, double fscale, hipStream_t st) {
