@@ -88,8 +88,8 @@ template void pk_bin<double>(const void *, int, double, int, int, double, double
 //   W > 0:   v is divided by |W(k)|^2 = prod_a sinc(k_a dx / 2)^(2 W) (mass-assignment window)
 // A thread takes one z and PK_XL consecutive x of a y row, so that its entries stay in one bin for a while:
 // their sums stay in registers until the bin changes (LDS atomics once per run of entries; neighbouring
-// lanes mostly share the bin, so one atomic per entry met 64 others at one address: 1.45 ms for 512^3, FP32,
-// with the window's sin and pow per entry, against 0.2 ms).  The window's factors are a table in LDS.
+// lanes mostly share the bin, so one atomic per entry met 64 others at one address: 482 us a call,
+// FP32, over three of 256^3 and one of 512^3 with the window's sin and pow per entry, against 84).  The window's factors are a table in LDS.
 constexpr int PK_XL = 16, PK_COPIES = 4;
 
 template <typename T, bool CROSS, bool KSUM>

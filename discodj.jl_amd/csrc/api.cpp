@@ -655,7 +655,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
             const bool last = s == ns - 1;
             // first pass stores acc, later passes add to it; the kick and drifts follow in particle order.  With
             // one pass the gather stores acc at the particles: kicking inside it, in list order, took 560 us at
-            // 256^3 (CIC, order 4), the gather and the streaming kick take 204 and 190
+            // 256^3 (CIC, order 4), the gather and the streaming kick take 224 and 155
             const int gmode = s == 0 ? GATHER_ASSIGN : GATHER_ACC;
             {
                 Prof p(c, listed_kick && last ? K_GATHER_LAST : K_GATHER);
