@@ -90,9 +90,11 @@ template void pk_bin<double>(const void *, int, double, int, int, double, double
 // their sums stay in registers until the bin changes (LDS atomics once per run of entries; neighbouring
 // lanes mostly share the bin, so one atomic per entry met 64 others at one address: 482 us a call,
 // FP32, over three of 256^3 and one of 512^3 with the window's sin and pow per entry, against 84).  The window's factors are a table in LDS.
-constexpr int PK_XL = 16, PK_COPIES = 4;
+// PK_XL is 16, and 4 on meshes up to 64^3, where few threads would walk long runs one after the other: the spectra
+// of 32^3 on 32^3 took 251 us with 16 and 215 with 4, of 64^3 on 64^3 259 and 231 (FP32).
+constexpr int PK_COPIES = 4;
 
-template <typename T, bool CROSS, bool KSUM>
+template <typename T, bool CROSS, bool KSUM, int PK_XL>
 __global__ __launch_bounds__(256) void k_pk_edges(const cx<T> *__restrict__ F1, const cx<T> *__restrict__ F2, int N,
                                                   double kf, double dx, int W, int wmode, double scale, PkEdges thr,
                                                   double *__restrict__ sums) {
@@ -227,14 +229,18 @@ void pk_edges(const void *F1, const void *F2, int N, double L, int W, int wmode,
     thr.nbins = nb;
     for (int b = 0; b <= nb; b++) thr.e[b] = pk_threshold(ed.e[b]);
     const size_t shm = sizeof(double) * ((size_t)(nb + 1) + PK_COPIES * 4 * (size_t)nb + (W > 0 ? H : 0));
+    const int xl = N <= 64 ? 4 : 16;
     // a block's bins reach memory once, so four blocks per CU walk the rows
-    const int items = N * (((H + PK_XL - 1) / PK_XL * N + 255) / 256), blocks = std::min(1024, items);
+    const int items = N * (((H + xl - 1) / xl * N + 255) / 256), blocks = std::min(1024, items);
     auto launch = [&](auto kern) {
         kern<<<blocks, 256, shm, st>>>((const cx<T> *)F1, (const cx<T> *)F2, N, 2 * M_PI / L, L / N, W, wmode, scale,
                                        thr, sums);
     };
-    if (F2) ksum ? launch(k_pk_edges<T, true, true>) : launch(k_pk_edges<T, true, false>);
-    else ksum ? launch(k_pk_edges<T, false, true>) : launch(k_pk_edges<T, false, false>);
+    auto pick = [&](auto k4, auto k16) { xl == 4 ? launch(k4) : launch(k16); };
+    if (F2) ksum ? pick(k_pk_edges<T, true, true, 4>, k_pk_edges<T, true, true, 16>)
+                 : pick(k_pk_edges<T, true, false, 4>, k_pk_edges<T, true, false, 16>);
+    else ksum ? pick(k_pk_edges<T, false, true, 4>, k_pk_edges<T, false, true, 16>)
+              : pick(k_pk_edges<T, false, false, 4>, k_pk_edges<T, false, false, 16>);
 }
 template void pk_edges<float>(const void *, const void *, int, double, int, int, double, const PkEdges &, bool,
                               double *, hipStream_t);
