@@ -582,6 +582,15 @@ void ik_force_mesh(dj_ctx *c, int ax, void *out) {
     else c->fft.xi(c->A, out, c->tw, c->st);
 }
 
+// With sheet resampling the particles' own lists would serve the spectral gradient's gather alone.  For few
+// particles their sort and the tiles cost more than reading the mesh in particle order: a step with linear
+// resampling (CIC) of 24^3 on 64^3 took 408 us with them and 285 without, 128^3 on 128^3 1389 and 1281; PCS, with
+// eight times the reads, 408 and 357 at 32^3 on 96^3 and 461 and 439 at 48^3 on 96^3.
+bool ik_in_particle_order(const dj_ctx *c) {
+    const int64_t side = c->cfg.worder == 2 ? 128 : c->cfg.worder == 3 ? 64 : 48;
+    return c->cfg.grad_order == 0 && c->cfg.n_resample > 1 && c->rs_tiled && c->np <= side * side * side;
+}
+
 dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool defer = false) {
     const dj_pm_config &cfg = c->cfg;
     const bool fixed = cfg.deposit == DJ_DEPOSIT_FIXED64;
@@ -597,8 +606,11 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
     // particle order (k_kick_listed), reading the sum through the own-list entry the bin records
     const bool listed_kick = mode == FORCE_KICK && ns > 1 && !ik;
     if (listed_kick && !c->own_at) HIPCHK(c, hipMalloc(&c->own_at, sizeof(unsigned) * (size_t)c->np));
-    dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
-    if (rs) return rs;
+    const bool unlisted = ik_in_particle_order(c);
+    if (!unlisted) {
+        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
+        if (rs) return rs;
+    }
     (void)mesh_bytes;
     // in a step the passes hand the acceleration over in tile-list order: both walk the same lists, so
     // the hand-over is read and written contiguously instead of at the particles' positions
@@ -670,8 +682,11 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
             for (int ax = 0; ax < 3; ax++) {
                 ik_force_mesh(c, ax, c->mesh);
                 Prof p(c, K_GATHER);
-                c->tiles.gather_comp(ta, cfg.worder, c->shifts[s], c->mesh, s == 0 ? GATHER_ASSIGN : GATHER_ACC, ax,
-                                     c->st);
+                const int gmode = s == 0 ? GATHER_ASSIGN : GATHER_ACC;
+                if (unlisted)
+                    c->part.gather_comp(psi, c->q1, c->n, c->shifts[s], c->mesh, c->res, cfg.boxsize, cfg.worder, gmode,
+                                        ax, c->acc, c->st);
+                else c->tiles.gather_comp(ta, cfg.worder, c->shifts[s], c->mesh, gmode, ax, c->st);
             }
         }
         dj_status r = check_launch(c, "force pass");

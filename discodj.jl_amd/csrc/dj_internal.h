@@ -65,6 +65,10 @@ struct PartOps {
                      hipStream_t st);
     // mom = alpha mom + beta acc/ns ; psi += dd2 mom [; psi += dd1_next mom]
     void (*kick_drift)(void *psi, void *mom, const void *acc, int64_t n3, const KickArgs &k, hipStream_t st);
+    // acc component comp = (assign) or += the field interpolated at the particles' positions psi + q + sh, in
+    // particle order, without tile lists
+    void (*gather_comp)(const void *psi, const void *q1, int n, const double *sh, const void *field, int res, double L,
+                        int W, int mode, int comp, void *acc, hipStream_t st);
     // x *= s
     void (*scale)(void *x, int64_t n, double s, hipStream_t st);
     // x = 0 (a fill kernel, graph-capture safe)

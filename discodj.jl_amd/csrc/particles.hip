@@ -1,10 +1,11 @@
-// Particle-side kernels of the PM step: kick and drift.
+// Particle-side kernels of the PM step: kick, drift and the interpolation in particle order.
 //
 // Particles are the reference's column-major (n,n,n,3) arrays: component c of particle i + n (j + n k) is at
 // that index + c n^3.
 #include <hip/hip_runtime.h>
 
 #include "dj_internal.h"
+#include "stencil.h"
 
 namespace dj {
 
@@ -43,6 +44,43 @@ __global__ __launch_bounds__(256) void k_kick_drift(T *__restrict__ psi, T *__re
     if (has_next) s = s + dd1n * m;
     mom[i] = m;
     psi[i] = s;
+}
+
+// One component of the force at every particle, read from the mesh at the W^3 cells: bound by the latency of its
+// scattered reads.  A tile of LDS serves them better once the particles are many, but needs the tile lists: see
+// ik_in_particle_order for the line and its figures.
+template <typename T, int W, int MODE>
+__global__ __launch_bounds__(256) void k_gather_comp(const T *__restrict__ psi, const T *__restrict__ q1, int n, T sx,
+                                                     T sy, T sz, const T *__restrict__ f, int res, T L, int comp,
+                                                     T *__restrict__ acc) {
+    const unsigned np = (unsigned)n * n * n, p = blockIdx.x * 256u + threadIdx.x;
+    if (p >= np) return;
+    const unsigned i = p % n, r = p / n, j = r % n, k = r / n;
+    const T X[3] = {(psi[p] + q1[i]) + sx, (psi[p + (size_t)np] + q1[j]) + sy, (psi[p + 2 * (size_t)np] + q1[k]) + sz};
+    T w[3][W];
+    int c[3][W];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const T g = tjmod(X[a], L) / L * (T)res;
+        const int b = twbase<W>(g) + twlo<W>();
+#pragma unroll
+        for (int o = 0; o < W; o++) {
+            w[a][o] = twk<W>(fabs(g - (T)(b + o)));
+            c[a][o] = timod(b + o, res);
+        }
+    }
+    T s = 0;
+#pragma unroll
+    for (int oz = 0; oz < W; oz++)
+#pragma unroll
+        for (int oy = 0; oy < W; oy++) {
+            const size_t row = (size_t)res * (c[1][oy] + (size_t)res * c[2][oz]);
+#pragma unroll
+            for (int ox = 0; ox < W; ox++) s += f[row + c[0][ox]] * (w[0][ox] * w[1][oy] * w[2][oz]);
+        }
+    T &out = acc[p + comp * (size_t)np];
+    if constexpr (MODE == GATHER_ACC) s = out + s;
+    out = s;
 }
 
 template <typename T>
@@ -84,6 +122,19 @@ static void kick_drift(void *psi, void *mom, const void *acc, int64_t n3, const 
 }
 
 template <typename T>
+static void gather_comp(const void *psi, const void *q1, int n, const double *sh, const void *field, int res, double L,
+                        int W, int mode, int comp, void *acc, hipStream_t st) {
+    auto launch = [&](auto kern) {
+        kern<<<lgrid((int64_t)n * n * n), 256, 0, st>>>((const T *)psi, (const T *)q1, n, (T)sh[0], (T)sh[1], (T)sh[2],
+                                                        (const T *)field, res, (T)L, comp, (T *)acc);
+    };
+    const bool add = mode == GATHER_ACC;
+    if (W == 2) add ? launch(k_gather_comp<T, 2, GATHER_ACC>) : launch(k_gather_comp<T, 2, GATHER_ASSIGN>);
+    else if (W == 3) add ? launch(k_gather_comp<T, 3, GATHER_ACC>) : launch(k_gather_comp<T, 3, GATHER_ASSIGN>);
+    else add ? launch(k_gather_comp<T, 4, GATHER_ACC>) : launch(k_gather_comp<T, 4, GATHER_ASSIGN>);
+}
+
+template <typename T>
 static void scale(void *x, int64_t n, double s, hipStream_t st) {
     k_scale<T><<<lgrid(n), 256, 0, st>>>((T *)x, n, (T)s);
 }
@@ -100,6 +151,7 @@ template <typename T> void part_ops(PartOps &ops) {
     ops.drift = drift<T>;
     ops.drift_to = drift_to<T>;
     ops.kick_drift = kick_drift<T>;
+    ops.gather_comp = gather_comp<T>;
     ops.scale = scale<T>;
     ops.zero = zero;
 }

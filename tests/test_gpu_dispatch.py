@@ -170,6 +170,20 @@ def test_spectral_force_over_tiles(W, res, n, aa, prec):
     assert G.rel(acc, ref) < (2e-5 if prec == 32 else 1e-12)
 
 
+@pytest.mark.parametrize("W, n, res, aa, prec", [(2, 7, 16, 1, 64), (2, 128, 128, 0, 32), (2, 129, 128, 1, 32),
+                                                 (3, 64, 64, 1, 64), (3, 65, 64, 1, 64), (4, 48, 96, 1, 32),
+                                                 (4, 49, 64, 0, 64)])
+def test_resampled_spectral_force_over_the_order_rule(W, n, res, aa, prec):
+    """The spectral gradient with sheet resampling, interpolated in particle order up to a number of particles and
+    from the tiles above it, against the oracle (the bounds of test_resampling_vs_oracle)."""
+    L = 2.0 * res
+    psi = _psi(n, 2.0, n + W, np.float32 if prec == 32 else np.float64)
+    kw = dict(worder=W, grad_order=0, antialias=aa, n_resample=2, resampling="linear")
+    acc = D.pm_acceleration(psi, D.PMConfig(res_pm=res, n_part=n, boxsize=L, **kw), precision=prec)
+    ref = O.pm_acceleration(psi.astype(np.float64), O.pm_config(res, n, L, **kw), "solver")
+    assert G.rel(acc, ref) < (1e-12 if prec == 64 else 5e-5)
+
+
 @pytest.mark.parametrize("n, order, prec", [(16, 2, 32), (24, 1, 64), (48, 1, 32), (96, 1, 64), (128, 2, 64), (192, 1, 64)])
 def test_ics_over_the_transform_sizes(n, order, prec):
     """Displacements and momenta of the ICs at sizes whose line groups differ (1e-12, or FP32's rounding of the
