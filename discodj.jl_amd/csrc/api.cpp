@@ -454,17 +454,32 @@ void free_lists(TileLists &tl) {
 // reserved from the previous sort's counts with room to double (particles move less than a tile per step), so
 // one fill pass writes them; a list that outgrows its reserve (or a full entry buffer) raises a flag,
 // and then the sort is repeated exactly: counting pass, lists of the exact sizes, fill.
-// defer: with lists to reserve from, enqueue the sort and leave the flag to the caller, whose kernels are
-// gated by it (SortGate) and read no entry beyond a list's reserve (list_len); a set flag means
-// sort_failed() and the force again.
+// What becomes of the fill's overflow flag:
+//   SORT_STOP   the stream ends and the host reads the flag (43 us a step of a run, whatever the mesh)
+//   SORT_ASK    with lists to reserve from, the host reads it from pinned memory as soon as the fill has ended
+//   SORT_DEFER  with lists to reserve from, the flag is left to the caller, whose kernels are gated by it (SortGate)
+//               and read no entry beyond a list's reserve (list_len); a set flag means sort_failed() and the force again
+enum SortCheck { SORT_STOP, SORT_ASK, SORT_DEFER };
+unsigned wait_report(dj_ctx *c, int slot);
+
 dj_status tile_sort_of(dj_ctx *c, TileLists &tl, const void *psi, const void *q1, int n, const double *d_shifts,
-                       int ns, int W, bool defer = false) {
+                       int ns, int W, SortCheck check = SORT_STOP) {
     TileArgs a = tile_args_of(c, tl, psi, q1, n, d_shifts, ns);
-    if (defer && tl.lists) {
-        Prof p(c, K_SORT);
-        c->tiles.scan(a, tl.cur, 1, c->st);
-        c->tiles.fill(a, W, c->st);
-        return check_launch(c, "tile binning");
+    if (check != SORT_STOP && tl.lists) {
+        {
+            Prof p(c, K_SORT);
+            c->tiles.scan(a, tl.cur, 1, c->st);
+            c->tiles.fill(a, W, c->st);
+        }
+        if (check == SORT_ASK) {
+            c->report[0] = 0;
+            c->tiles.report(SortGate{tl.flag, c->report}, c->st);
+        }
+        dj_status r = check_launch(c, "tile binning");
+        if (r || check == SORT_DEFER || wait_report(c, 0) == 1) return r;
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        tl.lists = false;
+        c->part.zero(tl.flag, sizeof(unsigned), c->st);
     }
     for (int attempt = 0; attempt < 3; attempt++) {
         const bool exact = !tl.lists || attempt > 0;
@@ -518,8 +533,8 @@ dj_status tile_sort_of(dj_ctx *c, TileLists &tl, const void *psi, const void *q1
     return fail(c, DJ_ERR_DEVICE, "tile binning: lists did not fit after an exact recount");
 }
 
-dj_status tile_sort(dj_ctx *c, const void *psi, const double *d_shifts, int ns, int W, bool defer = false) {
-    return tile_sort_of(c, c->tl, psi, c->q1, c->n, d_shifts, ns, W, defer);
+dj_status tile_sort(dj_ctx *c, const void *psi, const double *d_shifts, int ns, int W, SortCheck check = SORT_STOP) {
+    return tile_sort_of(c, c->tl, psi, c->q1, c->n, d_shifts, ns, W, check);
 }
 
 // after a deferred sort overflowed (the stream is idle): the next one counts first
@@ -528,13 +543,12 @@ void sort_failed(dj_ctx *c) {
     c->part.zero(c->tl.flag, sizeof(unsigned), c->st);
 }
 
-// The flag of a call's first sort may wait for the end of the call where a force made in vain is cheaper
-// than the pause: a stop of the stream costs about 25 us, the force of a 128^3 mesh some 250 us, and lists
-// reserved at twice their last counts rarely overflow.  The further steps of a run, sorted from the step
-// before, defer theirs at every size.
-bool defer_first_sort(const dj_ctx *c) {
-    return c->cfg.n_resample == 1 && c->tl.lists && c->M <= ((size_t)1 << 21) && c->np <= ((int64_t)1 << 21);
-}
+// The flag of a sort may wait for the end of its step where a force made in vain is cheap: a stop of the stream costs
+// 43 us, the force of a 128^3 mesh some 170 us, and lists reserved at twice their last counts rarely overflow.  On
+// larger meshes the force costs more than the stops of many steps (1.5 ms at 256^3, 38 ms at 1024^3): a run asks for
+// the flag before it enqueues the force (ten steps at 256^3: 14.97 ms with stops, 14.59 so, 14.55 deferred).
+bool force_in_vain_is_cheap(const dj_ctx *c) { return c->M <= ((size_t)1 << 21) && c->np <= ((int64_t)1 << 21); }
+bool defer_first_sort(const dj_ctx *c) { return c->cfg.n_resample == 1 && c->tl.lists && force_in_vain_is_cheap(c); }
 
 dj_status sort_reports(dj_ctx *c) {
     if (!c->report) HIPCHK(c, hipHostMalloc((void **)&c->report, sizeof(unsigned) * REPORTS, hipHostMallocDefault));
@@ -591,7 +605,7 @@ bool ik_in_particle_order(const dj_ctx *c) {
     return c->cfg.grad_order == 0 && c->cfg.n_resample > 1 && c->rs_tiled && c->np <= side * side * side;
 }
 
-dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool defer = false) {
+dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, SortCheck check = SORT_STOP) {
     const dj_pm_config &cfg = c->cfg;
     const bool fixed = cfg.deposit == DJ_DEPOSIT_FIXED64;
     const int ns = c->nshifts;
@@ -608,7 +622,7 @@ dj_status force(dj_ctx *c, const void *psi, int mode, const KickArgs &kick, bool
     if (listed_kick && !c->own_at) HIPCHK(c, hipMalloc(&c->own_at, sizeof(unsigned) * (size_t)c->np));
     const bool unlisted = ik_in_particle_order(c);
     if (!unlisted) {
-        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, defer);
+        dj_status rs = tile_sort(c, psi, c->d_shifts, ns, cfg.worder, check);
         if (rs) return rs;
     }
     (void)mesh_bytes;
@@ -1137,7 +1151,7 @@ dj_status dj_acceleration(dj_ctx *c, const void *psi, void *acc_out) {
     k.nshifts = c->nshifts;
     const bool defer = defer_first_sort(c);
     dj_status r = defer ? sort_reports(c) : DJ_OK;
-    if (!r) r = force(c, src, FORCE_ACC, k, defer);
+    if (!r) r = force(c, src, FORCE_ACC, k, defer ? SORT_DEFER : SORT_STOP);
     if (r) return r;
     if (defer) HIPCHK(c, hipMemcpyAsync(c->report, c->tl.flag, sizeof(unsigned), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipMemcpyAsync(acc_out, c->acc, (size_t)c->n3 * c->tsize, hipMemcpyDeviceToHost, c->st));
@@ -1165,7 +1179,7 @@ dj_status dj_step(dj_ctx *c, double dd1, double alpha, double beta, double dd2) 
         c->report[0] = 0;
         k.gate = SortGate{c->tl.flag, c->report};
     }
-    dj_status r = force(c, c->psi, FORCE_KICK, k, defer);
+    dj_status r = force(c, c->psi, FORCE_KICK, k, defer ? SORT_DEFER : SORT_STOP);
     if (r) return r;
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (defer && c->report[0] != 1) {
@@ -1191,11 +1205,12 @@ dj_status dj_run(dj_ctx *c, int32_t n_steps, const double *dd1, const double *al
     }
     if (n_steps == 0) return DJ_OK;
     { Prof p(c, K_DRIFT); c->part.drift(c->psi, c->mom, c->n3, dd1[0], c->st); }
-    // A step after the first sorts from the step before, and its overflow flag is not waited for: its kick looks
-    // at the flag and reports, and the host, at most two steps ahead, goes back to the step that reports an
-    // overflow (nothing has touched the state since) and sorts it exactly.
-    const bool ahead = c->cfg.n_resample == 1;
-    if (ahead) {
+    // A step after the first sorts from the step before.  On a large mesh the host asks for its overflow flag before
+    // it enqueues the force.  On a small one the flag is not waited for: the step's kick looks at it and reports, and
+    // the host, at most two steps ahead, goes back to the step that reports an overflow (nothing has touched the state
+    // since) and sorts it exactly.
+    const bool reports = c->cfg.n_resample == 1, ahead = reports && force_in_vain_is_cheap(c);
+    if (reports) {
         dj_status r = sort_reports(c);
         if (r) return r;
     }
@@ -1206,11 +1221,12 @@ dj_status dj_run(dj_ctx *c, int32_t n_steps, const double *dd1, const double *al
         const bool has_next = s + 1 < n_steps && !stop;
         KickArgs k{alpha[s], beta[s], dd2[s], has_next ? dd1[s + 1] : 0.0, has_next ? 1 : 0, c->nshifts};
         const bool defer = ahead && s > first && c->tl.lists;
+        const SortCheck check = defer ? SORT_DEFER : reports && !ahead && s > 0 ? SORT_ASK : SORT_STOP;
         if (defer) {
             c->report[s % REPORTS] = 0;
             k.gate = SortGate{c->tl.flag, c->report + s % REPORTS};
         }
-        dj_status r = force(c, c->psi, FORCE_KICK, k, defer);
+        dj_status r = force(c, c->psi, FORCE_KICK, k, check);
         if (r) return r;
         if (!defer) known = s + 1;
         const int upto = stop || s + 1 == n_steps ? s : s - 1;

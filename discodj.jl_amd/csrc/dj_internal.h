@@ -108,6 +108,8 @@ struct TileOps {
     // list capacities from src (2 nt counts; may be cur), plus slack when slack != 0; zeroes cur
     void (*scan)(const TileArgs &a, const unsigned *src, int slack, hipStream_t st);
     void (*fill)(const TileArgs &a, int W, hipStream_t st);
+    // the flag of the fill enqueued last to g.report (1 + flag), in pinned host memory
+    void (*report)(const SortGate &g, hipStream_t st);
     // reverse mode: out_c = sum_p W(X_p + sh - cell) vals[p + c np] scale (3 meshes, every cell written);
     // false when the mesh has a single tile along an axis or the accumulators exceed the LDS.  work: 16 bytes
     // of device memory (the FP32 fixed-point scales)

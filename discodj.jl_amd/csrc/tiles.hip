@@ -397,6 +397,8 @@ __global__ __launch_bounds__(1024) void k_scan_one(const unsigned *src, int nt, 
     }
 }
 
+__global__ void k_sort_report(SortGate g) { (void)g.closed(); }
+
 // Entries of a list of cnt entries that lie in its reserve [begin, end) and in the buffer of cap entries:
 // all of them, except after a sort that overflowed and has not been repeated yet (the fill's cursors then
 // count entries that it did not write)
@@ -1380,6 +1382,7 @@ struct TileLaunch {
     static void fill(const TileArgs &a, int W, hipStream_t st) {
         if (W == 2) bin_w<2, true>(a, st); else if (W == 3) bin_w<3, true>(a, st); else bin_w<4, true>(a, st);
     }
+    static void report(const SortGate &g, hipStream_t st) { k_sort_report<<<1, 1, 0, st>>>(g); }
     template <int W, int ACC>
     static void dep_w(const TileArgs &a, const double *sh, void *mesh, double fscale, hipStream_t st) {
         const TileGeom &g = a.g;
@@ -1527,6 +1530,7 @@ template <typename T> void tile_ops(TileOps &ops) {
     ops.count = TileLaunch<T>::count;
     ops.scan = TileLaunch<T>::scan;
     ops.fill = TileLaunch<T>::fill;
+    ops.report = TileLaunch<T>::report;
     ops.deposit = TileLaunch<T>::deposit;
     ops.deposit3 = TileLaunch<T>::deposit3;
     ops.gather = TileLaunch<T>::gather;

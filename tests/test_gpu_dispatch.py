@@ -214,3 +214,59 @@ def test_ics_over_the_transform_sizes(n, order, prec):
     # the sum's own scale: its two dot products' norms times the direction's
     scale = np.linalg.norm(wb) * np.linalg.norm(v)
     assert abs(float(np.vdot(wb, v)) - (f[0] - f[1]) / (2 * eps)) < 1e-9 * scale
+
+
+def _calls(S):
+    """Launch groups of the solver's last calls (profiling on), by name."""
+    return {k: v["calls"] for k, v in S.kernel_stats().items()}
+
+
+def _collapse_run(cfg, n, steps, net=None):
+    """A collapse over some steps in one run, its launch counts, and the same steps one at a time, each on a new
+    solver, whose first sort counts: both states.  net: (parameters, output scale, scale factors of the forces)."""
+    psi, pi = 0.5 * _psi(n, 1.0, 5, np.float32), _collapse(n, cfg.boxsize, np.float32)
+    dd1, dd2 = np.full(steps, 0.125), np.full(steps, 0.125)
+    alpha, beta = np.full(steps, 0.99), np.full(steps, 1e-3)
+
+    def ready(S, state, a):
+        if net:
+            S.nn_set_params(net[0])
+            S.nn_enable(True, net[1])
+            S.nn_set_schedule(a)
+        S.set_state(*state)
+
+    with D.PMSolverHIP(cfg, precision=32) as S:
+        ready(S, (psi, pi), net and net[2])
+        S.set_profiling(True)
+        S.run(dd1, alpha, beta, dd2)
+        calls, got = _calls(S), S.get_state()
+    ref = (psi, pi)
+    for s in range(steps):
+        with D.PMSolverHIP(cfg, precision=32) as S:
+            ready(S, ref, net and net[2][s:s + 1])
+            S.run(dd1[s:s + 1], alpha[s:s + 1], beta[s:s + 1], dd2[s:s + 1])
+            ref = S.get_state()
+    return calls, got, ref
+
+
+@pytest.mark.parametrize("res, aa", [(256, 0), (384, 1)])
+def test_run_of_a_large_mesh_makes_no_force_in_vain(res, aa):
+    """A sort that overflows in a run on a large mesh (4096 tiles, and 13824 with the three-launch scan) is repeated
+    before its force is made: the exact sort ran again, and there is one deposit per step and pass."""
+    n, steps = 32, 6
+    cfg = D.PMConfig(res_pm=res, n_part=n, boxsize=100.0, grad_order=4, antialias=aa)
+    calls, got, ref = _collapse_run(cfg, n, steps)
+    assert calls["bin_recount"] >= 2 and calls["scatter"] == steps * (1 + aa), calls
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("net", [False, True])
+def test_run_of_a_small_mesh_goes_back_to_a_sort_that_overflows(net):
+    """On a small mesh the overflow is seen after the step's force: the run has made forces in vain, and the steps it
+    goes back to take their own place in the learned correction's schedule."""
+    n, res, steps, L = 32, 64, 6, 100.0
+    cfg = D.PMConfig(res_pm=res, n_part=n, boxsize=L, grad_order=4)
+    params = (D.learned.init_params(1, out_std=1.0), (L / res) ** 2, np.linspace(0.3, 0.9, steps)) if net else None
+    calls, got, ref = _collapse_run(cfg, n, steps, params)
+    assert calls["bin_recount"] >= 2 and calls["scatter"] > steps, calls
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
