@@ -596,9 +596,11 @@ __device__ __forceinline__ void tile_deposit(const Entry<T> *__restrict__ ent, c
 }
 
 // Workgroup (tile, part): on a mesh of few tiles, each tile's z planes are shared by several workgroups, which all read
-// its lists (rows outside a part are skipped, the sums are the same; ten steps at 64^3: 0.70 against 0.69 ms, and 0.67
-// with each entry loaded during the one before it).
-inline int deposit_parts(const TileGeom &g) { return g.nt <= 128 ? 4 : g.nt <= 256 ? 2 : 1; }
+// its lists (rows outside a part are skipped, the sums are the same), up to one workgroup per CU.  A pass of 64^3 on 64^3
+// (64 tiles, FP32) in 1, 2 and 4 parts: 14.8, 14.5 and 13.9 us with CIC, 60, 51 and 46 with PCS; FP64 48^3 on 48^3 (108
+// tiles, PCS) 39, 31 and 38.  More tiles lose: 96^3 on 96^3 (216 tiles, FP32) 16, 20 and 28 us with CIC, 70, 82 and
+// 104 with PCS; FP64 64^3 on 64^3 (256 tiles, PCS) 39, 48 and 57.
+inline int deposit_parts(const TileGeom &g) { return g.nt <= 64 ? 4 : g.nt <= 128 ? 2 : 1; }
 // FP32 tiles (ACC_Q31) with fewer than 2^12 entries sum in 32 bits (ACC_Q32); the LDS holds 64-bit
 // accumulators either way
 template <typename T, int W, int ACC, bool PAD>

@@ -270,3 +270,15 @@ def test_run_of_a_small_mesh_goes_back_to_a_sort_that_overflows(net):
     calls, got, ref = _collapse_run(cfg, n, steps, params)
     assert calls["bin_recount"] >= 2 and calls["scatter"] > steps, calls
     assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("W", [2, 4])
+@pytest.mark.parametrize("res, n, prec", [(32, 20, 64), (48, 24, 64), (64, 40, 32), (64, 40, 64), (96, 40, 32)])
+def test_deposit_over_the_sharing_rule(res, n, prec, W):
+    """Tiles shared by 4, 2 and 1 workgroups (32, 108, 64, 256 and 216 tiles), against the oracle's deposit in the same
+    precision."""
+    L = 1.5 * res
+    psi = _psi(n, 2.0, res + W, np.float32 if prec == 32 else np.float64)
+    with D.PMSolverHIP(D.PMConfig(res_pm=res, n_part=n, boxsize=L, worder=W), precision=prec) as S:
+        m = S.deposit(psi)
+    assert G.rel(m, O.pm_scatter(O.lagrangian_positions(psi, L), res, L, W)) < (2e-5 if prec == 32 else 1e-12)
