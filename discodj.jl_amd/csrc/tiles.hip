@@ -1199,16 +1199,17 @@ struct MarchMap {
     bool patches;   // 4 x 4 column patches dealt round-robin to the XCDs
 };
 // Segments are as long as leaves MARCH_WGS workgroups (four per CU; 16 tiles at most, where a tile stages
-// TZ of S2 planes and longer ones gain nothing).  A mesh of too few tiles for that gives every tile up to
-// four workgroups, each of which stages the tile and takes its part of the list.  16 tiles everywhere left
-// a 64^3 mesh with 8 workgroups (97 us; 9 us with 256) and a 256^3 mesh with one per CU (279 us a pass,
-// CIC, order 4; 204 us with four).
+// TZ of S2 planes and longer ones gain nothing).  16 tiles everywhere left a 64^3 mesh with 8 workgroups (97 us; 9 us
+// with 256) and a 256^3 mesh with one per CU (279 us a pass, CIC, order 4; 224 us with four).
+// A mesh of too few tiles for that gives every tile up to four workgroups, each of which stages the tile and takes its
+// part of the list: four up to 128 tiles (64^3 on 64^3, CIC, order 4: 20 us, 14 with two, 11 with four), two up to 256
+// where a part fills its workgroups (96^3, 216 tiles: 24 and 22 us for 96^3 particles, but PCS 18.8 and 24.6 for 48^3).
 constexpr int MARCH_WGS = 1024;
-inline MarchMap march_map(const TileGeom &g) {
+inline MarchMap march_map(const TileGeom &g, size_t np) {
     MarchMap m;
     m.G = 1;
     while (m.G < 16 && g.ntz % (2 * m.G) == 0 && g.nt / (2 * m.G) >= MARCH_WGS) m.G *= 2;
-    m.parts = g.nt <= 128 ? 4 : g.nt <= 256 ? 2 : 1;
+    m.parts = g.nt <= 128 ? 4 : g.nt <= 256 && np >= (size_t)2048 * g.nt ? 2 : 1;
     m.patches = g.ntx % 4 == 0 && g.nty % 4 == 0 && ((g.ntx / 4) * (g.nty / 4)) % 8 == 0;
     return m;
 }
@@ -1471,7 +1472,7 @@ struct TileLaunch {
         constexpr int H = O / 2;
         const StageGeom q = gather_geom<T, W, true>(a.g, H);
         const size_t shm = sizeof(T) * (size_t)q.s[0] * q.s[1] * q.s[2];
-        const MarchMap mm = march_map(a.g);
+        const MarchMap mm = march_map(a.g, (size_t)a.n * a.n * a.n);
         auto kern = k_tile_gather_march<T, W, O, M>;
         (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         kern<<<a.g.nt / mm.G * mm.parts, gather_threads<T, W>(), shm, st>>>(

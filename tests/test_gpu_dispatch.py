@@ -282,3 +282,15 @@ def test_deposit_over_the_sharing_rule(res, n, prec, W):
     with D.PMSolverHIP(D.PMConfig(res_pm=res, n_part=n, boxsize=L, worder=W), precision=prec) as S:
         m = S.deposit(psi)
     assert G.rel(m, O.pm_scatter(O.lagrangian_positions(psi, L), res, L, W)) < (2e-5 if prec == 32 else 1e-12)
+
+
+@pytest.mark.parametrize("n, W", [(76, 2), (77, 2), (77, 4)])
+def test_force_on_both_sides_of_the_gather_sharing_rule(n, W):
+    """216 tiles, taken by one workgroup each or, from 2048 particles a tile, by two, against the oracle (the bound of
+    test_step_over_the_gather_segment_rule)."""
+    res, L = 96, 192.0
+    psi = _psi(n, 3.0, n, np.float32)
+    with D.PMSolverHIP(D.PMConfig(res_pm=res, n_part=n, boxsize=L, worder=W), precision=32) as S:
+        acc = S.pm_acceleration(psi)
+    ref = O.pm_acceleration(psi.astype(np.float64), O.pm_config(res, n, L, worder=W, grad_order=4), "solver")
+    assert G.rel(acc, ref) < 2e-5
