@@ -175,9 +175,7 @@ __device__ __forceinline__ bool fill_lists(const BinMasks &M, unsigned long long
     return fits;
 }
 
-// A workgroup takes 16 x BN x BN particles, a wave 16 x 4 x 1 of them.  BN = 4; on a mesh of few tiles, whose
-// list counters would see an atomic from every workgroup (80 each at 64^3), BN = 8 makes a quarter of them:
-// 0.71 against 0.76 ms for ten steps at 64^3, but 15.0 against 14.9 at 256^3.
+// A workgroup takes 16 x BN x BN particles, a wave 16 x 4 x 1 of them: BN = 4, or 8 (bin_size).
 template <typename T, int W, bool FILL, int BN>
 __global__ __launch_bounds__((16 * BN * BN)) void k_tile_bin(const T *__restrict__ psi, const T *__restrict__ q1, int n,
                                                   const double *__restrict__ shifts, int ns, T L, TileGeom g,
@@ -1355,6 +1353,12 @@ __global__ __launch_bounds__(256) void k_kick_listed(const unsigned *__restrict_
 // ------------------------------------------------------------------------------------ launchers
 static unsigned cap32(const TileArgs &a) { return (unsigned)std::min<size_t>(a.ent_cap, 0xffffffffu); }
 
+// Side of a bin workgroup's block of particles.  On a mesh of few tiles, every list counter sees an atomic from many
+// workgroups (80 each at 64^3 on 64^3), and blocks of 8 make a quarter of them: 23.7 against 18.8 us there (CIC, FP32),
+// 35.1 against 27.4 at 96^3 on 96^3.  With fewer particles the larger workgroups leave CUs idle: 13.7 against 16.6 us for
+// 16^3 on 32^3 in FP64, 18.5 against 16.4 for 48^3 on 48^3 in FP32.  On 256^3 (4096 tiles) they gain nothing.
+static int bin_size(const TileArgs &a) { return a.g.nt <= 256 && (int64_t)a.n * a.n * a.n >= 100000 ? 8 : 4; }
+
 template <typename T>
 struct TileLaunch {
     template <int W, bool FILL, int BN>
@@ -1366,7 +1370,7 @@ struct TileLaunch {
     }
     template <int W, bool FILL>
     static void bin_w(const TileArgs &a, hipStream_t st) {
-        if (a.g.nt <= 256) bin_n<W, FILL, 8>(a, st);
+        if (bin_size(a) == 8) bin_n<W, FILL, 8>(a, st);
         else bin_n<W, FILL, 4>(a, st);
     }
     static void count(const TileArgs &a, int W, hipStream_t st) {

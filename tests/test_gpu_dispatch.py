@@ -294,3 +294,16 @@ def test_force_on_both_sides_of_the_gather_sharing_rule(n, W):
         acc = S.pm_acceleration(psi)
     ref = O.pm_acceleration(psi.astype(np.float64), O.pm_config(res, n, L, worder=W, grad_order=4), "solver")
     assert G.rel(acc, ref) < 2e-5
+
+
+@pytest.mark.parametrize("n", [46, 47])
+@pytest.mark.parametrize("res, prec", [(48, 64), (64, 32)])
+def test_lists_on_both_sides_of_the_bin_size_rule(res, prec, n):
+    """Bins of 4 and 8 particles a side (up to and from 100000 particles): the deposit through an exact sort and through
+    one into reserved lists, against the oracle's in the same precision."""
+    L = 1.5 * res
+    psi = _psi(n, 2.0, n, np.float32 if prec == 32 else np.float64)
+    ref = O.pm_scatter(O.lagrangian_positions(psi, L), res, L, 3)
+    with D.PMSolverHIP(D.PMConfig(res_pm=res, n_part=n, boxsize=L, worder=3), precision=prec) as S:
+        for m in (S.deposit(psi), S.deposit(psi)):
+            assert G.rel(m, ref) < (2e-5 if prec == 32 else 1e-12)
