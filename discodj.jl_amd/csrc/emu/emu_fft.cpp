@@ -127,7 +127,11 @@ struct Emu {
             }
         for (int z = 0; z < N; z++)
             for (int yb = 0; yb < N / B; yb++) {
-                for (int t = 0; t < NT; t++) P::xi_load_pre(A, lds.data(), tw, yb, z, t);
+                for (int t = 0; t < NT; t++) {
+                    cx<T> va[P::XI_CNT], vb[P::XI_CNT];
+                    P::xi_fetch(A, yb, z, t, va, vb);
+                    P::xi_pre(lds.data(), tw, t, va, vb);
+                }
                 if constexpr (WAVE) {
                     emu_engine_wave<EX, +1, 2>(lds, tw);
                     for (int t = 0; t < NT; t++) P::xi_store_w(lds.data(), mesh, yb, z, t);

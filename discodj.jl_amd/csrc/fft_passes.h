@@ -195,14 +195,6 @@ struct Passes {
             }
         }
     }
-    // all reads of a thread are issued before its first LDS write
-    template <bool MUL = false>
-    DJ_HD static void xi_load_pre(const cx<T> *A, cx<T> *lds, const cx<T> *twN, int yb, int z, int tid,
-                                  const cx<T> *tab = nullptr) {
-        cx<T> va[XI_CNT], vb[XI_CNT];
-        xi_fetch(A, yb, z, tid, va, vb);
-        xi_pre<MUL>(lds, twN, tid, va, vb, tab);
-    }
     // SC: each value multiplied by s as it is stored (a normalisation that would otherwise be a pass of its own)
     template <bool SC = false>
     DJ_HD static void xi_store(const cx<T> *lds, T *mesh, int yb, int z, int tid, T s = (T)1) {
