@@ -601,9 +601,13 @@ void ik_force_mesh(dj_ctx *c, int ax, void *out) {
 }
 
 // With sheet resampling the particles' own lists would serve the spectral gradient's gather alone.  For few
-// particles their sort and the tiles cost more than reading the mesh in particle order: a step with linear
-// resampling (CIC) of 24^3 on 64^3 took 408 us with them and 285 without, 128^3 on 128^3 1389 and 1281; PCS, with
-// eight times the reads, 408 and 357 at 32^3 on 96^3 and 461 and 439 at 48^3 on 96^3.
+// particles their sort and the tiles cost more than reading the mesh in particle order.  A step with linear resampling
+// (FP32, one pass) in particle order and with the lists, in us:
+//   CIC  24^3 on 64^3 285, 408;  128^3 on 128^3 1285, 1375;  192^3 on 256^3 3298, 3345;  256^3 on 256^3 6774, 6904
+//   TSC  64^3 on 64^3 491, 539;  96^3 on 128^3 902, 935 (FP64 1230, 1216);  128^3 on 256^3 1688, 1622
+//   PCS  32^3 on 64^3 375, 397;  48^3 on 96^3 448, 469;  64^3 on 128^3 596, 584
+// Interlacing, FP64 and finer meshes favour the lists by a few percent more (TSC 96^3 on 256^3 in FP64 1827, 1701), so
+// the lines lie where particle order gains in all of them; for CIC the two differ by 3 % at most from 128^3 on.
 bool ik_in_particle_order(const dj_ctx *c) {
     const int64_t side = c->cfg.worder == 2 ? 128 : c->cfg.worder == 3 ? 64 : 48;
     return c->cfg.grad_order == 0 && c->cfg.n_resample > 1 && c->rs_tiled && c->np <= side * side * side;

@@ -43,7 +43,7 @@ enum { NN_RES_NONE = 0, NN_RES_INPUT = 1, NN_RES_TENSOR = 2 };  // the residual:
 
 // One block marches along z over a 64 (x) x 8 (y) footprint: the input planes z-1, z, z+1 (with a one-voxel x-y
 // halo, 66 x 10 voxels) sit in a three-slot LDS ring, so each input voxel is read from memory about 1.3 times
-// instead of once per tap.  Two blocks share a CU (63 KB of LDS each).  Wave w computes y rows 2w, 2w+1 of the
+// instead of once per tap.  Two blocks share a CU (64.5 KiB of LDS each).  Wave w computes y rows 2w, 2w+1 of the
 // plane (8 segments of 16 voxels), per tap one MFMA per segment.  The taps' weights (A) stay in registers for
 // the whole march; an input row (B) is read from LDS once for the two output rows that use it (48 reads of 8
 // bytes a lane and input plane instead of 72); and the plane after the next is loaded into registers while the
